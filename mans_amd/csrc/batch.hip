@@ -8,6 +8,7 @@ bool batch_shape_ok(BatchShape sh, int pb, bool decode) {
   if (sh.nw != 4 && sh.nw != 8 && sh.nw != 16) return false;
   if (sh.kb != 4 && sh.kb != 8 && sh.kb != 16 && !(decode && sh.kb == 1)) return false;
   if (pb < 9 || pb > 11) return false;
+  if (!decode && sh.nw == 16) return false;  // encode: 256 or 512 threads
   return (decode ? batch_decode_lds(sh, pb) : batch_encode_lds(sh)) <= kLdsBytes;
 }
 

@@ -39,11 +39,12 @@ constexpr uint32_t kRB = 10;           // ring: 1024 words per chain
 constexpr uint32_t kR = 1u << kRB, kH = kR / 2, kMask = kR - 1;
 constexpr uint32_t kGenShift = 48;
 constexpr uint64_t kValue48 = (1ull << kGenShift) - 1;
-// per-wave LDS in 32-bit words: two encoder tables (or the histogram
-// counters, or the normalisation keys) | two rings | dummy slots
-constexpr uint32_t kTabWords = 2 * 256 * 4;
-constexpr uint32_t kRingWords = 2 * kR / 2;
-constexpr uint32_t kWaveWords = kTabWords + kRingWords + 64;
+// per-wave LDS in 32-bit words: two encoder tables | the chains' stages; a
+// workgroup's waves together also hold the histogram phase's counters, keys
+// and flags
+constexpr uint32_t kTabWords = 2 * 256 * 2;
+constexpr uint32_t kStageWords = 4 * 512 / 2;
+constexpr uint32_t kWaveWords = kTabWords + kStageWords + 128;
 // Queue items a decode wavefront takes at once (BatchDecodeArgs::run, 1 or
 // 4): consecutive tickets of a buffer then run on one wavefront, which keeps
 // the buffer's LUTs in its LDS.  (Encode takes one at a time: a ticket's
@@ -254,10 +255,9 @@ __device__ void finish_buffer(const BatchBuf& B, uint32_t b, const BatchEncodeAr
     uint16_t pr[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      // the encoder's form (enc64_entry)
-      const uint4 f = enc64_entry(e[j].x, e[j].y, PB);
-      atomic_st64(t2 + 2 * (4 * lane + j), ((uint64_t)f.y << 32) | f.x);
-      atomic_st64(t2 + 2 * (4 * lane + j) + 1, ((uint64_t)f.w << 32) | f.z);
+      // the encoder's form (enc_entry)
+      const uint2 f = enc_entry(e[j], PB);
+      atomic_st64(t2 + 4 * lane + j, ((uint64_t)f.y << 32) | f.x);
       pr[j] = (uint16_t)e[j].x;
     }
     uint8_t* sec = B.out + B.section[k];
@@ -331,15 +331,14 @@ __device__ uint64_t encode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, ui
   constexpr uint32_t CSTAGE = chain_stage_words<PB>();
   constexpr uint32_t H = 256, H4 = H / 8, REG = H + 256;
   static_assert(kBlock / kL % KBB == 0 && KBB % 4 == 0, "KBB steps per prefetch batch, checks every 4");
-  static_assert((uint32_t)CH * REG <= 2 * kRingWords, "stages fit the wave's stage area");
+  static_assert((uint32_t)CH * REG <= 2 * kStageWords, "stages fit the wave's stage area");
   using T = typename ElemOf<EB>::T;
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t P = EB;
   const uint64_t U = (uint64_t)P * B.nb;
   const uint64_t u0 = (uint64_t)UTR * lt;
-  uint4* s_tab = (uint4*)wl;  // [SPB <= 2][256]
+  uint2* s_tab = (uint2*)wl;  // [SPB <= 2][256]
   uint16_t* wstage = (uint16_t*)(wl + kTabWords);
-  const uint32_t dummy_addr = lds_addr(wstage + CH * REG + 2u * lane);
   static_assert(UT <= kMaxTicketUnits, "a ticket's units fit its slot");
   uint32_t padj[UT];  // per unit of the ticket (wave-uniform)
 #pragma unroll
@@ -376,7 +375,7 @@ __device__ uint64_t encode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, ui
         const uint64_t* g = (const uint64_t*)(a.tables + ((uint64_t)b * 4u + p0 + q) * 256u);
         uint64_t* d = (uint64_t*)(s_tab + q * 256);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) d[lane + 64 * k] = atomic_ld64(g + lane + 64 * k);
+        for (int k = 0; k < 4; ++k) d[lane + 64 * k] = atomic_ld64(g + lane + 64 * k);
       }
       tkey = key;
     }
@@ -412,8 +411,39 @@ __device__ uint64_t encode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, ui
     const T* eb[BPT];
 #pragma unroll
     for (int d = 0; d < BPT; ++d) eb[d] = (const T*)B.in + blk[d * SPB] * kBlock;
+    // table entries of the chains for step k of a batch
+    auto lookup = [&](uint2 (&e)[CH], const uint32_t (&buf)[BPT][KBB], int k) {
+#pragma unroll
+      for (int d = 0; d < BPT; ++d) {
+        const uint32_t w = EB == 4 ? buf[d][k] >> (8u * p0) : buf[d][k];
+        e[d * SPB] = *(const uint2*)((const char*)s_tab + byte_x8<0>(w));
+        if constexpr (SPB > 1) e[d * SPB + 1] = *(const uint2*)((const char*)(s_tab + 256) + byte_x8<1>(w));
+      }
+    };
+    // the KBB steps from s0 on (FULL: every lane of every chain has a symbol
+    // at each of them; else those below n[c])
+    auto code = [&](const uint32_t (&buf)[BPT][KBB], uint32_t s0, auto full) {
+      constexpr bool FULL = decltype(full)::value;
+      uint2 e[CH];
+      lookup(e, buf, 0);
+#pragma unroll
+      for (int k = 0; k < KBB; ++k) {
+        uint2 en[CH];
+        if (k + 1 < KBB) lookup(en, buf, k + 1);
+        bool v[CH];
+#pragma unroll
+        for (int c = 0; c < CH; ++c) v[c] = FULL || (s0 + (uint32_t)k) * kL + lane < n[c];
+        enc_steps64<PB, CH, FULL>(x, sb, e, v);
+        if ((k & 3) == 3) spill_full();
+        if (k + 1 < KBB) {
+#pragma unroll
+          for (int c = 0; c < CH; ++c) e[c] = en[c];
+        }
+      }
+    };
     uint32_t s = 0;
-    if (n_min == kBlock && all_act) {
+    const uint32_t nbatch = all_act ? n_min / (kL * KBB) : 0u;
+    if (nbatch > 0) {
       auto load = [&](uint32_t (&buf)[BPT][KBB], uint32_t s0) {
 #pragma unroll
         for (int d = 0; d < BPT; ++d) {
@@ -422,54 +452,44 @@ __device__ uint64_t encode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, ui
           for (int k = 0; k < KBB; ++k) buf[d][k] = bp[k * kL];
         }
       };
-      auto lookup = [&](uint4 (&e)[CH], const uint32_t (&buf)[BPT][KBB], int k) {
-#pragma unroll
-        for (int d = 0; d < BPT; ++d) {
-          const uint32_t w = EB == 4 ? buf[d][k] >> (8u * p0) : buf[d][k];
-          e[d * SPB] = *(const uint4*)((const char*)s_tab + byte_x16<0>(w));
-          if constexpr (SPB > 1) e[d * SPB + 1] = *(const uint4*)((const char*)(s_tab + 256) + byte_x16<1>(w));
-        }
-      };
-      auto code = [&](const uint32_t (&buf)[BPT][KBB]) {
-        uint4 e[CH];
-        lookup(e, buf, 0);
-#pragma unroll
-        for (int k = 0; k < KBB; ++k) {
-          uint4 en[CH];
-          if (k + 1 < KBB) lookup(en, buf, k + 1);
-#pragma unroll
-          for (int c = 0; c < CH; ++c) enc_step64f(x[c], sb[c], dummy_addr, e[c]);
-          if ((k & 3) == 3) spill_full();
-          if (k + 1 < KBB) {
-#pragma unroll
-            for (int c = 0; c < CH; ++c) e[c] = en[c];
-          }
-        }
-      };
-      const uint32_t last = kBlock / kL - KBB;
+      const uint32_t last = (nbatch - 1) * KBB;
       uint32_t bA[BPT][KBB], bB[BPT][KBB];
       load(bA, 0);
       for (;;) {
         load(bB, s + KBB <= last ? s + KBB : last);
-        code(bA);
+        code(bA, s, std::true_type{});
         s += KBB;
         if (s > last) break;
         load(bA, s + KBB <= last ? s + KBB : last);
-        code(bB);
+        code(bB, s, std::true_type{});
         s += KBB;
         if (s > last) break;
       }
     }
-    for (; s < all; ++s) {
-      const uint32_t i = s * kL + lane;
+    // the rest (a buffer's last, partial blocks and the whole blocks beside
+    // them): lanes past a block's end load nothing and keep their state
+    if (s < all) {
+      auto load_part = [&](uint32_t (&buf)[BPT][KBB], uint32_t s0) {
 #pragma unroll
-      for (int c = 0; c < CH; ++c) {
-        const bool v = i < n[c];
-        const uint32_t w = v ? (uint32_t)eb[c / SPB][i] : 0u;
-        const uint32_t sy = (w >> (8u * (p0 + (uint32_t)(c % SPB)))) & 0xffu;
-        enc_step64(x[c], sb[c], dummy_addr, s_tab[(c % SPB) * 256 + sy], v);
+        for (int d = 0; d < BPT; ++d)
+#pragma unroll
+          for (int k = 0; k < KBB; ++k) {
+            const uint32_t i = (s0 + (uint32_t)k) * kL + lane;
+            buf[d][k] = i < n[d * SPB] ? (uint32_t)((gptr<T>)eb[d])[i] : 0u;
+          }
+      };
+      uint32_t buf[BPT][KBB], nxt[BPT][KBB];
+      load_part(buf, s);
+      for (;;) {
+        load_part(nxt, s + KBB);
+        code(buf, s, std::false_type{});
+        s += KBB;
+        if (s >= all) break;
+#pragma unroll
+        for (int d = 0; d < BPT; ++d)
+#pragma unroll
+          for (int k = 0; k < KBB; ++k) buf[d][k] = nxt[d][k];
       }
-      spill_full();
     }
 
     // pad, stage remainder to the slot, states, block sizes
@@ -540,7 +560,7 @@ __device__ uint64_t encode_ticket32(const BatchBuf& B, uint32_t b, uint32_t lt, 
   constexpr uint32_t H = 256, H4 = H / 8, REG = H + 256;
   constexpr uint32_t NT = EB == 1 ? 1u : 2u;  // tables of the ticket
   static_assert(BLOCK / L % KBB == 0 && KBB % 4 == 0, "KBB steps per prefetch batch, checks every 4");
-  static_assert(NU * REG + 128 <= 2 * (kRingWords + 64), "stages and dummy slots fit the wave's stage area");
+  static_assert(NU * REG <= 2 * kStageWords, "stages fit the wave's stage area");
   static_assert(SSTAGE % 8 == 0 && NU * SSTAGE <= kMaxTicketUnits * CSTAGE && NU <= (int)kMaxTicketUnits, "slot areas");
   using T = typename ElemOf<EB>::T;
   const uint32_t lane = threadIdx.x & 63u, half = lane >> 5, lin = lane & 31u;
@@ -560,9 +580,8 @@ __device__ uint64_t encode_ticket32(const BatchBuf& B, uint32_t b, uint32_t lt, 
     blk[c] = act[c] ? u / P : 0u;
     n[c] = act[c] ? (uint32_t)((B.n - blk[c] * BLOCK) < BLOCK ? (B.n - blk[c] * BLOCK) : BLOCK) : 0u;
   }
-  uint4* s_tab = (uint4*)wl;  // [NT][256]
+  uint2* s_tab = (uint2*)wl;  // [NT][256]
   uint16_t* wstage = (uint16_t*)(wl + kTabWords);
-  const uint32_t dummy_addr = lds_addr(wstage + NU * REG + 2u * lane);
   const uint64_t key = ((uint64_t)b << 4) | p0;
   if (key != tkey) {
     drain();  // the previous ticket's table reads are done
@@ -571,11 +590,11 @@ __device__ uint64_t encode_ticket32(const BatchBuf& B, uint32_t b, uint32_t lt, 
       const uint64_t* g = (const uint64_t*)(a.tables + ((uint64_t)b * 4u + p0 + q) * 256u);
       uint64_t* d = (uint64_t*)(s_tab + q * 256);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) d[lane + 64 * k] = atomic_ld64(g + lane + 64 * k);
+      for (int k = 0; k < 4; ++k) d[lane + 64 * k] = atomic_ld64(g + lane + 64 * k);
     }
     tkey = key;
   }
-  const uint4* tab[NC];
+  const uint2* tab[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) tab[c] = s_tab + (kp[c] - p0) * 256u;
   uint32_t x[NC];
@@ -624,8 +643,25 @@ __device__ uint64_t encode_ticket32(const BatchBuf& B, uint32_t b, uint32_t lt, 
 #pragma unroll
   for (int d = 0; d < NBK; ++d) ep[d] = (const T*)B.in + blk[d] * BLOCK;
   auto shift_of = [&](int c) -> uint32_t { return EB == 1 ? 0u : 8u * kp[c]; };
+  // the KBB steps from s0 on, as in encode_ticket
+  auto code = [&](const uint32_t (&buf)[NBK][KBB], uint32_t s0, auto full) {
+    constexpr bool FULL = decltype(full)::value;
+#pragma unroll
+    for (int k = 0; k < KBB; ++k) {
+      uint2 e[NC];
+      bool v[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        e[c] = tab[c][(buf[EB == 1 ? c : 0][k] >> shift_of(c)) & 0xffu];
+        v[c] = FULL || (s0 + (uint32_t)k) * L + lin < n[c];
+      }
+      enc_steps32<PB, NC, FULL>(x, sb, half, e, v);
+      if ((k & 3) == 3) spill_full();
+    }
+  };
   uint32_t s = 0;
-  if (n_min == BLOCK) {
+  const uint32_t nbatch = n_min / (L * KBB);
+  if (nbatch > 0) {
     auto load = [&](uint32_t (&buf)[NBK][KBB], uint32_t s0) {
 #pragma unroll
       for (int d = 0; d < NBK; ++d) {
@@ -634,40 +670,42 @@ __device__ uint64_t encode_ticket32(const BatchBuf& B, uint32_t b, uint32_t lt, 
         for (int k = 0; k < KBB; ++k) buf[d][k] = bp[k * L];
       }
     };
-    auto code = [&](const uint32_t (&buf)[NBK][KBB]) {
-#pragma unroll
-      for (int k = 0; k < KBB; ++k) {
-        uint4 e[NC];
-#pragma unroll
-        for (int c = 0; c < NC; ++c) e[c] = tab[c][(buf[EB == 1 ? c : 0][k] >> shift_of(c)) & 0xffu];
-#pragma unroll
-        for (int c = 0; c < NC; ++c) enc_step32f(x[c], sb[c], sb[NC + c], half, e[c]);
-        if ((k & 3) == 3) spill_full();
-      }
-    };
-    const uint32_t last = BLOCK / L - KBB;
+    const uint32_t last = (nbatch - 1) * KBB;
     uint32_t bA[NBK][KBB], bB[NBK][KBB];
     load(bA, 0);
     for (;;) {
       load(bB, s + KBB <= last ? s + KBB : last);
-      code(bA);
+      code(bA, s, std::true_type{});
       s += KBB;
       if (s > last) break;
       load(bA, s + KBB <= last ? s + KBB : last);
-      code(bB);
+      code(bB, s, std::true_type{});
       s += KBB;
       if (s > last) break;
     }
   }
-  for (; s < all; ++s) {
-    const uint32_t i = s * L + lin;
+  if (s < all) {
+    auto load_part = [&](uint32_t (&buf)[NBK][KBB], uint32_t s0) {
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const bool v = i < n[c];
-      const uint32_t w = v ? (uint32_t)ep[EB == 1 ? c : 0][i] : 0u;
-      enc_step32(x[c], sb[c], sb[NC + c], half, dummy_addr, tab[c][(w >> shift_of(c)) & 0xffu], v);
+      for (int d = 0; d < NBK; ++d)
+#pragma unroll
+        for (int k = 0; k < KBB; ++k) {
+          const uint32_t i = (s0 + (uint32_t)k) * L + lin;
+          buf[d][k] = i < n[d] ? (uint32_t)((gptr<T>)ep[d])[i] : 0u;
+        }
+    };
+    uint32_t buf[NBK][KBB], nxt[NBK][KBB];
+    load_part(buf, s);
+    for (;;) {
+      load_part(nxt, s + KBB);
+      code(buf, s, std::false_type{});
+      s += KBB;
+      if (s >= all) break;
+#pragma unroll
+      for (int d = 0; d < NBK; ++d)
+#pragma unroll
+        for (int k = 0; k < KBB; ++k) buf[d][k] = nxt[d][k];
     }
-    spill_full();
   }
 
   // pad each unit, its stage remainder to its slot area, states, block sizes

@@ -1110,7 +1110,7 @@ struct mans_batch {
   uint32_t* hist = nullptr;   // [cap_bufs][4][256]
   uint32_t* done = nullptr;   // [cap_bufs]
   uint32_t* ready = nullptr;  // [cap_bufs]
-  uint4* tables = nullptr;    // [cap_bufs][4][256]
+  uint2* tables = nullptr;    // [cap_bufs][4][256]
   uint64_t* status = nullptr; // [cap_ticks]
   uint32_t* ptot = nullptr;   // [cap_bufs][4]
   uint32_t* fin = nullptr;    // [cap_bufs]
@@ -1279,7 +1279,7 @@ mans_status batch_alloc(mans_batch* b, uint32_t cap_bufs, uint64_t cap_items, ui
   } else {
     HIP_TRY(hipMalloc(&b->hist, nb1 * 4096));
     HIP_TRY(hipMalloc(&b->done, nb1 * 4));
-    HIP_TRY(hipMalloc(&b->tables, nb1 * 4 * 256 * sizeof(uint4)));
+    HIP_TRY(hipMalloc(&b->tables, nb1 * 4 * 256 * sizeof(uint2)));
     HIP_TRY(hipMalloc(&b->status, std::max<uint64_t>(1, cap_ticks) * 8));
     HIP_TRY(hipMalloc(&b->ptot, nb1 * 16));
     HIP_TRY(hipMalloc(&b->fin, nb1 * 4));

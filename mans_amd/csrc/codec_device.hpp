@@ -4,6 +4,9 @@
 #pragma once
 #include "mans_internal.hpp"
 
+#ifndef SLEEPX
+#define SLEEPX 1
+#endif
 namespace mans {
 
 template <int S> struct ElemOf;
@@ -67,181 +70,170 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
 
-// Encoder table entry of the 64-lane coder, for probability precision p:
-// {pdf << (31 - p) | cdf, 2^p - pdf, lo, hi of rcp}, rcp = 1 / pdf rounded
-// up to a double.  (p <= 15, so the threshold pdf << (31 - p) has no bits
-// below bit 16 and cdf fits under it.)  For 0 <= x < 2^31 and pdf <= 2^11,
-// floor(RN(x * rcp)) = floor(x / pdf): x * rcp >= x / pdf >= q, and
-// x * rcp < x / pdf + 2^-21 <= q + 1 - 2^-11 + 2^-21, so neither the
-// product's rounding nor the truncating conversion can leave [q, q + 1).
-// This replaces the reference's magic-number division
-// (GpuANSCodec.h:36-61: q = (umulhi(x, magic) + x) >> shift) by two full-rate
-// conversions and one full-rate f64 multiply on gfx950; q is the same.
-__device__ __forceinline__ uint4 enc64_entry(uint32_t pdf, uint32_t cdf, int p) {
-  double r = 0.0;
-  if (pdf > 0) {
-    r = 1.0 / (double)pdf;
-    // round up: the exact residual r * pdf - 1 (one fma) below zero means
-    // the correctly rounded quotient is below 1 / pdf
-    if (__fma_rn(r, (double)pdf, -1.0) < 0.0) r = __longlong_as_double(__double_as_longlong(r) + 1);
-  }
-  const uint64_t rb = (uint64_t)__double_as_longlong(r);
-  return make_uint4((pdf << (31 - p)) | cdf, (1u << p) - pdf, (uint32_t)rb, (uint32_t)(rb >> 32));
+// Encoder table entry of the multi-chain coders for probability precision p,
+// 8 bytes, from a normalised symbol {pdf, cdf, magic, shift}:
+//   x = (2^p - pdf) << 16 | cdf << 5 | s,   s = ceil(log2 pdf)
+//   y = m = ceil(2^(31 + s) / pdf)
+// (2^p - pdf and cdf are below 2^11 and s <= 11; a shift by x takes its low
+// five bits, s.)  floor(floor(2 x m / 2^32) / 2^s) = floor(x / pdf) for every
+// x < 2^31: with e = m pdf - 2^(31 + s) < pdf <= 2^s, x m / 2^(31 + s) =
+// x / pdf + x e / (pdf 2^(31 + s)), and the second term is below 1 / pdf.
+// The reference's magic (GpuANSCodec.h:36-61) is floor(2^32 (2^s - pdf) / pdf)
+// + 1, so m = 2^31 + ceil(magic / 2) (for a power of two one more than the
+// ceiling: then e = 2^s, still below since x < 2^31).
+// (16-byte entries took 12 LDS cycles a wave read on random symbols, these 7.)
+__device__ __forceinline__ uint2 enc_entry(const uint4& t, int p) {
+  return make_uint2((((1u << p) - t.x) << 16) | (t.y << 5) | t.w, 0x80000000u + (t.z >> 1) + (t.z & 1u));
 }
 
-// x / pdf for the entry e (see enc64_entry).
-__device__ __forceinline__ uint32_t enc64_quot(uint32_t x, const uint4& e) {
-  const double r = __hiloint2double((int)e.w, (int)e.z);
-  return (uint32_t)((double)x * r);
+// floor(x / pdf) for the entry e.  (The doubling as v_add_u32: the compiler
+// would pick a shift.)
+__device__ __forceinline__ uint32_t enc_quot(uint32_t x, const uint2& e) {
+  uint32_t x2;
+  __asm__("v_add_u32 %0, %1, %1" : "=v"(x2) : "v"(x));
+  return __umulhi(x2, e.y) >> (e.x & 31u);
+}
+// The next state q 2^p + (x - q pdf) + cdf of a renormalised state x with
+// quotient q = x / pdf (below 2^22).
+__device__ __forceinline__ uint32_t enc_next(uint32_t x, uint32_t q, const uint2& e) {
+  uint32_t qf;
+  __asm__("v_mul_u32_u24_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1"
+          : "=v"(qf)
+          : "v"(q), "v"(e.x));
+  return qf + x + ((e.x >> 5) & 0x7ffu);
 }
 
 // sbase += 2 * popcount(m) in two scalar instructions
 __device__ __forceinline__ void advance2(uint32_t& sbase, uint64_t m) {
   uint32_t c;
+  // (the compiler cannot always see that the base is wave-uniform)
+  sbase = __builtin_amdgcn_readfirstlane(sbase);
   __asm__("s_bcnt1_i32_b64 %0, %1" : "=s"(c) : "s"(m) : "scc");
   __asm__("s_lshl1_add_u32 %0, %1, %0" : "+s"(sbase) : "s"(c) : "scc");
 }
 
-// One symbol of one chain in the 64-lane format with a linear stage, table
-// entry e (enc64_entry).  An emitted word goes to LDS byte address
-// sbase + 2 * rank, where sbase (wave uniform) is where the chain's next word
-// goes and rank the number of emitting lanes below this one; a lane that
-// emits nothing writes its own dummy slot at byte address dummy.  sbase
-// advances by two bytes per emitted word.  Lanes with v false keep their
-// state and emit nothing.
-__device__ __forceinline__ void enc_step64(uint32_t& x, uint32_t& sbase, uint32_t dummy, const uint4& e,
-                                           bool v = true) {
-  const bool w = v && (x >> 16) >= (e.x >> 16);
-  const uint64_t m = __ballot(w);
-  const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-  // sbase as one scalar and the emit address computed by every lane: one
-  // v_lshl_add and one v_cndmask, no exec-mask branch around them
-  __asm__ volatile("" : "+s"(sbase));
-  uint32_t emit = sbase + 2u * rank;
-  __asm__ volatile("" : "+v"(emit));
-  uint32_t addr = w ? emit : dummy;
-  // an opaque address keeps one unconditional store (no branch)
-  __asm__ volatile("" : "+v"(addr));
-  *(lds_u16*)(uintptr_t)addr = (uint16_t)x;
-  x = w ? x >> 16 : x;
-  advance2(sbase, m);
-  const uint32_t xn = __umul24(enc64_quot(x, e), e.y) + x + (e.x & 0xffffu);
-  x = v ? xn : x;
+// Emits and renormalises CH chains: chain c's lanes in m[c] store the low half
+// of x[c] at LDS byte address addr[c] and shift x[c] and its quotient q[c]
+// right by 16 (floor((x >> 16) / pdf) = floor(x / pdf) >> 16).  exec is
+// narrowed per chain and set back to all lanes (every caller runs whole
+// wavefronts, with no lane masked off); s_mov does not write SCC.
+template <int CH>
+__device__ __forceinline__ void emit_renorm(const uint64_t (&m)[CH], const uint32_t (&addr)[CH], uint32_t (&x)[CH],
+                                            uint32_t (&q)[CH]) {
+  static_assert(CH == 1 || CH == 2 || CH == 4, "chains per lane");
+  if constexpr (CH == 1) {
+    __asm__ volatile(
+        "s_mov_b64 exec, %2\n\tds_write_b16 %3, %0\n\tv_lshrrev_b32 %0, 16, %0\n\tv_lshrrev_b32 %1, 16, %1\n\t"
+        "s_mov_b64 exec, -1"
+        : "+v"(x[0]), "+v"(q[0])
+        : "s"(m[0]), "v"(addr[0])
+        : "memory");
+  } else {
+#pragma unroll
+    for (int c = 0; c < CH; c += 2)
+      __asm__ volatile(
+          "s_mov_b64 exec, %4\n\tds_write_b16 %5, %0\n\tv_lshrrev_b32 %0, 16, %0\n\tv_lshrrev_b32 %1, 16, %1\n\t"
+          "s_mov_b64 exec, %6\n\tds_write_b16 %7, %2\n\tv_lshrrev_b32 %2, 16, %2\n\tv_lshrrev_b32 %3, 16, %3\n\t"
+          "s_mov_b64 exec, -1"
+          : "+v"(x[c]), "+v"(q[c]), "+v"(x[c + 1]), "+v"(q[c + 1])
+          : "s"(m[c]), "v"(addr[c]), "s"(m[c + 1]), "v"(addr[c + 1])
+          : "memory");
+  }
 }
 
-// enc_step64 for a step where every lane codes a symbol, written with
-// sub-dword operand selects: the threshold compare reads the high halves of
-// x and e.x, the renormalising shift is a select of x's high half, and cdf
-// is added from e.x's low half.
-__device__ __forceinline__ void enc_step64f(uint32_t& x, uint32_t& sbase, uint32_t dummy, const uint4& e) {
-  uint64_t m;
-  uint32_t xr;
-  __asm__(
-      "v_cmp_ge_u32_sdwa vcc, %2, %3 src0_sel:WORD_1 src1_sel:WORD_1\n\t"
-      "v_cndmask_b32_sdwa %1, %2, %2, vcc dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1\n\t"
-      "s_mov_b64 %0, vcc"
-      : "=s"(m), "=&v"(xr)
-      : "v"(x), "v"(e.x)
-      : "vcc");
-  const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-  __asm__ volatile("" : "+s"(sbase));
-  const uint32_t emit = sbase + 2u * rank;
-  // only the emitting lanes store: exec is narrowed to m for the store and
-  // restored inside the same block (s_and_saveexec also writes SCC)
-  uint64_t saved;
-  __asm__ volatile(
-      "s_and_saveexec_b64 %0, %1\n\t"
-      "ds_write_b16 %2, %3\n\t"
-      "s_mov_b64 exec, %0"
-      : "=&s"(saved)
-      : "s"(m), "v"(emit), "v"(x)
-      : "memory", "scc");
-  (void)dummy;
-  advance2(sbase, m);
-  const uint32_t xn = __umul24(enc64_quot(xr, e), e.y) + xr;
-  __asm__("v_add_u32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_0"
-          : "=v"(x)
-          : "v"(xn), "v"(e.x));
+// One symbol of each of CH chains in the 64-lane format with linear stages,
+// table entries e (enc_entry).  A lane emits when its state is at or above
+// pdf << (31 - p), that is when its quotient has reached 2^(31 - p).  Chain
+// c's emitted words go to LDS byte address sb[c] + 2 * rank, sb[c] (wave
+// uniform) where the chain's next word goes and rank the number of emitting
+// lanes below this one; sb[c] advances by two bytes per emitted word.  The
+// phases (quotients and emitting lanes; ranks; stores and renormalisation;
+// next states) each run over all chains, so the dependent operations of one
+// chain have the others' between them.  13 vector operations a symbol bound
+// the step (about 4.2 cycles each per SIMD).  FULL: every lane codes a
+// symbol; else lanes with v[c] false keep their state and emit nothing.
+template <int PB, int CH, bool FULL = true>
+__device__ __forceinline__ void enc_steps64(uint32_t (&x)[CH], uint32_t (&sb)[CH], const uint2 (&e)[CH],
+                                            const bool (&v)[CH]) {
+  uint64_t m[CH];
+  uint32_t q[CH], addr[CH], x0[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    q[c] = enc_quot(x[c], e[c]);
+    m[c] = __ballot((FULL || v[c]) && q[c] >= (1u << (31 - PB)));
+    x0[c] = x[c];
+  }
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const uint32_t rank =
+        __builtin_amdgcn_mbcnt_hi((uint32_t)(m[c] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m[c], 0u));
+    addr[c] = sb[c] + 2u * rank;
+  }
+  emit_renorm<CH>(m, addr, x, q);
+#pragma unroll
+  for (int c = 0; c < CH; ++c) advance2(sb[c], m[c]);
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const uint32_t xn = enc_next(x[c], q[c], e[c]);
+    x[c] = FULL || v[c] ? xn : x0[c];
+  }
 }
 
-// The 32-lane format on a 64-lane wavefront: lanes 0-31 code one unit and
-// lanes 32-63 another (halfv = 0 / 1 per lane), each unit with its own stage.
-// An emitted word of the lower half goes to sbA + 2 * rank, one of the upper
-// half to sbB + 2 * (rank - emitters of the lower half); the two bases are
-// scalars, the per-lane choice one 24-bit multiply-add:
+// The 32-lane format on a 64-lane wavefront: lanes 0-31 code one unit of a
+// chain and lanes 32-63 another (halfv = 0 / 1 per lane), each unit with its
+// own stage.  An emitted word of the lower half goes to sbA + 2 * rank, one
+// of the upper half to sbB + 2 * (rank - emitters of the lower half); the two
+// bases are scalars, the per-lane choice one 24-bit multiply-add:
 // emit = (sbA + 2 rank) + halfv * (sbB - sbA - 2 lo).
 __device__ __forceinline__ uint32_t emit32(uint64_t m, uint32_t& sbA, uint32_t& sbB, uint32_t halfv) {
   const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-  uint32_t lo, hi;
-  __asm__("s_bcnt1_i32_b32 %0, %1" : "=s"(lo) : "s"((uint32_t)m) : "scc");
-  __asm__("s_bcnt1_i32_b32 %0, %1" : "=s"(hi) : "s"((uint32_t)(m >> 32)) : "scc");
-  __asm__ volatile("" : "+s"(sbA), "+s"(sbB));
-  uint32_t a2 = sbA;
-  __asm__("s_lshl1_add_u32 %0, %1, %0" : "+s"(a2) : "s"(lo) : "scc");
-  const int32_t delta = (int32_t)sbB - (int32_t)a2;
+  const uint32_t lo = (uint32_t)__popc((uint32_t)m), hi = (uint32_t)__popc((uint32_t)(m >> 32));
+  const uint32_t a2 = __builtin_amdgcn_readfirstlane(sbA + 2u * lo);
+  const int32_t delta = (int32_t)(sbB - a2);
   const uint32_t emit = (uint32_t)((int32_t)(sbA + 2u * rank) + __mul24((int32_t)halfv, delta));
   sbA = a2;
-  __asm__("s_lshl1_add_u32 %0, %1, %0" : "+s"(sbB) : "s"(hi) : "scc");
+  sbB = __builtin_amdgcn_readfirstlane(sbB + 2u * hi);
   return emit;
 }
 
-// enc_step64f for the 32-lane format (every lane codes a symbol).
-__device__ __forceinline__ void enc_step32f(uint32_t& x, uint32_t& sbA, uint32_t& sbB, uint32_t halfv,
-                                            const uint4& e) {
-  uint64_t m;
-  uint32_t xr;
-  __asm__(
-      "v_cmp_ge_u32_sdwa vcc, %2, %3 src0_sel:WORD_1 src1_sel:WORD_1\n\t"
-      "v_cndmask_b32_sdwa %1, %2, %2, vcc dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1\n\t"
-      "s_mov_b64 %0, vcc"
-      : "=s"(m), "=&v"(xr)
-      : "v"(x), "v"(e.x)
-      : "vcc");
-  const uint32_t emit = emit32(m, sbA, sbB, halfv);
-  uint64_t saved;
-  __asm__ volatile(
-      "s_and_saveexec_b64 %0, %1\n\t"
-      "ds_write_b16 %2, %3\n\t"
-      "s_mov_b64 exec, %0"
-      : "=&s"(saved)
-      : "s"(m), "v"(emit), "v"(x)
-      : "memory", "scc");
-  const uint32_t xn = __umul24(enc64_quot(xr, e), e.y) + xr;
-  __asm__("v_add_u32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_0"
-          : "=v"(x)
-          : "v"(xn), "v"(e.x));
+// enc_steps64 for the 32-lane format: chain c's lower half advances sb[c],
+// its upper half sb[CH + c].
+template <int PB, int CH, bool FULL = true>
+__device__ __forceinline__ void enc_steps32(uint32_t (&x)[CH], uint32_t (&sb)[2 * CH], uint32_t halfv,
+                                            const uint2 (&e)[CH], const bool (&v)[CH]) {
+  uint64_t m[CH];
+  uint32_t q[CH], addr[CH], x0[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    q[c] = enc_quot(x[c], e[c]);
+    m[c] = __ballot((FULL || v[c]) && q[c] >= (1u << (31 - PB)));
+    x0[c] = x[c];
+  }
+#pragma unroll
+  for (int c = 0; c < CH; ++c) addr[c] = emit32(m[c], sb[c], sb[CH + c], halfv);
+  emit_renorm<CH>(m, addr, x, q);
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const uint32_t xn = enc_next(x[c], q[c], e[c]);
+    x[c] = FULL || v[c] ? xn : x0[c];
+  }
 }
 
-// enc_step64 (lanes with v false keep their state) for the 32-lane format.
-__device__ __forceinline__ void enc_step32(uint32_t& x, uint32_t& sbA, uint32_t& sbB, uint32_t halfv, uint32_t dummy,
-                                           const uint4& e, bool v) {
-  const bool w = v && (x >> 16) >= (e.x >> 16);
-  const uint64_t m = __ballot(w);
-  uint32_t emit = emit32(m, sbA, sbB, halfv);
-  __asm__ volatile("" : "+v"(emit));
-  uint32_t addr = w ? emit : dummy;
-  __asm__ volatile("" : "+v"(addr));
-  *(lds_u16*)(uintptr_t)addr = (uint16_t)x;
-  x = w ? x >> 16 : x;
-  const uint32_t xn = __umul24(enc64_quot(x, e), e.y) + x + (e.x & 0xffffu);
-  x = v ? xn : x;
-}
-
-// 16 * byte B of w: a byte offset into a table of 16-byte entries.
+// 8 * byte B of w: a byte offset into a table of 8-byte entries.
 template <int B>
-__device__ __forceinline__ uint32_t byte_x16(uint32_t w) {
+__device__ __forceinline__ uint32_t byte_x8(uint32_t w) {
   uint32_t r;
   if constexpr (B == 0)
-    __asm__("v_lshlrev_b32_sdwa %0, 4, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_0"
+    __asm__("v_lshlrev_b32_sdwa %0, 3, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_0"
             : "=v"(r) : "v"(w));
   else if constexpr (B == 1)
-    __asm__("v_lshlrev_b32_sdwa %0, 4, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_1"
+    __asm__("v_lshlrev_b32_sdwa %0, 3, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_1"
             : "=v"(r) : "v"(w));
   else if constexpr (B == 2)
-    __asm__("v_lshlrev_b32_sdwa %0, 4, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_2"
+    __asm__("v_lshlrev_b32_sdwa %0, 3, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_2"
             : "=v"(r) : "v"(w));
   else
-    __asm__("v_lshlrev_b32_sdwa %0, 4, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_3"
+    __asm__("v_lshlrev_b32_sdwa %0, 3, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_3"
             : "=v"(r) : "v"(w));
   return r;
 }
@@ -297,7 +289,7 @@ __device__ __forceinline__ uint64_t look_back_window(const uint64_t* status, int
     excl += wave_sum(part);
     if (found) return excl;
     j -= 64 * groups;
-    if (groups < K) __builtin_amdgcn_s_sleep(1);
+    if (groups < K) __builtin_amdgcn_s_sleep(SLEEPX);
   }
 }
 

@@ -5,42 +5,47 @@
 // :180-284 (ansEncodeCoalesceBatch).  The reference encodes each 4 KiB block
 // into an uncoalesced staging buffer in HBM, scans the word counts with up to
 // three launches (limit 512^2 blocks) and copies every block again into the
-// final container.  Here one persistent launch does all of it:
-//  * a wavefront takes a ticket (atomic counter) for a group of units: the
-//    CH planes of one element block (two blocks, one per half-wave, in the
-//    32-lane reference format), taking the next one when it is done.  Each
-//    lane runs CH independent rANS chains, one per byte plane, fed
-//    by a single element load per step, so the serial per-chain dependency is
-//    interleaved CH ways;
-//  * element loads are software-pipelined: the next 16 steps are in flight
-//    while the current 16 are coded, and the table entries of a step are read
-//    one step ahead;
+// final container.  Here one persistent launch does all of it
+// (encode_mc_kernel):
+//  * a workgroup takes a ticket (atomic counter) for a run of units, each
+//    coding wavefront a few of them.  Each lane runs CH independent rANS
+//    chains, one per unit, fed by the same element loads where units are byte
+//    planes of one block, so the serial per-chain dependency is interleaved;
+//  * elements arrive 16 bytes a lane, two chunks ahead, and pass through LDS;
+//    the table entries of a step are read one step ahead;
 //  * emitted 16-bit words are compacted in lane order within each step
-//    (64-bit ballot + mbcnt) into LDS.  In the 64-lane format a chain keeps
-//    a linear stage of H + 256 words: at most every 4 steps, once H words are
-//    waiting, they go to one of the wave's two spill slots in HBM and the
-//    rest moves to the front, so a wave needs a few KiB of LDS and many waves
-//    stay resident.  The 32-lane format stages units whole (bounded by
-//    lane_max_words);
-//  * the wave publishes its padded word count and resolves its output offset
-//    by decoupled look-back over earlier tickets, 512 of them per round trip
-//    (tickets are taken by running waves, so every wave waited on is resident
-//    and finishes).  In the 64-lane format the look-back of a ticket runs
-//    only after the wave has coded its next ticket, so it rarely waits;
-//  * it then writes states, block words and the unit's words straight to
-//    their final place, 16 bytes per lane per store.
+//    (64-bit ballot + mbcnt) into a linear LDS stage of H + 256 words a
+//    unit: at most every 4 steps, once H words are waiting, they go to a
+//    spill slot in HBM and the rest moves to the front, so a wave needs a few
+//    KiB of LDS and many waves stay resident;
+//  * an extra wavefront per workgroup publishes each ticket's padded word
+//    count and resolves its output offset by decoupled look-back over earlier
+//    tickets (tickets are taken by running workgroups, so every ticket waited
+//    on belongs to a resident one and finishes), while the others code on;
+//  * the units' words then go from the slot straight to their final place, 16
+//    bytes per lane per store.
+// encode_kernel is the 32-lane coder without spill slots: units staged whole
+// in LDS (bounded by lane_max_words), used by the allocation-free entry point
+// and for concatenated planes.
 // The arithmetic per symbol is the reference's: emit x & 0xffff when
-// x >= pdf * 2^(31-p); q = (umulhi(x, magic) + x) >> shift = x / pdf;
-// x = q * 2^p + (x - q * pdf) + cdf, computed as x + q * (2^p - pdf) + cdf.
+// x >= pdf * 2^(31-p); q = x / pdf; x = q * 2^p + (x - q * pdf) + cdf,
+// computed as x + q * (2^p - pdf) + cdf.
 #include "codec_device.hpp"
 
 namespace mans {
 namespace {
 
 constexpr int kBatch = 16;  // steps per prefetch batch
+// encode_mc_kernel: spill slots of a coding wavefront (on 1 GiB of uint16
+// codes 3 and 4 slots take 0.62 ms, 6 no less, 2 0.84: with one ticket of
+// slack every workgroup waits for the slowest), and workgroups per CU
+constexpr uint32_t kEncSlots = 4;
+constexpr int kEncGroups = 4;
 
 template <typename T>
 using gptr = const __attribute__((address_space(1))) T*;
+template <typename T>
+using lds_ptr = __attribute__((address_space(3))) T*;
 // 16 bytes as a native vector: arrays of it stay in registers
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -302,57 +307,81 @@ __global__ __launch_bounds__(64 * NW) void encode_kernel(EncodeArgs a) {
   }
 }
 
-// The multi-chain coder, for both formats.  A ticket is BPT consecutive
-// element blocks per unit half (CH = S * BPT consecutive units: the S planes
-// of each block), one chain per unit per lane, so a lane runs several
-// interleaved chains whatever the element width.  In the 64-lane format a
-// wavefront codes CH units; in the 32-lane format it codes 2 CH, lanes 0-31
-// the first CH and lanes 32-63 the next CH (the units of one chain are
-// "streams" h * CH + c, h the half).  A stream's words go to a linear LDS
-// stage of H + 256 words; once H are waiting (checked at most 4 steps apart)
-// they go to the wave's spill slot in HBM and the rest moves to the front.
-// When the ticket is coded, the stage's remainder follows them, so the slot
-// holds all of the ticket's words, padded, and the wave publishes its
-// aggregate.  The offset is resolved only after the NEXT ticket has been
-// coded (two slots per wave, used in turn): by then the predecessors have
-// had a whole ticket's time to publish their own aggregates, so the
-// look-back sums published entries instead of waiting for the slowest wave
-// still coding.  The copy to the final place issues a batch of loads before
-// any store.  (32 lanes: unit order 0 or single streams only, so both halves
-// of a chain share its plane.)
+// The multi-chain coder, for both formats.  A workgroup is NW coding
+// wavefronts and one placing wavefront.  A ticket (one atomic, one look-back
+// entry) is NW x NS consecutive units; a coding wavefront's NS units are BPT
+// consecutive element blocks per unit half (CH = S * BPT chains a lane: the S
+// planes of each block).  In the 64-lane format a wavefront codes CH units;
+// in the 32-lane format 2 CH, lanes 0-31 the first CH and lanes 32-63 the
+// next CH (the units of one chain are "streams" h * CH + c, h the half).  A
+// stream's words go to a linear LDS stage of H + 256 words; once H are
+// waiting (checked at most 4 steps apart) they go to the wave's spill slot
+// in HBM and the rest moves to the front.  When the ticket is coded the
+// stage's remainder follows them, so the slot holds all of the unit's words,
+// padded.
+//
+// One barrier a ticket hands its padded word counts to the resolving
+// wavefront, which publishes their sum, resolves the offsets of coded tickets
+// in turn (decoupled look-back) and writes their units' block word offsets
+// while the coding wavefronts code the next ticket into the next of NSLOT
+// slots.  After each barrier a coding wavefront copies its units of the
+// tickets resolved by then from their slots to their final place; a ticket
+// has to be resolved only when its slot is needed again.
+//
+// What bounds it: memory.  A unit's words are written to the slot, read back
+// and written out (2.6 GB for 1 GiB of codes of ratio 2.1, the 1.6 GB of input
+// and output and twice the output): 0.56 ms, 4.6 TB/s against the 4.7 of a
+// large copy; with every load and store taken out of the loop the steps take
+// 0.39 ms.  (Before: a ticket per wavefront, its look-back and the next
+// ticket's atomic in the coding wavefronts' way, the chains' steps one after
+// another, table entries of 16 bytes: 0.69 ms.  Atomics on one address run at
+// 11 ns each whatever their number.)
+// (32 lanes: unit order 0 or single streams only, so both halves of a chain
+// share its plane.)
 template <int L, int PB, int S, int BPT, int NW, int HB>
-__global__ __launch_bounds__(64 * NW, L == 32 ? 3 : 4) void encode_mc_kernel(EncodeArgs a) {
+__global__ __launch_bounds__(64 * (NW + 1), 5) void encode_mc_kernel(EncodeArgs a) {
   constexpr int CH = S * BPT;                     // chains per lane
   constexpr int HALVES = L == 32 ? 2 : 1;
-  constexpr int NS = CH * HALVES;                 // streams (units) per ticket
-  constexpr int KB = 8 / BPT < 4 ? 4 : 8 / BPT;  // steps per prefetch batch (elements loaded ahead per block)
+  constexpr int NS = CH * HALVES;                 // streams (units) per coding wavefront
+  constexpr int CK = 16 / S;          // steps per input chunk: a 16-byte load per lane and block
+  constexpr int KB = CK < 8 ? CK : 8;  // steps per batch of symbols in registers
+  constexpr int DP = 2;               // chunks loaded ahead
   constexpr uint32_t BLOCK = L == 32 ? 4096u : 8192u;
   constexpr uint32_t CSTAGE = chain_stage_words<PB>();
   constexpr uint32_t SSTAGE = CSTAGE / HALVES;    // a unit's words at most, rounded
   constexpr uint32_t H = 1u << HB;  // spill chunk words
   constexpr uint32_t H4 = H / 8;    // spill chunk uint4s
   constexpr uint32_t REG = H + 256u;  // LDS stage words per stream
-  constexpr uint32_t SLOT = CH * CSTAGE;  // spill slot words
+  constexpr uint32_t SLOT = CH * CSTAGE;  // spill slot words of a coding wavefront
+  constexpr uint32_t TU = NW * NS;        // units per ticket
+  constexpr uint32_t NSLOT = kEncSlots;   // tickets coded and not yet placed, with the one being coded
+  constexpr int NT = 64 * (NW + 1);
   constexpr int CB = 8;  // copy batch: uint4 loads per lane in flight
   constexpr int TP = L == 32 ? S : (S > 1 ? S : kMaxPlanes);  // tables held
-  static_assert(BPT == 1 || (S < 4 && BLOCK / L % KB == 0), "blocks per ticket");
+  constexpr uint32_t IN = BPT * 1024u;  // LDS bytes of a chunk per wavefront
+  static_assert(BLOCK / L % CK == 0, "whole chunks per block");
   static_assert(H >= 256 && H4 <= 64, "256 <= spill chunk <= 512 words");
   static_assert(CSTAGE % 16 == 0 && SSTAGE % 8 == 0 && REG % 8 == 0, "uint4-aligned areas");
+  static_assert(TU <= 64 && TU % S == 0, "a lane of the resolving wavefront per unit");
   extern __shared__ uint4 smem[];
   __shared__ LanePlane s_pl[kMaxPlanes];
   __shared__ uint64_t s_ubase[kMaxPlanes + 1];
+  // per slot, of the ticket in it: its number and each unit's padded words;
+  // once resolved, its offset and each unit's within it
+  __shared__ uint32_t s_tk[NSLOT], s_pad[NSLOT][TU], s_ex[NSLOT][TU];
+  __shared__ uint64_t s_excl[NSLOT];
+  // the next ticket and the group's tickets resolved so far (of two tickets
+  // in turn); the ticket (counted from 1) whose coding is nearly done
+  __shared__ uint32_t s_next[2], s_res[2], s_near;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int P = a.d.num_planes;
   const uint32_t half = L == 32 ? (uint32_t)(lane >> 5) : 0u;
   const uint32_t lin = (uint32_t)lane & (L - 1);
 
-  // [P][256] entries of enc64_entry, at a fixed LDS address so each chain's
+  // [P][256] entries of enc_entry, at a fixed LDS address so each chain's
   // base is an immediate offset of its reads
-  __shared__ uint4 s_tab[TP * kNumSymbols];
-  for (int i = t; i < P * (int)kNumSymbols; i += 64 * NW) {
-    const uint4 e = a.table[i];
-    s_tab[i] = enc64_entry(e.x, e.y, PB);
-  }
+  __shared__ uint2 s_tab[TP * kNumSymbols];
+  for (int i = t; i < P * (int)kNumSymbols; i += NT) s_tab[i] = enc_entry(a.table[i], PB);
   if (t < P) {
     s_pl[t].src = a.d.plane[t].src;
     s_pl[t].nsym = a.d.plane[t].nsym;
@@ -360,41 +389,157 @@ __global__ __launch_bounds__(64 * NW, L == 32 ? 3 : 4) void encode_mc_kernel(Enc
     s_pl[t].nb = a.d.plane[t].nb;
     s_ubase[t] = a.d.plane[t].unit_base;
   }
-  if (t == 0) s_ubase[P] = a.d.total_units;
+  if (t == 0) {
+    s_ubase[P] = a.d.total_units;
+    s_next[1] = atomicAdd(a.ticket, TU);
+    s_near = 0;
+  }
   __syncthreads();
 
-  // staging: per wave, NS stages of REG words, then one dword-spaced dummy
-  // slot per lane
   const uint32_t wave_u = __builtin_amdgcn_readfirstlane((uint32_t)wave);
-  uint16_t* wstage = (uint16_t*)smem + wave_u * (NS * REG + 128);
-  const uint32_t dummy_addr = lds_addr(wstage + NS * REG + 2u * (uint32_t)lane);
-  // this wave's two spill slots of NS streams of SSTAGE words
-  uint16_t* const spill = a.spill + ((uint64_t)blockIdx.x * NW + wave_u) * (2 * SLOT);
-  uint32_t ptot[kMaxPlanes];  // words coded per plane by this wave
-#pragma unroll
-  for (int k = 0; k < kMaxPlanes; ++k) ptot[k] = 0;
+  // the group's spill: per coding wavefront NSLOT slots of NS streams of
+  // SSTAGE words
+  uint16_t* const gspill = a.spill + (uint64_t)blockIdx.x * NW * (NSLOT * SLOT);
+  // plane and block of a unit
+  auto plane_of = [&](uint64_t unit, int& k, uint64_t& b) {
+    if (a.d.order == 0) {  // planes of one element array: P is 1, 2 or 4
+      k = (int)((uint32_t)unit & (uint32_t)(P - 1));
+      b = unit >> (P == 4 ? 2 : (P == 2 ? 1 : 0));
+    } else {
+      k = 0;
+      while (k + 1 < P && unit >= s_ubase[k + 1]) ++k;
+      b = unit - s_ubase[k];
+    }
+  };
 
-  // the ticket coded last, whose offset is not resolved yet (wave-uniform)
-  bool pend = false;
-  uint32_t p_tk = 0, p_slot = 0;
-  uint64_t p_agg = 0;
-  uint32_t p_pad[NS];
-  uint64_t p_bw[NS];  // byte offset of the unit's block-word pair, 0: inactive
-#pragma unroll
-  for (int c = 0; c < NS; ++c) p_pad[c] = 0, p_bw[c] = 0;
+  uint32_t tk = __builtin_amdgcn_readfirstlane(s_next[1]);
+  uint32_t it = 0;  // the group's tickets coded: ticket it goes to slot it % NSLOT
 
-  // resolve the pending ticket's offset, write its units' word offsets and
-  // copy its words from its slot to their final place
-  auto finish_pending = [&]() {
-    uint32_t qb[NS + 1];  // first uint4 of each stream in the ticket's output
+  if (wave_u == NW) {
+    // ---- the resolving wavefront: lane u handles unit u of a ticket --------
+    uint32_t ptot[kMaxPlanes];  // words of this lane's units per plane
+#pragma unroll
+    for (int k = 0; k < kMaxPlanes; ++k) ptot[k] = 0;
+    auto tk_of = [&](uint32_t sl) { return (uint32_t)__builtin_amdgcn_readfirstlane(s_tk[sl]); };
+    // the units' offsets within the ticket in slot sl and its words
+    auto scan = [&](uint32_t sl, uint32_t& pw, uint32_t& ex) -> uint32_t {
+      pw = (uint32_t)lane < TU ? s_pad[sl][lane] : 0u;
+      uint32_t inc = pw;
+#pragma unroll
+      for (int o = 1; o < (int)TU; o <<= 1) {
+        const uint32_t v = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += v;
+      }
+      ex = inc - pw;
+      return __builtin_amdgcn_readlane(inc, TU - 1);
+    };
+    // resolves the ticket in slot sl; with TRY, returns false if one of its
+    // predecessors has not yet published
+    auto resolve = [&](uint32_t sl, auto try_) -> bool {
+      constexpr bool TRY = decltype(try_)::value;
+      const uint32_t p_tk = tk_of(sl);
+      const uint64_t tix = p_tk / TU;
+      uint32_t pw, ex;
+      const uint32_t total = scan(sl, pw, ex);
+      uint64_t excl = 0;
+      if (tix > 0) {
+        excl = look_back_window<8, TRY>(a.status, (int64_t)tix - 1, 0, kFlagPrefix, lane,
+                                        [](uint64_t v, uint32_t& f, uint64_t& val) {
+                                          f = (uint32_t)(v >> 62);
+                                          val = v & kValueMask;
+                                        });
+        if (TRY && excl == ~0ull) return false;
+        if (lane == 0)
+          __hip_atomic_store(a.status + tix, kFlagPrefix | (excl + total), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      if ((uint32_t)lane < TU) s_ex[sl][lane] = ex;
+      if (lane == 0) s_excl[sl] = excl;
+      const uint64_t unit = (uint64_t)p_tk + lane;
+      if ((uint32_t)lane < TU && unit < a.d.total_units) {
+        int k;
+        uint64_t b;
+        plane_of(unit, k, b);
+        const LanePlane& pl = s_pl[k];
+        ((uint32_t*)(a.out + pl.section + kSectionFixed + 4ull * L * pl.nb + 8ull * b))[1] = (uint32_t)(excl + ex);
+#pragma unroll
+        for (int q = 0; q < kMaxPlanes; ++q) ptot[q] += k == q ? pw : 0u;
+      }
+      if ((uint64_t)p_tk + TU >= a.d.total_units && lane == 0) {
+        const uint64_t total_words = excl + total;
+        const uint64_t size = a.d.data_off + 2ull * total_words;
+        if (a.d_out_size32) *a.d_out_size32 = (uint32_t)size;
+        if (a.d_out_size64) *a.d_out_size64 = size;
+        if (a.frame) {
+          ((uint64_t*)a.out)[6] = total_words;  // data_words at byte 48
+          ((uint64_t*)a.out)[7] = size;         // total_size at byte 56
+        }
+      }
+      return true;
+    };
+    auto publish = [&](uint32_t i) {
+      uint32_t pw, ex;
+      const uint32_t total = scan(i % NSLOT, pw, ex);
+      publish_aggregate(a.status, tk_of(i % NSLOT) / TU, total, lane);
+    };
+    uint32_t res = 0;  // tickets resolved
+    while ((uint64_t)tk < a.d.total_units) {
+      if (lane == 0) s_tk[it % NSLOT] = tk;
+      if (it > 0) publish(it - 1);
+      // the ticket after this one goes to slot (it + 1) % NSLOT, whose
+      // ticket must be resolved (the coding wavefronts place it after the
+      // barrier); the others if they can be
+      while (res + NSLOT < it + 2) {
+        resolve(res % NSLOT, std::false_type{});
+        ++res;
+      }
+      while (res < it && resolve(res % NSLOT, std::true_type{})) ++res;
+      // the next ticket, taken shortly before it is needed: groups run at
+      // different rates, and a ticket held long before it is coded keeps
+      // those after it waiting.  (The launch drains: the lowest unpublished
+      // ticket is being coded, or its group waits only for lower ones, all
+      // of them published.)
+      while (__hip_atomic_load(&s_near, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != it + 1)
+        __builtin_amdgcn_s_sleep(4);
+      if (lane == 0) {
+        s_next[it & 1u] = atomicAdd(a.ticket, TU);
+        s_res[it & 1u] = res;
+      }
+      __syncthreads();
+      tk = __builtin_amdgcn_readfirstlane(s_next[it & 1u]);
+      ++it;
+    }
+    if (it > 0) publish(it - 1);
+    for (; res < it; ++res) resolve(res % NSLOT, std::false_type{});
+    __syncthreads();
+    // total coded words of each plane (the section headers start at 0)
+#pragma unroll
+    for (int k = 0; k < kMaxPlanes; ++k) {
+      if (k < P) {
+        const uint32_t v = wave_sum32(ptot[k]);
+        if (lane == 0 && v) atomicAdd((uint32_t*)(a.out + s_pl[k].section + 12), v);
+      }
+    }
+    return;
+  }
+
+  // ---- a coding wavefront: staging NS stages of REG words ------------------
+  uint16_t* wstage = (uint16_t*)smem + wave_u * (NS * REG);
+  const uint32_t win = lds_addr(smem) + NW * NS * REG * 2u + wave_u * IN;  // the chunk being coded (LDS address)
+  uint16_t* const spill = gspill + wave_u * (NSLOT * SLOT);
+  // Copies this wavefront's units of the resolved ticket in slot sl to their
+  // final place, a batch of loads before any store.  (The slot was written
+  // by other lanes of this wavefront, before a barrier.)
+  auto place = [&](uint32_t sl) {
+    const u32x4* s4 = (const u32x4*)(spill + sl * SLOT);
+    uint32_t qb[NS + 1];  // first uint4 of each stream in the wavefront's output
     qb[0] = 0;
 #pragma unroll
-    for (int c = 0; c < NS; ++c) qb[c + 1] = qb[c] + p_pad[c] / 8;
+    for (int c = 0; c < NS; ++c)
+      qb[c + 1] = qb[c] + __builtin_amdgcn_readfirstlane(s_pad[sl][wave_u * NS + c]) / 8;
     const uint32_t nq = qb[NS];
-    // the slot was written by other lanes of this wave: their stores first
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    const u32x4* s4 = (const u32x4*)(spill + p_slot * SLOT);
-    auto load = [&](u32x4 (&q)[CB], uint32_t j0) {
+    u32x4* const dst = (u32x4*)(a.out + a.d.data_off + 2ull * (s_excl[sl] + s_ex[sl][wave_u * NS]));
+    for (uint32_t j0 = 0; j0 < nq; j0 += CB * 64) {
+      u32x4 q[CB];
 #pragma unroll
       for (int u = 0; u < CB; ++u) {
         if (j0 + u * 64 < nq) {  // wave-uniform
@@ -408,50 +553,19 @@ __global__ __launch_bounds__(64 * NW, L == 32 ? 3 : 4) void encode_mc_kernel(Enc
           q[u] = s4[jj + d];
         }
       }
-    };
-    auto store = [&](const u32x4 (&q)[CB], u32x4* dst, uint32_t j0) {
 #pragma unroll
       for (int u = 0; u < CB; ++u) {
         const uint32_t j = j0 + u * 64 + (uint32_t)lane;
-        if (j < nq) dst[j] = q[u];
-      }
-    };
-    // the first batch is in flight during the look-back
-    u32x4 q[CB];
-    load(q, 0);
-    const uint64_t excl = resolve_prefix<4>(a.status, p_tk / NS, p_agg, lane);
-    uint64_t y = excl;
-#pragma unroll
-    for (int c = 0; c < NS; ++c) {
-      if (p_bw[c] && lane == 0) ((uint32_t*)(a.out + p_bw[c]))[1] = (uint32_t)y;
-      y += p_pad[c];
-    }
-    u32x4* dst = (u32x4*)(a.out + a.d.data_off + 2ull * excl);
-    store(q, dst, 0);
-    for (uint32_t j0 = CB * 64; j0 < nq; j0 += CB * 64) {
-      load(q, j0);
-      store(q, dst, j0);
-    }
-    if ((uint64_t)p_tk + NS >= a.d.total_units && lane == 0) {
-      const uint64_t total_words = excl + p_agg;
-      const uint64_t size = a.d.data_off + 2ull * total_words;
-      if (a.d_out_size32) *a.d_out_size32 = (uint32_t)size;
-      if (a.d_out_size64) *a.d_out_size64 = size;
-      if (a.frame) {
-        ((uint64_t*)a.out)[6] = total_words;  // data_words at byte 48
-        ((uint64_t*)a.out)[7] = size;         // total_size at byte 56
+        if (j < nq) __builtin_nontemporal_store(q[u], dst + j);
       }
     }
   };
-
-  uint32_t slot = 0;
-  uint32_t tk = 0;
-  if (lane == 0) tk = atomicAdd(a.ticket, NS);
-  tk = __builtin_amdgcn_readfirstlane(tk);
+  uint32_t placed = 0;  // the group's tickets placed
   while ((uint64_t)tk < a.d.total_units) {
+    const uint32_t slot = it % NSLOT;
     // per chain (this lane's half): unit, plane, block, symbols
     uint32_t x[CH], n[CH];
-    const uint4* tab[CH];
+    const uint2* tab[CH];
     uint64_t blk[CH];
     int kp[CH];
     bool act[CH];
@@ -462,19 +576,11 @@ __global__ __launch_bounds__(64 * NW, L == 32 ? 3 : 4) void encode_mc_kernel(Enc
     uint16_t* const wslot = spill + slot * SLOT;
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      const uint64_t unit = (uint64_t)tk + half * CH + c;
+      const uint64_t unit = (uint64_t)tk + wave_u * NS + half * CH + c;
       act[c] = unit < a.d.total_units;
       int k = 0;
       uint64_t b = 0;
-      if (act[c]) {
-        if (a.d.order == 0) {  // planes of one element array: P is 1, 2 or 4
-          k = (int)((uint32_t)unit & (uint32_t)(P - 1));
-          b = unit >> (P == 4 ? 2 : (P == 2 ? 1 : 0));
-        } else {
-          while (k + 1 < P && unit >= s_ubase[k + 1]) ++k;
-          b = unit - s_ubase[k];
-        }
-      }
+      if (act[c]) plane_of(unit, k, b);
       kp[c] = k;
       blk[c] = b;
       const LanePlane pl = s_pl[k];
@@ -490,7 +596,7 @@ __global__ __launch_bounds__(64 * NW, L == 32 ? 3 : 4) void encode_mc_kernel(Enc
 #pragma unroll
     for (int c = 0; c < NS; ++c) {
       fl[c] = 0;
-      cb[c] = lds_addr(wstage + c * REG);
+      cb[c] = lds_addr(smem) + (wave_u * NS + (uint32_t)c) * REG * 2u;  // = wstage + c * REG
       sb[c] = cb[c];
     }
     uint32_t n_min = n[0], n_max = n[0];
@@ -523,13 +629,10 @@ __global__ __launch_bounds__(64 * NW, L == 32 ? 3 : 4) void encode_mc_kernel(Enc
         }
       }
     };
-    auto step_full = [&](int c, const uint4& e) {
-      if constexpr (L == 64) enc_step64f(x[c], sb[c], dummy_addr, e);
-      else enc_step32f(x[c], sb[c], sb[CH + c], half, e);
-    };
-    auto step_part = [&](int c, const uint4& e, bool v) {
-      if constexpr (L == 64) enc_step64(x[c], sb[c], dummy_addr, e, v);
-      else enc_step32(x[c], sb[c], sb[CH + c], half, dummy_addr, e, v);
+    auto steps = [&](const uint2 (&e)[CH], const bool (&v)[CH], auto full) {
+      constexpr bool FULL = decltype(full)::value;
+      if constexpr (L == 64) enc_steps64<PB, CH, FULL>(x, sb, e, v);
+      else enc_steps32<PB, CH, FULL>(x, sb, half, e, v);
     };
 
     {
@@ -542,43 +645,60 @@ __global__ __launch_bounds__(64 * NW, L == 32 ? 3 : 4) void encode_mc_kernel(Enc
 #pragma unroll
       for (int d = 0; d < BPT; ++d) eb[d] = src[d * S] + blk[d * S] * BLOCK * S;
       uint32_t s = 0;
-      // Full blocks: each lane loads its element of each block
-      // (zero-extended: byte b of the register is byte b of the element).
-      // Two register buffers: while one batch is coded the next is loading.
+      // Whole chunks: CK steps of each block are 1 KiB (512 B per half), read
+      // with one 16-byte load per lane and passed through LDS, where each
+      // lane then finds its element of every step.  (Elements loaded one by
+      // one, 128 B a load and 8 steps ahead: 0.58 ms on 1 GiB of uint16
+      // codes.)
       using EL = typename ElemOf<S>::T;
-      auto load = [&](uint32_t (&buf)[BPT][KB], uint32_t s0) {
+      typedef uint32_t u32x4a __attribute__((ext_vector_type(4), aligned(4)));  // inputs are 4-byte aligned
+      auto load = [&](u32x4 (&r)[BPT], uint32_t s0) {
 #pragma unroll
-        for (int d = 0; d < BPT; ++d) {
-          const gptr<EL> bp = (gptr<EL>)eb[d] + lin + (uint64_t)s0 * L;
+        for (int d = 0; d < BPT; ++d)
+          r[d] = __builtin_nontemporal_load((const __attribute__((address_space(1))) u32x4a*)(eb[d] + (uint64_t)s0 * L * S + lin * 16u));
+      };
+      auto stash = [&](const u32x4 (&r)[BPT]) {
 #pragma unroll
-          for (int j = 0; j < KB; ++j) buf[d][j] = bp[j * L];
-        }
+        for (int d = 0; d < BPT; ++d) *(lds_ptr<u32x4>)(uintptr_t)(win + d * 1024u + (uint32_t)lane * 16u) = r[d];
+      };
+      // steps j0 .. j0 + KB - 1 of the chunk in LDS
+      auto unpack = [&](uint32_t (&buf)[BPT][KB], uint32_t j0) {
+        const uint32_t at = win + half * 512u + (j0 * L + lin) * S;
+#pragma unroll
+        for (int d = 0; d < BPT; ++d)
+#pragma unroll
+          for (int j = 0; j < KB; ++j) buf[d][j] = *(lds_ptr<EL>)(uintptr_t)(at + d * 1024u + j * L * S);
       };
       // table entries of the chains for step j of a batch
-      auto lookup = [&](uint4 (&e)[CH], const uint32_t (&buf)[BPT][KB], int j) {
+      auto lookup = [&](uint2 (&e)[CH], const uint32_t (&buf)[BPT][KB], int j) {
 #pragma unroll
         for (int d = 0; d < BPT; ++d) {
           const uint32_t w = buf[d][j];
-          e[d * S] = *(const uint4*)((const char*)tab[d * S] + byte_x16<0>(w));
-          if constexpr (S > 1) e[d * S + 1] = *(const uint4*)((const char*)tab[d * S + 1] + byte_x16<1>(w));
+          e[d * S] = *(const uint2*)((const char*)tab[d * S] + byte_x8<0>(w));
+          if constexpr (S > 1) e[d * S + 1] = *(const uint2*)((const char*)tab[d * S + 1] + byte_x8<1>(w));
           if constexpr (S > 2) {
-            e[d * S + 2] = *(const uint4*)((const char*)tab[d * S + 2] + byte_x16<2>(w));
-            e[d * S + 3] = *(const uint4*)((const char*)tab[d * S + 3] + byte_x16<3>(w));
+            e[d * S + 2] = *(const uint2*)((const char*)tab[d * S + 2] + byte_x8<2>(w));
+            e[d * S + 3] = *(const uint2*)((const char*)tab[d * S + 3] + byte_x8<3>(w));
           }
         }
       };
       // The table entries of step j + 1 are read before step j is coded:
       // they depend on the symbols only, not on the states.  The stage is
       // checked every 4 steps: at most 4 * 64 words arrive in between.
-      auto code = [&](const uint32_t (&buf)[BPT][KB]) {
-        uint4 e[CH];
+      // FULL: every lane has a symbol at every step of the batch; else step
+      // s0 + j of block d has one in the lanes below nb[d].
+      auto code = [&](const uint32_t (&buf)[BPT][KB], uint32_t s0, auto full) {
+        constexpr bool FULL = decltype(full)::value;
+        uint2 e[CH];
         lookup(e, buf, 0);
 #pragma unroll
         for (int j = 0; j < KB; ++j) {
-          uint4 en[CH];
+          uint2 en[CH];
           if (j + 1 < KB) lookup(en, buf, j + 1);
+          bool v[CH];
 #pragma unroll
-          for (int c = 0; c < CH; ++c) step_full(c, e[c]);
+          for (int c = 0; c < CH; ++c) v[c] = FULL || (s0 + (uint32_t)j) * L + lin < n[c];
+          steps(e, v, full);
           if ((j & 3) == 3) spill_full();
           if (j + 1 < KB) {
 #pragma unroll
@@ -587,43 +707,69 @@ __global__ __launch_bounds__(64 * NW, L == 32 ? 3 : 4) void encode_mc_kernel(Enc
         }
       };
       static_assert(KB % 4 == 0, "stage checks at batch-relative steps 3, 7, ...");
-      // The prefetch is unconditional (the last batch reloads itself) so the
-      // wait before each batch only covers that batch's loads.  Partial blocks
-      // (one per plane) take the byte path below, which never reads past the
-      // end of the input.
-      const uint32_t nbatch = n_min == BLOCK ? BLOCK / L / KB : 0u;
-      if (nbatch > 0) {
-        const uint32_t last = (nbatch - 1) * KB;
-        uint32_t bufA[BPT][KB], bufB[BPT][KB];
-        load(bufA, 0);
-        for (;;) {
-          load(bufB, s + KB <= last ? s + KB : last);
-          code(bufA);
-          s += KB;
-          if (s > last) break;
-          load(bufA, s + KB <= last ? s + KB : last);
-          code(bufB);
-          s += KB;
-          if (s > last) break;
-        }
-      }
-      for (; s < all; ++s) {
-        const uint32_t i = s * L + lin;
+      // Chunks of CK steps where every lane of every chain has a symbol, DP of
+      // them in flight.  (Loads past the last chunk reload it, so the wait
+      // before each chunk only covers that chunk's loads.)
+      const uint32_t nchunk = n_min / (L * CK);
+      // three quarters through, the resolving wavefront takes the next ticket
+      const uint32_t near_at = nchunk >= 8 ? nchunk * 3 / 4 : ~0u;
+      auto near = [&]() {
+        if (wave_u == 0 && lane == 0) __hip_atomic_store(&s_near, it + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      };
+      if (nchunk < 8) near();
+      if (nchunk > 0) {
+        u32x4 r[DP][BPT];
 #pragma unroll
-        for (int c = 0; c < CH; ++c) {
-          const bool v = i < n[c];
-          const uint32_t sym = v ? (uint32_t)eb[c / S][(uint64_t)i * S + (c % S)] : 0u;
-          step_part(c, tab[c][sym], v);
+        for (uint32_t k = 0; k < DP; ++k) load(r[k], (k < nchunk ? k : nchunk - 1) * CK);
+        for (uint32_t c = 0; c < nchunk;) {
+#pragma unroll
+          for (uint32_t k = 0; k < DP; ++k) {
+            stash(r[k]);
+            load(r[k], (c + DP < nchunk ? c + DP : nchunk - 1) * CK);
+            if (c == near_at) near();
+#pragma unroll 1
+            for (uint32_t j0 = 0; j0 < CK; j0 += KB) {
+              uint32_t buf[BPT][KB];
+              unpack(buf, j0);
+              code(buf, c * CK + j0, std::true_type{});
+            }
+            if (++c == nchunk) break;
+          }
         }
-        spill_full();
+        s = nchunk * CK;
+      }
+      // The rest (a plane's last, partial block; the whole blocks beside it):
+      // batches whose lanes past a block's end load nothing and keep their
+      // state, also loaded one batch ahead.
+      if (s < all) {
+        auto load_part = [&](uint32_t (&buf)[BPT][KB], uint32_t s0) {
+#pragma unroll
+          for (int d = 0; d < BPT; ++d) {
+            const gptr<EL> bp = (gptr<EL>)eb[d];
+#pragma unroll
+            for (int j = 0; j < KB; ++j) {
+              const uint32_t i = (s0 + (uint32_t)j) * L + lin;
+              buf[d][j] = i < n[d * S] ? (uint32_t)bp[i] : 0u;
+            }
+          }
+        };
+        uint32_t buf[BPT][KB], nxt[BPT][KB];
+        load_part(buf, s);
+        for (;;) {
+          load_part(nxt, s + KB);
+          code(buf, s, std::false_type{});
+          s += KB;
+          if (s >= all) break;
+#pragma unroll
+          for (int d = 0; d < BPT; ++d)
+#pragma unroll
+            for (int j = 0; j < KB; ++j) buf[d][j] = nxt[d][j];
+        }
       }
     }
 
     // ---- per stream: pad, move the stage's remainder to the slot; per chain
-    // and half: states and block words; ticket aggregate
-    uint64_t agg = 0;
-    uint32_t pad[NS];
-    uint64_t bwo[NS];
+    // and half: states and block words
 #pragma unroll
     for (int c = 0; c < NS; ++c) {
       const uint32_t rem = (sb[c] - cb[c]) >> 1;  // words still in the stage
@@ -634,7 +780,7 @@ __global__ __launch_bounds__(64 * NW, L == 32 ? 3 : 4) void encode_mc_kernel(Enc
       if ((uint32_t)lane < padded - cnt) st[rem + lane] = 0;
       const uint32_t nr = (padded - fl[c]) / 8;
       for (uint32_t j = lane; j < nr; j += 64) ((uint4*)(wslot + c * SSTAGE + fl[c]))[j] = ((const uint4*)st)[j];
-      pad[c] = padded;  // set to 0 below for inactive units
+      if (lane == 0) s_pad[slot][wave_u * NS + c] = padded;  // (0 for inactive units: they code nothing)
     }
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
@@ -648,49 +794,17 @@ __global__ __launch_bounds__(64 * NW, L == 32 ? 3 : 4) void encode_mc_kernel(Enc
         const uint32_t cnt = fl[sidx] + ((sb[sidx] - cb[sidx]) >> 1);
         cnt_h = (uint32_t)h == half ? cnt : cnt_h;
       }
-      const uint64_t bw = pl.section + kSectionFixed + 4ull * L * pl.nb + 8ull * blk[c];
-      if (act[c] && lin == 0) ((uint32_t*)(a.out + bw))[0] = (n[c] << 16) | cnt_h;
-#pragma unroll
-      for (int h = 0; h < HALVES; ++h) {
-        const int sidx = h * CH + c;
-        const uint32_t src_lane = (uint32_t)h * 32u;
-        const bool ah = L == 32 ? (bool)__builtin_amdgcn_readlane((uint32_t)act[c], src_lane) : act[c];
-        const uint32_t kh = L == 32 ? __builtin_amdgcn_readlane((uint32_t)kp[c], src_lane) : (uint32_t)kp[c];
-        const uint64_t bwh =
-            L == 32 ? ((uint64_t)__builtin_amdgcn_readlane((uint32_t)(bw >> 32), src_lane) << 32) |
-                          __builtin_amdgcn_readlane((uint32_t)bw, src_lane)
-                    : bw;
-        pad[sidx] = ah ? pad[sidx] : 0u;
-        bwo[sidx] = ah ? bwh : 0ull;
-#pragma unroll
-        for (int k = 0; k < kMaxPlanes; ++k) ptot[k] += kh == (uint32_t)k ? pad[sidx] : 0u;
-      }
+      if (act[c] && lin == 0)
+        ((uint32_t*)(a.out + pl.section + kSectionFixed + 4ull * L * pl.nb + 8ull * blk[c]))[0] = (n[c] << 16) | cnt_h;
     }
-#pragma unroll
-    for (int c = 0; c < NS; ++c) agg += pad[c];
-    publish_aggregate(a.status, tk / NS, agg, lane);
-    if (pend) finish_pending();
-    pend = true;
-    p_tk = tk;
-    p_slot = slot;
-    p_agg = agg;
-#pragma unroll
-    for (int c = 0; c < NS; ++c) p_pad[c] = pad[c], p_bw[c] = bwo[c];
-    slot ^= 1u;
-    // the next ticket only once this one is published: tickets start in
-    // ticket order, and every ticket a look-back waits on belongs to a wave
-    // that is coding it
-    __threadfence_block();
-    if (lane == 0) tk = atomicAdd(a.ticket, NS);
-    tk = __builtin_amdgcn_readfirstlane(tk);
+    __syncthreads();
+    for (const uint32_t res = __builtin_amdgcn_readfirstlane(s_res[it & 1u]); placed < res; ++placed)
+      place(placed % NSLOT);
+    tk = __builtin_amdgcn_readfirstlane(s_next[it & 1u]);
+    ++it;
   }
-  if (pend) finish_pending();
-  // total coded words of each plane (the section headers start at 0)
-  if (lane == 0) {
-#pragma unroll
-    for (int k = 0; k < kMaxPlanes; ++k)
-      if (k < P && ptot[k]) atomicAdd((uint32_t*)(a.out + s_pl[k].section + 12), ptot[k]);
-  }
+  __syncthreads();
+  for (; placed < it; ++placed) place(placed % NSLOT);
 }
 
 // The whole-unit staged 32-lane kernel (encode_kernel): CH == S chains, no
@@ -722,26 +836,27 @@ hipError_t launch_mc(const EncodeArgs& a, int cu, hipStream_t s, uint64_t* need_
   constexpr uint32_t CSTAGE = chain_stage_words<PB>();
   constexpr int CH = S * BPT, NS = CH * (L == 32 ? 2 : 1);
   constexpr uint32_t REG = (1u << HB) + 256u;
-  // dynamic LDS: the staging areas (the tables are static)
-  const size_t lds = (size_t)NW * (NS * REG + 128) * 2u;
+  // dynamic LDS: the stages and the input chunks (the tables are static)
+  const size_t lds = (size_t)NW * (NS * REG * 2u + BPT * 1024u);
   int per_cu = 0;
   hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, encode_mc_kernel<L, PB, S, BPT, NW, HB>,
-                                                              64 * NW, lds);
+                                                              64 * (NW + 1), lds);
   if (e != hipSuccess) return e;
   if (per_cu < 1) per_cu = 1;
+  if (per_cu > kEncGroups) per_cu = kEncGroups;  // (more are no faster, and each has its slots)
   const uint64_t waves = div_up(a.d.total_units, NS);
   uint64_t grid = div_up(waves, NW);
   const uint64_t cap = (uint64_t)cu * (uint64_t)per_cu;
   if (grid > cap) grid = cap;
   if (grid < 1) grid = 1;
-  // two slots per wave of CH chains of 64 lanes
-  const uint64_t spill_bytes = grid * NW * 2ull * CH * CSTAGE * 2ull;
+  // kEncSlots slots per coding wavefront of CH chains of 64 lanes
+  const uint64_t spill_bytes = grid * NW * kEncSlots * CH * CSTAGE * 2ull;
   if (need_spill) {
     *need_spill = spill_bytes;
     return hipSuccess;
   }
   if (!a.spill || spill_bytes > a.spill_bytes) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((encode_mc_kernel<L, PB, S, BPT, NW, HB>), dim3((uint32_t)grid), dim3(64 * NW), lds, s, a);
+  hipLaunchKernelGGL((encode_mc_kernel<L, PB, S, BPT, NW, HB>), dim3((uint32_t)grid), dim3(64 * (NW + 1)), lds, s, a);
   return hipGetLastError();
 }
 
@@ -752,17 +867,17 @@ hipError_t launch_s(const EncodeArgs& a, int cu, hipStream_t s, uint64_t* need_s
   const int P = a.d.num_planes;
   const uint32_t S = a.d.plane[0].stride;
   if constexpr (L == 64) {
-    // four chains per lane, linear stages of 256 + 256 words: 4.3 KiB of
-    // LDS per wave
-    if (a.d.order == 0 && P == 2 && S == 2) return launch_mc<64, PB, 2, 2, 4, 8>(a, cu, s, need_spill);
+    // two chains per lane (four for uint32: its planes share the element
+    // loads), linear stages of 256 + 256 words; four coding wavefronts
+    if (a.d.order == 0 && P == 2 && S == 2) return launch_mc<64, PB, 2, 1, 4, 8>(a, cu, s, need_spill);
     if (a.d.order == 0 && P == 4 && S == 4) return launch_mc<64, PB, 4, 1, 4, 8>(a, cu, s, need_spill);
-    if (S == 1) return launch_mc<64, PB, 1, 4, 4, 8>(a, cu, s, need_spill);
+    if (S == 1) return launch_mc<64, PB, 1, 2, 4, 8>(a, cu, s, need_spill);
   } else {
     if (!staged && a.d.order == 0) {
-      // four chains per lane, two units per chain (one per half-wave)
-      if (P == 2 && S == 2) return launch_mc<32, PB, 2, 2, 4, 8>(a, cu, s, need_spill);
+      // as above, two units per chain (one per half-wave)
+      if (P == 2 && S == 2) return launch_mc<32, PB, 2, 1, 4, 8>(a, cu, s, need_spill);
       if (P == 4 && S == 4) return launch_mc<32, PB, 4, 1, 4, 8>(a, cu, s, need_spill);
-      if (P == 1 && S == 1) return launch_mc<32, PB, 1, 4, 4, 8>(a, cu, s, need_spill);
+      if (P == 1 && S == 1) return launch_mc<32, PB, 1, 2, 4, 8>(a, cu, s, need_spill);
     }
     if (a.d.order == 0 && P == 2 && S == 2) return launch_staged<L, PB, 2, 2, 2>(a, cu, s, need_spill);
     if (a.d.order == 0 && P == 4 && S == 4) return launch_staged<L, PB, 4, 4, 1>(a, cu, s, need_spill);

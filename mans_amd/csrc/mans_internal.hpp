@@ -234,7 +234,7 @@ struct BatchEncodeArgs {
   uint32_t* hist;                // [nbufs][4][256] accumulators (left zeroed)
   uint32_t* done;                // [nbufs] histogram items finished (left zeroed)
   uint32_t* ready;               // [nbufs] generation whose tables are ready
-  uint4* tables;                 // [nbufs][4][256] encoder table entries
+  uint2* tables;                 // [nbufs][4][256] encoder table entries (enc_entry)
   uint64_t* status;              // [tickets] look-back words tagged with gen
   uint32_t* ptot;                // [nbufs][4] words per plane (left zeroed)
   uint32_t* fin;                 // [nbufs] encode tickets finished (left zeroed)
@@ -349,9 +349,9 @@ struct BatchShape {
 };
 constexpr BatchShape kBatchEncodeDefault = {4, 16};
 constexpr BatchShape kBatchDecodeDefault = {4, 8};
-// LDS bytes per workgroup of a shape (encode: table | ring | dummies per
+// LDS bytes per workgroup of a shape (encode: tables | stages per
 // wave; decode: two LUTs | two rings per wave)
-constexpr uint64_t batch_encode_lds(BatchShape sh) { return (uint64_t)sh.nw * (2u * 256u * 4u + 1024u + 64u) * 4u; }
+constexpr uint64_t batch_encode_lds(BatchShape sh) { return (uint64_t)sh.nw * (2u * 256u * 2u + 1024u + 128u) * 4u; }
 constexpr uint64_t batch_decode_lds(BatchShape sh, int pb) {
   return (uint64_t)sh.nw * (2ull * (1u << pb) * 4u +
                             2ull * 2u * ((2u * (64u * sh.kb > 512u ? 64u * sh.kb : 512u)) + 64u));
