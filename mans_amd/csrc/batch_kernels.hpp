@@ -29,6 +29,7 @@
 // generation, so nothing needs clearing between launches.
 #pragma once
 #include "codec_device.hpp"
+#include "hist_device.hpp"
 
 namespace mans {
 namespace {
@@ -39,12 +40,11 @@ constexpr uint32_t kRB = 10;           // ring: 1024 words per chain
 constexpr uint32_t kR = 1u << kRB, kH = kR / 2, kMask = kR - 1;
 constexpr uint32_t kGenShift = 48;
 constexpr uint64_t kValue48 = (1ull << kGenShift) - 1;
-// per-wave LDS in 32-bit words: two encoder tables | the chains' stages; a
-// workgroup's waves together also hold the histogram phase's counters, keys
-// and flags
+// per-wave LDS in 32-bit words: two encoder tables | the chains' stages (the
+// histogram phase's counts, keys and flags take the workgroup's)
 constexpr uint32_t kTabWords = 2 * 256 * 2;
 constexpr uint32_t kStageWords = 4 * 512 / 2;
-constexpr uint32_t kWaveWords = kTabWords + kStageWords + 128;
+constexpr uint32_t kWaveWords = kTabWords + kStageWords;
 // Queue items a decode wavefront takes at once (BatchDecodeArgs::run, 1 or
 // 4): consecutive tickets of a buffer then run on one wavefront, which keeps
 // the buffer's LUTs in its LDS.  (Encode takes one at a time: a ticket's
@@ -111,100 +111,37 @@ __device__ uint64_t resolve_gen(uint64_t* status, uint64_t idx, uint64_t first, 
 
 // ---- histogram chunks -----------------------------------------------------
 // A histogram item (bytes [c0, c1) of a buffer; plane = byte offset % P) is
-// counted by a whole workgroup into its LDS counters [P][256 bins][R]
-// (32-bit words, R = 32 / P replicas, thread t adding into replica t % R:
-// the 32 lanes of an LDS pass hit at most two words of one bank, and for
-// uint8 buffers none), which it then adds to the buffer's accumulators.
-// Loads: kHistLoads 16-byte loads per thread in flight while the previous
-// ones are counted.
-constexpr uint32_t kHistCntWords = 8192;  // P x 256 x 32 / P
-constexpr int kHistLoads = 4;
-
+// counted by a whole workgroup, its whole tiles on the matrix cores
+// (hist_device.hpp), the bytes after them one by one, and added to the
+// buffer's accumulators.
 template <uint32_t EB, int NW>
-__device__ __forceinline__ void wg_hist_chunk(const uint8_t* in, uint64_t c0, uint64_t c1, uint32_t* cnt) {
-  constexpr uint32_t P = EB, R = 32u / EB, T = 64u * NW;
-  const uint32_t t = threadIdx.x;
-  uint32_t* const c = cnt + t % R;
-  const uint4* p4 = (const uint4*)(in + c0);
-  const uint32_t n16 = (uint32_t)((c1 - c0) / 16u);  // (a chunk is at most 512 KiB)
-  auto count16 = [&](const uint4& v) {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int m = 0; m < 4; ++m)
-        atomicAdd(c + ((uint32_t)((4 * q + m) % (int)P) * 256u + __builtin_amdgcn_ubfe(w[q], 8u * (uint32_t)m, 8u)) * R,
-                  1u);
-  };
-  // rows of kHistLoads uint4 per thread, two buffers; loads are
-  // unconditional (indices past the end re-read uint4 0 and are not counted)
-  constexpr uint32_t ROW = T * kHistLoads;
-  auto load = [&](uint4 (&buf)[kHistLoads], uint32_t base) {
-#pragma unroll
-    for (int k = 0; k < kHistLoads; ++k) {
-      const uint32_t i = base + T * (uint32_t)k + t;
-      buf[k] = p4[i < n16 ? i : 0u];
-    }
-  };
-  auto count = [&](const uint4 (&buf)[kHistLoads], uint32_t base) {
-#pragma unroll
-    for (int k = 0; k < kHistLoads; ++k)
-      if (base + T * (uint32_t)k + t < n16) count16(buf[k]);
-  };
-  if (n16 > 0) {
-    uint4 bufA[kHistLoads], bufB[kHistLoads];
-    uint32_t r = 0;
-    load(bufA, 0);
-    for (;;) {
-      load(bufB, r + ROW);
-      count(bufA, r);
-      r += ROW;
-      if (r >= n16) break;
-      load(bufA, r + ROW);
-      count(bufB, r);
-      r += ROW;
-      if (r >= n16) break;
-    }
-  }
-  const uint64_t tail = c0 + 16ull * n16;  // (a multiple of P from c0: plane t % P)
-  if (tail + t < c1) atomicAdd(c + ((t % P) * 256u + in[tail + t]) * R, 1u);
-}
-
-// Adds the workgroup's counters to buffer b's accumulators and zeroes them:
-// thread t sums bin t (t + T, ...) of the P x 256, its replicas read from a
-// rotated start so the lanes of a pass spread over the banks.
-template <uint32_t EB, int NW>
-__device__ __forceinline__ void wg_hist_merge(uint32_t b, uint32_t* cnt, uint32_t* ghist) {
-  constexpr uint32_t P = EB, R = 32u / EB, T = 64u * NW;
-  for (uint32_t i = threadIdx.x; i < P * 256u; i += T) {
-    uint32_t* const row = cnt + i * R;
-    uint32_t sum = 0;
-#pragma unroll
-    for (uint32_t q = 0; q < R; ++q) {
-      const uint32_t qq = (q + i) % R;
-      sum += row[qq];
-      row[qq] = 0;
-    }
-    if (sum) atomicAdd(ghist + (uint64_t)b * 1024u + i, sum);
-  }
+__device__ __forceinline__ void wg_hist_chunk(const uint8_t* in, uint64_t c0, uint64_t c1, uint32_t* cnt,
+                                              uint32_t* ghist) {
+  const uint32_t t = threadIdx.x, n = (uint32_t)(c1 - c0);  // (a chunk is at most 512 KiB)
+  const uint32_t ntiles = n / (16u * kTileU4);
+  int32_t sum[EB][4] = {};
+  count_tiles<(int)EB>((const uint4*)(in + c0), wave_u32(t >> 6), ntiles, NW, sum);
+  for (uint32_t i = 16u * kTileU4 * ntiles + t; i < n; i += 64u * NW) count_byte(cnt, i % EB, in[c0 + i]);
+  __syncthreads();
+  flush_counts<(int)EB, 64 * NW>(sum, cnt, ghist);
 }
 
 // The histogram phase of a workgroup that starts on histograms: it takes
 // chunk items from their own counter (queue[3]) until none is left, one
 // workgroup barrier round per chunk (the next grab is taken while the
 // current chunk is counted); the workgroup that counts a buffer's last chunk
-// runs its finisher on wavefront 0.  LDS: the counters, the finisher's 256
+// runs its finisher on wavefront 0.  LDS: the counts, the finisher's 256
 // keys, the two grabbed items and the finish flag.
 template <int PB>
 __device__ void finish_buffer(const BatchBuf& B, uint32_t b, const BatchEncodeArgs& a, uint32_t gen, uint32_t* keys);
 
 template <int PB, int NW>
 __device__ void hist_phase(const BatchEncodeArgs& a, uint32_t gen, uint32_t* lds) {
-  static_assert(kHistCntWords + 256u + 4u <= NW * kWaveWords, "the histogram phase fits the workgroup's LDS");
+  static_assert(kFlushWords + 256u + 4u <= NW * kWaveWords, "the histogram phase fits the workgroup's LDS");
   uint32_t* const cnt = lds;
-  uint32_t* const keys = lds + kHistCntWords;
+  uint32_t* const keys = lds + kFlushWords;
   uint32_t* const s_it = keys + 256;  // [0..1] grabbed items, [2] finish flag
-  for (uint32_t i = threadIdx.x; i < kHistCntWords; i += 64u * NW) cnt[i] = 0;
+  for (uint32_t i = threadIdx.x; i < kFlushWords; i += 64u * NW) cnt[i] = 0;
   if (threadIdx.x == 0) s_it[0] = atomicAdd(a.queue + 3, 1u);
   __syncthreads();
   for (uint32_t k = 0;; ++k) {
@@ -217,15 +154,12 @@ __device__ void hist_phase(const BatchEncodeArgs& a, uint32_t gen, uint32_t* lds
     const uint64_t bytes = B.n * B.eb;
     const uint64_t c0 = (uint64_t)li * a.hist_chunk;
     const uint64_t c1 = c0 + a.hist_chunk < bytes ? c0 + a.hist_chunk : bytes;
+    uint32_t* const ghist = a.hist + (uint64_t)b * 1024u;
     if (c0 < c1) {
-      if (B.eb == 1) wg_hist_chunk<1, NW>(B.in, c0, c1, cnt);
-      else if (B.eb == 2) wg_hist_chunk<2, NW>(B.in, c0, c1, cnt);
-      else wg_hist_chunk<4, NW>(B.in, c0, c1, cnt);
+      if (B.eb == 1) wg_hist_chunk<1, NW>(B.in, c0, c1, cnt, ghist);
+      else if (B.eb == 2) wg_hist_chunk<2, NW>(B.in, c0, c1, cnt, ghist);
+      else wg_hist_chunk<4, NW>(B.in, c0, c1, cnt, ghist);
     }
-    __syncthreads();
-    if (B.eb == 1) wg_hist_merge<1, NW>(b, cnt, a.hist);
-    else if (B.eb == 2) wg_hist_merge<2, NW>(b, cnt, a.hist);
-    else wg_hist_merge<4, NW>(b, cnt, a.hist);
     publish();
     __syncthreads();
     if (threadIdx.x == 0) s_it[2] = atomicAdd(a.done + b, 1u) + 1u == B.nhist ? 1u : 0u;
@@ -974,7 +908,6 @@ hipError_t launch_enc(const BatchEncodeArgs& a, BatchShape sh, int cu, hipStream
   switch (sh.nw) {
     case 4: return launch_enc_nw<PB, 4>(a, sh.kb, cu, s, need_spill);
     case 8: return launch_enc_nw<PB, 8>(a, sh.kb, cu, s, need_spill);
-    case 16: return launch_enc_nw<PB, 16>(a, sh.kb, cu, s, need_spill);
   }
   return hipErrorInvalidValue;
 }

@@ -439,43 +439,50 @@ __device__ __forceinline__ uint32_t wave_sum32(uint32_t v) {
   return v;
 }
 
-// Normalises one plane with a single wavefront: lane l owns symbols
-// 4l .. 4l + 3 (count[j] is symbol 4l + j).  The same restatement of
-// GpuANSStatistics.h:186-385 as the 256-thread finisher of the histogram
-// launch (fp32 quantisation, rank by (q << 16 | s) descending, the +1 rule
-// for symbol ids below diff % 256, repeated decrements at ranks
-// [G - it, G)), with wave-wide sums and scans.  s_keys: 256 words of this
-// wave's LDS.  Returns {pdf, cdf, magic, shift} per owned symbol.
-__device__ inline void normalize_wave(const uint32_t (&count)[4], uint32_t total, int p, uint32_t* s_keys,
-                                      uint4 (&out)[4], bool& bad) {
+// Normalisation of one plane, by a wavefront whose lane l owns symbols 4l ..
+// 4l + 3 (element j is symbol 4l + j).  Restates GpuANSStatistics.h:186-385
+// exactly, in three parts:
+//  * quantize_syms: q = (u32)(float(2^p) * (float(count) / float(total))),
+//    IEEE round to nearest on both operations, truncating conversion; present
+//    symbols get at least 1.  Returns their sum;
+//  * rank_syms: rank = position of (q << 16 | s) in descending order, the
+//    number of the keys [k0, k1) (multiples of 4) above this lane's;
+//  * settle_syms: with the sum below 2^p, q[s] += diff / 256 + (s < diff %
+//    256) (the reference's repeated "+1 to symbol ids < min(diff, 256)"
+//    loop); above, repeatedly G = #{q > 1}, it = min(diff, G), one subtracted
+//    at the ranks [G - it, G) of the original order.  Then cdf = exclusive
+//    scan in symbol order, shift = 32 - clz(pdf - 1), magic = 2^32 (2^shift -
+//    pdf) / pdf + 1 (0 for pdf == 0), giving {pdf, cdf, magic, shift}.
+__device__ __forceinline__ uint32_t quantize_syms(const uint32_t (&count)[4], uint32_t total, int p, uint32_t (&q)[4],
+                                                  uint32_t (&key)[4]) {
   const uint32_t lane = threadIdx.x & 63u;
-  if (total == 0) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) out[j] = make_uint4(0, 0, 0, 0);
-    return;
-  }
-  const uint32_t W = 1u << p;
-  uint32_t q[4], key[4], qs = 0;
+  uint32_t qs = 0;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const float ratio = __fdiv_rn((float)count[j], (float)total);
-    const float prod = __fmul_rn((float)W, ratio);
+    const float prod = __fmul_rn((float)(1u << p), ratio);
     q[j] = (uint32_t)prod;
     if (count[j] > 0 && q[j] == 0) q[j] = 1;
     qs += q[j];
     key[j] = (q[j] << 16) | (4u * lane + (uint32_t)j);
-    s_keys[4u * lane + (uint32_t)j] = key[j];
   }
-  const uint32_t qsum = wave_sum32(qs);
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  int rank[4] = {0, 0, 0, 0};
-  for (int i = 0; i < (int)kNumSymbols; ++i) {
-    const uint32_t k = s_keys[i];
+  return wave_sum32(qs);
+}
+__device__ __forceinline__ void rank_syms(const uint32_t (&key)[4], const uint32_t* s_keys, uint32_t k0, uint32_t k1,
+                                          uint32_t (&rank)[4]) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) rank[j] += k > key[j];
+  for (int j = 0; j < 4; ++j) rank[j] = 0;
+#pragma unroll 4
+  for (uint32_t i = k0; i < k1; i += 4) {
+    const uint4 k = *(const uint4*)(s_keys + i);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) rank[j] += (k.x > key[j]) + (k.y > key[j]) + (k.z > key[j]) + (k.w > key[j]);
   }
-  const int diff = (int)W - (int)qsum;
+}
+__device__ __forceinline__ void settle_syms(uint32_t (&q)[4], uint32_t qsum, const uint32_t (&rank)[4], int p,
+                                            uint4 (&out)[4], bool& bad) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const int diff = (1 << p) - (int)qsum;
   if (diff > 0) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) q[j] += (uint32_t)(diff >> 8) + ((4u * lane + (uint32_t)j < (uint32_t)(diff & 255)) ? 1u : 0u);
@@ -493,7 +500,7 @@ __device__ inline void normalize_wave(const uint32_t (&count)[4], uint32_t total
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (rank[j] >= g - it && rank[j] < g) q[j] -= 1;
+        if ((int)rank[j] >= g - it && (int)rank[j] < g) q[j] -= 1;
       d -= it;
     }
   }
@@ -518,6 +525,28 @@ __device__ inline void normalize_wave(const uint32_t (&count)[4], uint32_t total
     out[j] = make_uint4(pdf, cdf, magic, shift);
     cdf += pdf;
   }
+}
+
+// Normalises one plane with a single wavefront.  s_keys: 256 words of this
+// wave's LDS (16-byte aligned).
+__device__ inline void normalize_wave(const uint32_t (&count)[4], uint32_t total, int p, uint32_t* s_keys,
+                                      uint4 (&out)[4], bool& bad) {
+  const uint32_t lane = threadIdx.x & 63u;
+  if (total == 0) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) out[j] = make_uint4(0, 0, 0, 0);
+    return;
+  }
+  uint32_t q[4], key[4], rank[4] = {0, 0, 0, 0};
+  const uint32_t qsum = quantize_syms(count, total, p, q, key);
+  if (qsum > (1u << p)) {  // (the ranks are needed only to take some away)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s_keys[4u * lane + (uint32_t)j] = key[j];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    rank_syms(key, s_keys, 0, kNumSymbols, rank);
+  }
+  settle_syms(q, qsum, rank, p, out, bad);
 }
 
 }  // namespace mans

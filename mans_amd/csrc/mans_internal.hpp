@@ -131,7 +131,9 @@ struct HistArgs {
   uint64_t plane_section[kMaxPlanes];
   uint32_t* hist;                // [P][256] self-cleaning accumulators
   uint32_t* done;                // self-cleaning WG counter
-  uint32_t* grab;                // [2] self-cleaning row-chunk counters, one per source
+  uint32_t* grab;                // [2] self-cleaning chunk counters, one per source
+  uint32_t chunk_tiles;          // tiles per chunk (set at launch)
+  uint32_t pad0_;
   uint4* table;                  // [P][256] {pdf, cdf, magic, shift}
   uint32_t* hist_out;            // optional copy of the final histogram
   uint8_t* out;                  // container base (headers), may be null
@@ -351,7 +353,7 @@ constexpr BatchShape kBatchEncodeDefault = {4, 16};
 constexpr BatchShape kBatchDecodeDefault = {4, 8};
 // LDS bytes per workgroup of a shape (encode: tables | stages per
 // wave; decode: two LUTs | two rings per wave)
-constexpr uint64_t batch_encode_lds(BatchShape sh) { return (uint64_t)sh.nw * (2u * 256u * 2u + 1024u + 128u) * 4u; }
+constexpr uint64_t batch_encode_lds(BatchShape sh) { return (uint64_t)sh.nw * (2u * 256u * 2u + 1024u) * 4u; }
 constexpr uint64_t batch_decode_lds(BatchShape sh, int pb) {
   return (uint64_t)sh.nw * (2ull * (1u << pb) * 4u +
                             2ull * 2u * ((2u * (64u * sh.kb > 512u ? 64u * sh.kb : 512u)) + 64u));
