@@ -45,16 +45,10 @@ constexpr uint64_t kValue48 = (1ull << kGenShift) - 1;
 constexpr uint32_t kTabWords = 2 * 256 * 2;
 constexpr uint32_t kStageWords = 4 * 512 / 2;
 constexpr uint32_t kWaveWords = kTabWords + kStageWords;
-// Queue items a decode wavefront takes at once (BatchDecodeArgs::run, 1 or
-// 4): consecutive tickets of a buffer then run on one wavefront, which keeps
-// the buffer's LUTs in its LDS.  (Encode takes one at a time: a ticket's
-// look-back waits for its predecessor's count, and with runs that
-// predecessor would be the last of another wavefront's run, so the runs of a
-// buffer would follow one another.)  An item waits only on lower items, each
-// held by a running wavefront that reaches it, so the launch drains.
-
 template <typename T>
 using gptr = const __attribute__((address_space(1))) T*;
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ uint32_t wave_u32(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 
@@ -929,43 +923,50 @@ struct DecRing {
   static_assert(64u * KB <= H, "KB steps must fit in a half");
 };
 
-// LUT item: check buffer b's frame against its plan and build the packed LUT
-// (slot - cdf) << 20 | pdf << 8 | sym of every plane into global memory.
+// Decoder LUT entries (dec_steps): 4 bytes.  With the workgroup's two LUTs in
+// 8 KiB, 24 wavefronts fit a CU; with 8-byte entries, which the single-buffer
+// decoder takes (its LUTs serve eight wavefronts), 16, and 1024 buffers of 590
+// MB take 0.45 ms against 0.38.
+__device__ __forceinline__ uint32_t lut_entry(uint32_t sym, uint32_t pdf, uint32_t off) {
+  return (off << 20) | (pdf << 8) | sym;
+}
+
+// Buffer b's frame against its plan: magic, version, element width, mode 0,
+// lanes, precision, planes, order, block bytes, n, data offset and section
+// offsets, and each plane's section header.
 template <int PB>
-__device__ void build_luts(const BatchBuf& B, uint32_t b, const BatchDecodeArgs& a, uint32_t gen, uint32_t* wl) {
-  constexpr uint32_t W = 1u << PB;
-  const uint32_t lane = threadIdx.x & 63u;
+__device__ bool frame_bad(const BatchBuf& B) {
   const uint32_t P = B.eb;
-  bool bad = B.in_bytes < B.data_off;
-  if (!bad) {
-    const uint32_t* fh = (const uint32_t*)B.in;
-    const uint8_t* fb = B.in;
-    // magic, version, element width, mode 0, lanes, precision, planes, order,
-    // block bytes, n, data offset and section offsets must match the plan
-    bad = fh[0] != kFrameMagic || fb[4] != kFrameVersion || fb[5] != 0 || fb[6] != P || fb[7] != 0 ||
-          fb[8] != B.lanes || fb[9] != PB || fb[10] != P || fb[11] != 0 || fh[3] != 128u * B.lanes ||
-          ((const uint64_t*)B.in)[2] != B.n || ((const uint64_t*)B.in)[5] != B.data_off;
-    for (uint32_t k = 0; k < P && !bad; ++k) bad = ((const uint64_t*)B.in)[8 + k] != B.section[k];
-    const uint64_t data_words = ((const uint64_t*)B.in)[6];
-    bad = bad || B.data_off + 2ull * data_words > B.in_bytes;
+  if (B.in_bytes < B.data_off) return true;
+  // (bitwise: the reads are independent and go out together)
+  const gptr<uint32_t> fh = (gptr<uint32_t>)B.in;
+  const gptr<uint64_t> fq = (gptr<uint64_t>)B.in;
+  bool bad = (fh[0] != kFrameMagic) | (fh[1] != (kFrameVersion | (P << 16))) |
+             (fh[2] != (B.lanes | ((uint32_t)PB << 8) | (P << 16))) | (fh[3] != 128u * B.lanes) | (fq[2] != B.n) |
+             (fq[5] != B.data_off);
+  bad |= B.data_off + 2ull * fq[6] > B.in_bytes;
+  for (uint32_t k = 0; k < P; ++k) {
+    const gptr<uint32_t> h = (gptr<uint32_t>)(B.in + B.section[k]);
+    bad |= (fq[8 + k] != B.section[k]) | (h[0] != ((kAnsMagic << 16) | (B.lanes == 32 ? 1u : 2u))) |
+           ((h[4] & 0xfu) != (uint32_t)PB) | (h[1] != B.nb) | (h[2] != (uint32_t)B.n);
   }
-  uint32_t* cdf = wl;  // 257 words
-  for (uint32_t k = 0; k < P && !bad; ++k) {
-    const uint8_t* sec = B.in + B.section[k];
-    const uint32_t* h = (const uint32_t*)sec;
-    if ((h[0] >> 16) != kAnsMagic || (h[0] & 0xffffu) != (B.lanes == 32 ? 1u : 2u) || (h[4] & 0xfu) != (uint32_t)PB ||
-        h[1] != B.nb ||
-        h[2] != (uint32_t)B.n) {
-      bad = true;
-      break;
-    }
-    const uint16_t* probs = (const uint16_t*)(sec + kAnsHeaderBytes);
-    uint32_t v[4], ls = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      v[j] = probs[4 * lane + j];
-      ls += v[j];
-    }
+  return bad;
+}
+
+// The LUTs of planes p0 .. p0 + np - 1 of buffer B into lut[2^p each], by the
+// whole workgroup: wavefront k scans plane p0 + k's frequencies into cdf[k],
+// then every thread searches its slots, all of them at once (one after
+// another a slot's eight dependent reads took most of the build).  Returns
+// true if a table does not sum to 2^p.
+template <int PB, int NW>
+__device__ __forceinline__ bool build_luts(const BatchBuf& B, uint32_t p0, uint32_t np, uint32_t* lut,
+                                           uint32_t (*cdf)[kNumSymbols + 1]) {
+  constexpr uint32_t W = 1u << PB, T = 64u * NW;
+  const uint32_t t = threadIdx.x, lane = t & 63u, wave = wave_u32(t >> 6);
+  if (wave < np) {
+    const u32x2 q = ((gptr<u32x2>)(B.in + B.section[p0 + wave] + kAnsHeaderBytes))[lane];
+    const uint32_t v[4] = {q.x & 0xffffu, q.x >> 16, q.y & 0xffffu, q.y >> 16};
+    const uint32_t ls = v[0] + v[1] + v[2] + v[3];
     uint32_t inc = ls;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -975,49 +976,48 @@ __device__ void build_luts(const BatchBuf& B, uint32_t b, const BatchDecodeArgs&
     uint32_t run = inc - ls;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      cdf[4 * lane + j] = run;
+      cdf[wave][4 * lane + j] = run;
       run += v[j];
     }
-    if (lane == 63) cdf[256] = run;
-    drain();
-    if (B.n > 0 && cdf[256] != W) {
+    if (lane == 63) cdf[wave][kNumSymbols] = run;
+  }
+  __syncthreads();
+  bool bad = false;
+  for (uint32_t k = 0; k < np; ++k) {
+    if (B.n > 0 && cdf[k][kNumSymbols] != W) {
       bad = true;
-      break;
+      continue;
     }
-    uint32_t* g = a.luts + ((uint64_t)b * 4u + k) * W;
-    for (uint32_t slot = 2 * lane; slot < W; slot += 128) {
-      uint32_t ent[2];
+    constexpr uint32_t PER = W > T ? W / T : 1u;
+    uint32_t lo[PER];
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const uint32_t sl = slot + q;
-        uint32_t lo = 0, hi = kNumSymbols;
-        while (hi - lo > 1) {
-          const uint32_t mid = (lo + hi) >> 1;
-          if (cdf[mid] <= sl) lo = mid; else hi = mid;
-        }
-        const uint32_t c = cdf[lo], pdf = cdf[lo + 1] - c;
-        ent[q] = ((sl - c) << 20) | (pdf << 8) | lo;
+    for (uint32_t j = 0; j < PER; ++j) lo[j] = 0;
+    // largest symbol s with cdf[s] <= slot (that symbol has pdf > 0)
+#pragma unroll
+    for (uint32_t step = kNumSymbols / 2; step > 0; step >>= 1)
+#pragma unroll
+      for (uint32_t j = 0; j < PER; ++j) lo[j] = cdf[k][lo[j] + step] <= t + T * j ? lo[j] + step : lo[j];
+#pragma unroll
+    for (uint32_t j = 0; j < PER; ++j) {
+      const uint32_t slot = t + T * j;
+      if (slot < W) {
+        const uint32_t c = cdf[k][lo[j]];
+        lut[k * W + slot] = lut_entry(lo[j], cdf[k][lo[j] + 1] - c, slot - c);
       }
-      atomic_st64((uint64_t*)(g + slot), ((uint64_t)ent[1] << 32) | ent[0]);
     }
-    drain();
   }
-  bad = __ballot(bad) != 0;
-  if (bad && lane == 0) {
-    atomicOr(a.err, kErrMagic);
-    atomicOr(a.bad + b, kErrMagic);
-  }
-  publish();
-  if (lane == 0) atomic_st32(a.ready + b, gen | (bad ? kBatchBad : 0u));
+  return bad;
 }
 
-// Decode ticket: units u0, u0 + 1 of buffer B with the 64-lane ring decoder.
-// SAME: two planes of the same elements (stored together as 16 bits at byte
-// kp[0] of each element); otherwise two blocks of a uint8 buffer.
-// tkey: which LUTs the wave's LDS holds, as for encode_ticket.
-template <int PB, bool SAME, int KB>
-__device__ void decode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, const BatchDecodeArgs& a, uint32_t* wl,
-                              uint64_t& tkey) {
+// Decode ticket lt of buffer B with the 64-lane ring decoder: two blocks (2
+// lt, 2 lt + 1) of a uint8 buffer, or planes p0, p0 + 1 of block lt, stored
+// together as 16 bits at byte p0 of each element.  lut: the planes' LUTs
+// (uint8: one for both blocks); wstage: this wavefront's two rings.
+template <int PB, int EB, int KB>
+__device__ __forceinline__ void decode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, uint32_t p0,
+                                              const BatchDecodeArgs& a, const uint32_t* s_lut, uint16_t* wstage) {
+  constexpr bool SAME = EB != 1;
+  constexpr uint32_t P = EB;
   constexpr uint32_t W = 1u << PB;
   constexpr uint32_t kH = DecRing<KB>::H, kR = DecRing<KB>::R, kMask = DecRing<KB>::MASK;
   constexpr uint32_t kDecRing = DecRing<KB>::WORDS;
@@ -1025,32 +1025,40 @@ __device__ void decode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, const 
   constexpr int QH = (int)(H4 / 64);  // uint4 per lane per half
   constexpr uint32_t UNIT_CAP = kL * lane_max_words(kBlock / kL, PB);
   const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t P = B.eb;
-  const uint64_t U = (uint64_t)P * B.nb;
-  const uint64_t u0 = 2ull * lt;
-  const uint64_t data_words = ((const uint64_t*)B.in)[6];
-  uint32_t* s_lut = wl;                                   // [2][W]
-  uint16_t* wstage = (uint16_t*)(wl + 2 * W);             // [2][R + 64]
-  uint32_t x[2], ptr[2], n[2], wds[2], taken[2], lo[2], kp[2];
+  const uint64_t data_words = ((gptr<uint64_t>)B.in)[6];
+  uint32_t x[2], ptr[2], n[2], taken[2], lo[2], kp[2];
   bool act[2], pend[2];
   uint64_t blk[2];
-  uint4 rv[2][QH];
-  const uint4* src4[2];
+  u32x2 bw[2];
+  u32x4 rv[2][QH];
+  gptr<u32x4> src4[2];
   const uint32_t* lut[2];
   const uint16_t* stage[2];
+  // the units' block words and states, then their top two ring halves: each
+  // group's loads go out together (a wavefront waits for memory twice)
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
-    const uint64_t u = u0 + c;
-    act[c] = u < U;
-    kp[c] = act[c] ? (uint32_t)(u % P) : 0u;
-    blk[c] = act[c] ? u / P : 0u;
-    const uint8_t* sec = B.in + B.section[kp[c]];
-    uint32_t nn = 0, words = 0, y = 0;
+    const uint64_t bc = SAME ? lt : 2ull * lt + c;
+    act[c] = bc < B.nb;
+    kp[c] = SAME ? p0 + (uint32_t)c : 0u;
+    blk[c] = act[c] ? bc : 0u;
+    const gptr<uint8_t> sec = (gptr<uint8_t>)B.in + B.section[kp[c]];
+    bw[c] = u32x2{0, 0};
+    x[c] = kMinState;
     if (act[c]) {
-      const uint2 bw = *(const uint2*)(sec + kSectionFixed + 4ull * kL * B.nb + 8ull * blk[c]);
-      nn = bw.x >> 16;
-      words = bw.x & 0xffffu;
-      y = bw.y;
+      bw[c] = *(gptr<u32x2>)(sec + kSectionFixed + 4ull * kL * B.nb + 8ull * blk[c]);
+      x[c] = ((gptr<uint32_t>)(sec + kSectionFixed))[blk[c] * kL + lane];
+    }
+  }
+  u32x4 first[2][2 * QH];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    n[c] = 0;
+    uint32_t words = 0, y = 0;
+    if (act[c]) {
+      const uint32_t b0 = wave_u32(bw[c].x), nn = b0 >> 16;
+      words = b0 & 0xffffu;
+      y = wave_u32(bw[c].y);
       const uint64_t start = blk[c] * kBlock;
       const uint64_t expect = (B.n - start) < kBlock ? (B.n - start) : kBlock;
       if (nn != expect || words > UNIT_CAP || (uint64_t)y + round_up(words, 8) > data_words ||
@@ -1060,50 +1068,37 @@ __device__ void decode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, const 
           atomicOr(a.bad + b, kErrBlockWords);
         }
         act[c] = false;
-        nn = 0;
+        x[c] = kMinState;
         words = 0;
+      } else {
+        n[c] = nn;
       }
     }
-    n[c] = nn;
-    words = wave_u32(words);
-    y = wave_u32(y);
-    lut[c] = s_lut + c * W;
-    src4[c] = (const uint4*)(B.in + B.data_off + 2ull * y);
-    uint16_t* reg = wstage + c * kDecRing;
-    stage[c] = reg;
-    lo[c] = 0;
+    lut[c] = s_lut + (SAME ? c : 0) * W;
+    src4[c] = (gptr<u32x4>)(B.in + B.data_off + 2ull * y);
+    stage[c] = wstage + c * kDecRing;
+    lo[c] = words > kH ? (words - 1) / kH * kH - kH : 0u;
     pend[c] = false;
-#pragma unroll
-    for (int q = 0; q < QH; ++q) rv[c][q] = make_uint4(0, 0, 0, 0);
-    if (words > 0) {
-      const uint32_t jt = (words - 1) / kH;
-      const uint32_t j0 = jt > 0 ? jt - 1 : 0;
-      lo[c] = j0 * kH;
-      for (uint32_t j = j0; j <= jt; ++j) {
-        const uint32_t left = words - j * kH;
-        const uint32_t n4 = (uint32_t)div_up(left < kH ? left : kH, 8);
-        for (uint32_t i = lane; i < n4; i += 64) {
-          const uint4 q = src4[c][j * H4 + i];
-          ((uint4*)(reg + (j & 1) * kH))[i] = q;
-          if ((j & 1) == 0 && i < 8) ((uint4*)(reg + kR))[i] = q;
-        }
-      }
-    }
-    x[c] = act[c] ? ((const uint32_t*)(sec + kSectionFixed))[blk[c] * kL + lane] : kMinState;
     ptr[c] = words;
-    wds[c] = words;
     taken[c] = 0;
-  }
-  // the chains' LUTs, built by the buffer's LUT item
-  const uint64_t key = ((uint64_t)b << 4) | (kp[0] << 2) | kp[1];
-  if (key != tkey) {
+    const uint32_t n4 = (uint32_t)div_up(words, 8);
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const uint64_t* g = (const uint64_t*)(a.luts + ((uint64_t)b * 4u + kp[c]) * W);
-      uint64_t* d = (uint64_t*)(s_lut + c * W);
-      for (uint32_t j = lane; j < W / 2; j += 64) d[j] = atomic_ld64(g + j);
+    for (int i = 0; i < 2 * QH; ++i) {
+      rv[c][i % QH] = first[c][i] = u32x4{0, 0, 0, 0};
+      const uint32_t at = lo[c] / 8 + 64 * i + lane;
+      if (at < n4) first[c][i] = src4[c][at];
     }
-    tkey = key;
+  }
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    uint16_t* reg = wstage + c * kDecRing;
+    const uint32_t j0 = lo[c] / kH;
+#pragma unroll
+    for (int i = 0; i < 2 * QH; ++i) {
+      const uint32_t h = (j0 + (uint32_t)(i / QH)) & 1u;
+      ((u32x4*)(reg + h * kH))[64 * (i % QH) + lane] = first[c][i];
+      if (h == 0 && i % QH == 0 && lane < 8) ((u32x4*)(reg + kR))[lane] = first[c][i];
+    }
   }
 #pragma unroll
   for (int c = 0; c < 2; ++c) __asm__ volatile("" : "+v"(x[c]));
@@ -1119,8 +1114,8 @@ __device__ void decode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, const 
     const uint32_t j = lo[c] / kH - 1;
     uint16_t* reg = wstage + c * kDecRing;
 #pragma unroll
-    for (int q = 0; q < QH; ++q) ((uint4*)(reg + (j & 1) * kH))[64 * q + lane] = rv[c][q];
-    if ((j & 1) == 0 && lane < 8) ((uint4*)(reg + kR))[lane] = rv[c][0];
+    for (int q = 0; q < QH; ++q) ((u32x4*)(reg + (j & 1) * kH))[64 * q + lane] = rv[c][q];
+    if ((j & 1) == 0 && lane < 8) ((u32x4*)(reg + kR))[lane] = rv[c][0];
     lo[c] -= kH;
     pend[c] = false;
   };
@@ -1128,11 +1123,11 @@ __device__ void decode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, const 
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       if constexpr (KB == 1) {
-        if (!pend[c] && lo[c] > 0 && ptr[c] <= lo[c] + kH) fetch(c);
-        if (pend[c] && ptr[c] < lo[c] + 64u) commit(c);
+        if (!pend[c] && lo[c] > 0 && (int32_t)ptr[c] <= (int32_t)(lo[c] + kH)) fetch(c);
+        if (pend[c] && (int32_t)ptr[c] < (int32_t)(lo[c] + 64u)) commit(c);
       } else {
         if (!pend[c] && lo[c] > 0) fetch(c);
-        if (pend[c] && ptr[c] <= lo[c] + kH) {
+        if (pend[c] && (int32_t)ptr[c] <= (int32_t)(lo[c] + kH)) {
           commit(c);
           if (lo[c] > 0) fetch(c);
         }
@@ -1162,13 +1157,13 @@ __device__ void decode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, const 
       --s;
       const uint32_t i = s * kL + lane;
       bool v[2] = {i < n[0], i < n[1]};
-      const uint32_t el = dec_steps<kL, PB, 2, kMask, uint32_t>(x, ptr, taken, lut, stage, v, 0u);
+      const uint32_t el = dec_steps<kL, PB, 2, kMask, uint32_t, false>(x, ptr, taken, lut, stage, v, 0u);
       store(s, el, v[0], v[1]);
       refill();
     }
     for (uint32_t s = full; s > 0;) {
       --s;
-      const uint32_t el = dec_steps<kL, PB, 2, kMask, uint32_t>(x, ptr, taken, lut, stage, vall, 0u);
+      const uint32_t el = dec_steps<kL, PB, 2, kMask, uint32_t, false>(x, ptr, taken, lut, stage, vall, 0u);
       store(s, el, true, true);
       refill();
     }
@@ -1181,23 +1176,33 @@ __device__ void decode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, const 
       --s;
       const uint32_t i = s * kL + lane;
       bool v[2] = {i < n[0], i < n[1]};
-      const uint32_t el = dec_steps<kL, PB, 2, kMask, uint32_t>(x, ptr, taken, lut, stage, v, 0u);
+      const uint32_t el = dec_steps<kL, PB, 2, kMask, uint32_t, false>(x, ptr, taken, lut, stage, v, 0u);
       store(s, el, v[0], v[1]);
       if (s % KB == 0) refill();
     }
     while (s > 0) {
+      // one address per block for the KB steps, whose stores take immediate
+      // offsets from it
+      s -= KB;
+      uint8_t* const g0 = o0 + ((uint64_t)s * kL + lane) * P;
+      uint8_t* const g1 = o1 + ((uint64_t)s * kL + lane) * P;
 #pragma unroll
-      for (int j = 0; j < KB; ++j) {
-        --s;
-        const uint32_t el = dec_steps<kL, PB, 2, kMask, uint32_t>(x, ptr, taken, lut, stage, vall, 0u);
-        store(s, el, true, true);
+      for (int j = KB - 1; j >= 0; --j) {
+        const uint32_t el = dec_steps<kL, PB, 2, kMask, uint32_t, false>(x, ptr, taken, lut, stage, vall, 0u);
+        if constexpr (SAME) {
+          ((__attribute__((address_space(1))) uint16_t*)g0)[j * (int)kL * EB / 2] = (uint16_t)el;
+        } else {
+          ((__attribute__((address_space(1))) uint8_t*)g0)[j * (int)kL] = (uint8_t)el;
+          ((__attribute__((address_space(1))) uint8_t*)g1)[j * (int)kL] = (uint8_t)(el >> 8);
+        }
       }
       refill();
     }
   }
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
-    const bool bad = act[c] && (taken[c] != wds[c] || x[c] != kMinState);
+    // (ptr goes below 0 on a corrupt stream, every read masked into the ring)
+    const bool bad = act[c] && (ptr[c] != 0u || x[c] != kMinState);
     if (__ballot(bad) && lane == 0) {
       atomicOr(a.err, kErrFinalState);
       atomicOr(a.bad + b, kErrFinalState);
@@ -1205,14 +1210,15 @@ __device__ void decode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, const 
   }
 }
 
-// Decode ticket of the 32-lane format: units u0 = 2 lt and u0 + 1 of buffer
-// B, lanes 0-31 decoding the first and lanes 32-63 the second (one chain per
-// lane, each unit with its own ring and LUT slot; a unit consumes at most 32
-// words per step, inside the ring schedule's 64).  Each half stores its
-// plane's bytes.
-template <int PB, int KB>
-__device__ void decode_ticket32(const BatchBuf& B, uint32_t b, uint32_t lt, const BatchDecodeArgs& a, uint32_t* wl,
-                                uint64_t& tkey) {
+// Decode ticket of the 32-lane format, two units as in decode_ticket: lanes
+// 0-31 decode the first and lanes 32-63 the second (one chain per lane, each
+// unit with its own ring; a unit consumes at most 32 words per step, inside
+// the ring schedule's 64).  Each half stores its plane's bytes.
+template <int PB, int EB, int KB>
+__device__ __forceinline__ void decode_ticket32(const BatchBuf& B, uint32_t b, uint32_t lt, uint32_t p0,
+                                                const BatchDecodeArgs& a, const uint32_t* s_lut, uint16_t* wstage) {
+  constexpr bool SAME = EB != 1;
+  constexpr uint32_t P = EB;
   constexpr uint32_t L = 32, BLOCK = 4096;
   constexpr uint32_t W = 1u << PB;
   constexpr uint32_t kH = DecRing<KB>::H, kR = DecRing<KB>::R, kMask = DecRing<KB>::MASK;
@@ -1221,32 +1227,37 @@ __device__ void decode_ticket32(const BatchBuf& B, uint32_t b, uint32_t lt, cons
   constexpr int QH = (int)(H4 / 64);  // uint4 per lane per half ring
   constexpr uint32_t UNIT_CAP = L * lane_max_words(BLOCK / L, PB);
   const uint32_t lane = threadIdx.x & 63u, half = lane >> 5, lin = lane & 31u;
-  const uint32_t P = B.eb;
-  const uint64_t U = (uint64_t)P * B.nb;
-  const uint64_t u0 = 2ull * lt;
-  const uint64_t data_words = ((const uint64_t*)B.in)[6];
-  uint32_t* s_lut = wl;                        // [2][W]
-  uint16_t* wstage = (uint16_t*)(wl + 2 * W);  // [2][R + 64]
+  const uint64_t data_words = ((gptr<uint64_t>)B.in)[6];
   // per unit (stream h, wave-uniform): validity, plane, block, symbols,
   // words, where its words are, ring state
   bool acth[2], pend[2];
   uint32_t kph[2], nh[2], wordsh[2], lo[2];
   uint64_t blkh[2];
-  const uint4* ssrc4[2];
-  uint4 rv[2][QH];
+  u32x2 bw[2];
+  gptr<u32x4> ssrc4[2];
+  u32x4 rv[2][QH], first[2][2 * QH];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    const uint64_t u = u0 + h;
-    acth[h] = u < U;
-    kph[h] = acth[h] ? (uint32_t)(u % P) : 0u;
-    blkh[h] = acth[h] ? u / P : 0u;
-    const uint8_t* sec = B.in + B.section[kph[h]];
+    const uint64_t bh = SAME ? lt : 2ull * lt + h;
+    acth[h] = bh < B.nb;
+    kph[h] = SAME ? p0 + (uint32_t)h : 0u;
+    blkh[h] = acth[h] ? bh : 0u;
+    bw[h] = u32x2{0, 0};
+    if (acth[h]) bw[h] = *(gptr<u32x2>)(B.in + B.section[kph[h]] + kSectionFixed + 4ull * L * B.nb + 8ull * blkh[h]);
+  }
+  uint32_t x[1], ptr[1], taken[1];
+  const uint32_t kp = half ? kph[1] : kph[0];
+  const uint64_t blk = half ? blkh[1] : blkh[0];
+  x[0] = kMinState;
+  if (half ? acth[1] : acth[0]) x[0] = ((gptr<uint32_t>)(B.in + B.section[kp] + kSectionFixed))[blk * L + lin];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
     uint32_t nn = 0, words = 0, y = 0;
     if (acth[h]) {
-      const uint2 bw = *(const uint2*)(sec + kSectionFixed + 4ull * L * B.nb + 8ull * blkh[h]);
-      nn = bw.x >> 16;
-      words = bw.x & 0xffffu;
-      y = bw.y;
+      const uint32_t b0 = wave_u32(bw[h].x);
+      nn = b0 >> 16;
+      words = b0 & 0xffffu;
+      y = wave_u32(bw[h].y);
       const uint64_t start = blkh[h] * BLOCK;
       const uint64_t expect = (B.n - start) < BLOCK ? (B.n - start) : BLOCK;
       if (nn != expect || words > UNIT_CAP || (uint64_t)y + round_up(words, 8) > data_words ||
@@ -1260,52 +1271,38 @@ __device__ void decode_ticket32(const BatchBuf& B, uint32_t b, uint32_t lt, cons
         words = 0;
       }
     }
-    nh[h] = wave_u32(nn);
-    wordsh[h] = wave_u32(words);
-    y = wave_u32(y);
-    ssrc4[h] = (const uint4*)(B.in + B.data_off + 2ull * y);
-    uint16_t* reg = wstage + h * kDecRing;
-    lo[h] = 0;
+    nh[h] = nn;
+    wordsh[h] = words;
+    ssrc4[h] = (gptr<u32x4>)(B.in + B.data_off + 2ull * y);
+    lo[h] = wordsh[h] > kH ? (wordsh[h] - 1) / kH * kH - kH : 0u;
     pend[h] = false;
+    const uint32_t n4 = (uint32_t)div_up(wordsh[h], 8);
 #pragma unroll
-    for (int q = 0; q < QH; ++q) rv[h][q] = make_uint4(0, 0, 0, 0);
-    if (wordsh[h] > 0) {
-      const uint32_t jt = (wordsh[h] - 1) / kH;
-      const uint32_t j0 = jt > 0 ? jt - 1 : 0;
-      lo[h] = j0 * kH;
-      for (uint32_t j = j0; j <= jt; ++j) {
-        const uint32_t left = wordsh[h] - j * kH;
-        const uint32_t n4 = (uint32_t)div_up(left < kH ? left : kH, 8);
-        for (uint32_t i = lane; i < n4; i += 64) {
-          const uint4 q = ssrc4[h][j * H4 + i];
-          ((uint4*)(reg + (j & 1) * kH))[i] = q;
-          if ((j & 1) == 0 && i < 8) ((uint4*)(reg + kR))[i] = q;
-        }
-      }
+    for (int i = 0; i < 2 * QH; ++i) {
+      rv[h][i % QH] = first[h][i] = u32x4{0, 0, 0, 0};
+      const uint32_t at = lo[h] / 8 + 64 * i + lane;
+      if (at < n4) first[h][i] = ssrc4[h][at];
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    uint16_t* reg = wstage + h * kDecRing;
+    const uint32_t j0 = lo[h] / kH;
+#pragma unroll
+    for (int i = 0; i < 2 * QH; ++i) {
+      const uint32_t hf = (j0 + (uint32_t)(i / QH)) & 1u;
+      ((u32x4*)(reg + hf * kH))[64 * (i % QH) + lane] = first[h][i];
+      if (hf == 0 && i % QH == 0 && lane < 8) ((u32x4*)(reg + kR))[lane] = first[h][i];
     }
   }
   // this lane's unit
   const bool act = half ? acth[1] : acth[0];
-  const uint32_t kp = half ? kph[1] : kph[0];
-  const uint64_t blk = half ? blkh[1] : blkh[0];
   const uint32_t n = half ? nh[1] : nh[0];
-  uint32_t x[1], ptr[1], taken[1];
-  x[0] = act ? ((const uint32_t*)(B.in + B.section[kp] + kSectionFixed))[blk * L + lin] : kMinState;
+  if (!act) x[0] = kMinState;
   ptr[0] = half ? wordsh[1] : wordsh[0];
   taken[0] = 0;
-  const uint32_t* lut[1] = {s_lut + half * W};
+  const uint32_t* lut[1] = {s_lut + (SAME ? half * W : 0u)};
   const uint16_t* stage[1] = {wstage + half * kDecRing};
-  // the units' LUTs, built by the buffer's LUT item
-  const uint64_t key = ((uint64_t)b << 4) | (kph[0] << 2) | kph[1];
-  if (key != tkey) {
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const uint64_t* g = (const uint64_t*)(a.luts + ((uint64_t)b * 4u + kph[c]) * W);
-      uint64_t* d = (uint64_t*)(s_lut + c * W);
-      for (uint32_t j = lane; j < W / 2; j += 64) d[j] = atomic_ld64(g + j);
-    }
-    tkey = key;
-  }
   __asm__ volatile("" : "+v"(x[0]));
   drain();
 
@@ -1319,21 +1316,21 @@ __device__ void decode_ticket32(const BatchBuf& B, uint32_t b, uint32_t lt, cons
     const uint32_t j = lo[h] / kH - 1;
     uint16_t* reg = wstage + h * kDecRing;
 #pragma unroll
-    for (int q = 0; q < QH; ++q) ((uint4*)(reg + (j & 1) * kH))[64 * q + lane] = rv[h][q];
-    if ((j & 1) == 0 && lane < 8) ((uint4*)(reg + kR))[lane] = rv[h][0];
+    for (int q = 0; q < QH; ++q) ((u32x4*)(reg + (j & 1) * kH))[64 * q + lane] = rv[h][q];
+    if ((j & 1) == 0 && lane < 8) ((u32x4*)(reg + kR))[lane] = rv[h][0];
     lo[h] -= kH;
     pend[h] = false;
   };
   auto refill = [&]() {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const uint32_t p = __builtin_amdgcn_readlane(ptr[0], (uint32_t)h * 32u);
+      const int32_t p = (int32_t)__builtin_amdgcn_readlane(ptr[0], (uint32_t)h * 32u);
       if constexpr (KB == 1) {
-        if (!pend[h] && lo[h] > 0 && p <= lo[h] + kH) fetch(h);
-        if (pend[h] && p < lo[h] + 64u) commit(h);
+        if (!pend[h] && lo[h] > 0 && p <= (int32_t)(lo[h] + kH)) fetch(h);
+        if (pend[h] && p < (int32_t)(lo[h] + 64u)) commit(h);
       } else {
         if (!pend[h] && lo[h] > 0) fetch(h);
-        if (pend[h] && p <= lo[h] + kH) {
+        if (pend[h] && p <= (int32_t)(lo[h] + kH)) {
           commit(h);
           if (lo[h] > 0) fetch(h);
         }
@@ -1356,12 +1353,12 @@ __device__ void decode_ticket32(const BatchBuf& B, uint32_t b, uint32_t lt, cons
     for (uint32_t s = all; s > full;) {
       --s;
       const bool v[1] = {s * L + lin < n};
-      store(s, dec_steps<L, PB, 1, kMask, uint32_t>(x, ptr, taken, lut, stage, v, half), v[0]);
+      store(s, dec_steps<L, PB, 1, kMask, uint32_t, false>(x, ptr, taken, lut, stage, v, half), v[0]);
       refill();
     }
     for (uint32_t s = full; s > 0;) {
       --s;
-      store(s, dec_steps<L, PB, 1, kMask, uint32_t>(x, ptr, taken, lut, stage, vall, half), true);
+      store(s, dec_steps<L, PB, 1, kMask, uint32_t, false>(x, ptr, taken, lut, stage, vall, half), true);
       refill();
     }
   } else {
@@ -1369,80 +1366,100 @@ __device__ void decode_ticket32(const BatchBuf& B, uint32_t b, uint32_t lt, cons
     while (s > full || s % KB != 0) {
       --s;
       const bool v[1] = {s * L + lin < n};
-      store(s, dec_steps<L, PB, 1, kMask, uint32_t>(x, ptr, taken, lut, stage, v, half), v[0]);
+      store(s, dec_steps<L, PB, 1, kMask, uint32_t, false>(x, ptr, taken, lut, stage, v, half), v[0]);
       if (s % KB == 0) refill();
     }
     while (s > 0) {
 #pragma unroll
       for (int j = 0; j < KB; ++j) {
         --s;
-        store(s, dec_steps<L, PB, 1, kMask, uint32_t>(x, ptr, taken, lut, stage, vall, half), true);
+        store(s, dec_steps<L, PB, 1, kMask, uint32_t, false>(x, ptr, taken, lut, stage, vall, half), true);
       }
       refill();
     }
   }
-  const bool bad = act && (taken[0] != (half ? wordsh[1] : wordsh[0]) || x[0] != kMinState);
+  const bool bad = act && (ptr[0] != 0u || x[0] != kMinState);
   if (__ballot(bad) && lane == 0) {
     atomicOr(a.err, kErrFinalState);
     atomicOr(a.bad + b, kErrFinalState);
   }
 }
 
+// A workgroup takes an item, some tickets of one buffer (of one plane pair of a
+// uint32 buffer), builds the buffer's LUTs in LDS and decodes the tickets there, a
+// wavefront at a time.  Bound by LDS reads and their latency, as the
+// single-buffer decoder, and by the end of the launch, where a ticket takes
+// some 60 us.  1024 buffers of 590 MB: 0.38 ms; with LUTs built once per
+// buffer by queue items of their own, copied by every wavefront into its LDS,
+// 0.71 (12 wavefronts a CU).  A split of the tickets into equal shares, one a
+// workgroup, took 0.50: workgroups that get more buffers build more LUTs and
+// wait for their slowest wavefront more often.  The frames are read through
+// global pointers: by generic ones the compiler takes the loads' results for
+// divergent, keeps the ring positions in vector registers and waits for LDS
+// on every fetch (0.42).
 template <int PB, int NW, int KB, int L>
 __global__ __launch_bounds__(64 * NW) void batch_decode_kernel(BatchDecodeArgs a) {
   constexpr uint32_t W = 1u << PB;
-  constexpr uint32_t WAVE_WORDS = 2 * W + DecRing<KB>::WORDS;  // two LUTs | two rings (u16)
-  extern __shared__ uint32_t lds[];
-  const uint32_t lane = threadIdx.x & 63u;
+  extern __shared__ uint4 lds4[];  // [2][W] LUT entries | per wavefront two rings (u16)
+  __shared__ uint32_t s_item[2];
   const uint32_t wave = wave_u32(threadIdx.x >> 6);
-  uint32_t* wl = lds + wave * WAVE_WORDS;
-  const uint32_t gen = wave_u32(lane == 0 ? atomic_ld32(a.queue + 2) : 0u);
-  uint64_t tkey = ~0ull;  // LUTs held in this wave's LDS
-  uint32_t it = 0;
-  const uint32_t run = a.run;
-  if (lane == 0) it = atomicAdd(a.queue, run);
-  it = wave_u32(it);
-  uint32_t run_end = it + run;
-  while (it < a.nitems) {
-    const uint32_t b = wave_u32(a.items[it].x);
+  uint32_t* const lut = (uint32_t*)lds4;
+  uint16_t* const rings = (uint16_t*)(lut + 2 * W);
+  uint16_t* const wstage = rings + wave * (2 * DecRing<KB>::WORDS);
+  // (the build's cumulative sums take the rings' place)
+  uint32_t (*const cdf)[kNumSymbols + 1] = (uint32_t(*)[kNumSymbols + 1]) rings;
+  static_assert(sizeof(uint32_t) * 2 * (kNumSymbols + 1) <= NW * 4 * DecRing<KB>::WORDS, "cdf in the rings");
+  // (the first item is the workgroup's number: the queue's atomics take 11 ns
+  // each, 17 us for a launch's first ones)
+  for (uint32_t k = 0, it = blockIdx.x; it < a.nitems; it = wave_u32(s_item[k++ & 1u])) {
+    if (threadIdx.x == 0) s_item[k & 1u] = gridDim.x + atomicAdd(a.queue, 1u);
+    const uint2 itm = a.items[it];
+    const uint32_t b = wave_u32(itm.x), first = wave_u32(itm.y) & kItemFirst,
+                   cnt = (wave_u32(itm.y) >> kItemFirstBits) + 1u;
     const BatchBuf& B = a.bufs[b];
-    if (it < a.nbufs) {
-      build_luts<PB>(B, b, a, gen, wl);  // uses the LUT area as scratch
-      tkey = ~0ull;
-    } else {
-      uint32_t r = 0;
-      while (((r = wave_u32(lane == 0 ? atomic_ld32(a.ready + b) : 0u)) & ~kBatchBad) != gen)
-        __builtin_amdgcn_s_sleep(2);
-      if (!(r & kBatchBad)) {
-        const uint32_t lt = it - a.nbufs - B.tick_first;
-        if constexpr (L == 32) decode_ticket32<PB, KB>(B, b, lt, a, wl, tkey);
-        else if (B.eb == 1) decode_ticket<PB, false, KB>(B, b, lt, a, wl, tkey);
-        else decode_ticket<PB, true, KB>(B, b, lt, a, wl, tkey);
+    // (a uint32 buffer numbers the second pair's tickets after the first's)
+    const uint32_t nt = B.eb == 1 ? (uint32_t)div_up(B.nb, 2) : (uint32_t)B.nb;
+    const uint32_t pair = nt > 0 && first >= nt ? 1u : 0u;
+    const uint32_t np = B.eb == 1 ? 1u : 2u, p0 = 2u * pair;
+    bool bad = frame_bad<PB>(B);
+    if (!bad) bad = build_luts<PB, NW>(B, p0, np, lut, cdf);
+    if (bad && threadIdx.x == 0) {
+      atomicOr(a.err, kErrMagic);
+      atomicOr(a.bad + b, kErrMagic);
+    }
+    __syncthreads();
+    if (!bad && nt > 0) {
+      for (uint32_t i = wave; i < cnt; i += NW) {
+        const uint32_t lt = first + i - pair * nt;
+        if constexpr (L == 32) {
+          if (B.eb == 1) decode_ticket32<PB, 1, KB>(B, b, lt, p0, a, lut, wstage);
+          else if (B.eb == 2) decode_ticket32<PB, 2, KB>(B, b, lt, p0, a, lut, wstage);
+          else decode_ticket32<PB, 4, KB>(B, b, lt, p0, a, lut, wstage);
+        } else {
+          if (B.eb == 1) decode_ticket<PB, 1, KB>(B, b, lt, p0, a, lut, wstage);
+          else if (B.eb == 2) decode_ticket<PB, 2, KB>(B, b, lt, p0, a, lut, wstage);
+          else decode_ticket<PB, 4, KB>(B, b, lt, p0, a, lut, wstage);
+        }
+        drain();
       }
     }
-    drain();
-    if (++it == run_end) {
-      uint32_t nxt = 0;
-      if (lane == 0) nxt = atomicAdd(a.queue, run);
-      it = wave_u32(nxt);
-      run_end = it + run;
-    }
+    __syncthreads();  // (the LUTs are rebuilt)
   }
-  if (lane == 0) {
-    const uint32_t total = gridDim.x * NW;
-    if (atomicAdd(a.queue + 1, 1u) + 1 == total) {
+  // the last workgroup out resets the queue for the next launch
+  if (threadIdx.x == 0) {
+    if (atomicAdd(a.queue + 1, 1u) + 1 == gridDim.x) {
       atomic_st32(a.queue, 0u);
       atomic_st32(a.queue + 1, 0u);
-      atomic_st32(a.queue + 2, gen % kBatchGenMask + 1u);
     }
   }
 }
 
 template <int PB, int NW, int KB>
 hipError_t launch_dec_shape(const BatchDecodeArgs& a, int cu, hipStream_t s) {
-  constexpr size_t lds = (size_t)NW * (2 * (1u << PB) + DecRing<KB>::WORDS) * 4u;
-  static_assert(lds == batch_decode_lds(BatchShape{NW, KB}, PB), "decode LDS layout");
-  if constexpr (lds > kLdsBytes) {
+  constexpr size_t rings = (size_t)NW * 2u * DecRing<KB>::WORDS * 2u;
+  constexpr size_t lds = 2u * (1u << PB) * sizeof(uint32_t) + rings;
+  static_assert(lds + 64u <= batch_decode_lds(BatchShape{NW, KB}, PB), "every admitted shape fits the LDS");
+  if constexpr (batch_decode_lds(BatchShape{NW, KB}, PB) > kLdsBytes) {
     return hipErrorInvalidConfiguration;
   } else {
     int per_cu = 0;
@@ -1452,8 +1469,7 @@ hipError_t launch_dec_shape(const BatchDecodeArgs& a, int cu, hipStream_t s) {
     if (e != hipSuccess) return e;
     if (per_cu < 1) per_cu = 1;
     uint64_t grid = (uint64_t)cu * (uint64_t)per_cu;
-    const uint64_t want = div_up(a.nitems, (uint64_t)NW * a.run);
-    if (want < grid) grid = want;
+    if (a.nitems < grid) grid = a.nitems;
     if (grid < 1) grid = 1;
     if (a.lanes == 32) hipLaunchKernelGGL((batch_decode_kernel<PB, NW, KB, 32>), dim3((uint32_t)grid), dim3(64 * NW), lds, s, a);
     else hipLaunchKernelGGL((batch_decode_kernel<PB, NW, KB, 64>), dim3((uint32_t)grid), dim3(64 * NW), lds, s, a);

@@ -1115,7 +1115,6 @@ struct mans_batch {
   uint32_t* ptot = nullptr;   // [cap_bufs][4]
   uint32_t* fin = nullptr;    // [cap_bufs]
   uint32_t* queue = nullptr;  // [4] next item, exited waves, generation, next chunk
-  uint32_t* luts = nullptr;   // decode: [cap_bufs][4][2^p]
   BatchBuf* h_bufs = nullptr; // pinned staging for asynchronous plans (or null):
                               // descriptors then items, one upload
   const uint2* items_dev = nullptr;  // the plan's items (item_buf, or after the
@@ -1141,7 +1140,7 @@ namespace {
 
 void batch_free(mans_batch* b) {
   void* dev[] = {b->bufs, b->item_buf, b->hist, b->done, b->ready, b->tables,
-                 b->status, b->ptot, b->fin, b->queue, b->luts, b->spill_buf, b->bad, b->arch_off};
+                 b->status, b->ptot, b->fin, b->queue, b->spill_buf, b->bad, b->arch_off};
   for (void* q : dev)
     if (q) (void)hipFree(q);
   if (b->h_bufs) (void)hipHostFree(b->h_bufs);
@@ -1153,16 +1152,15 @@ std::atomic<uint32_t> g_force_chunk{0}, g_force_rounds{0}, g_force_run{0};
 
 // The work-item grain of a batch of `bytes` uncompressed bytes in `units`
 // byte-plane blocks on a chip of `cu` compute units: the largest items that
-// still leave about 32 histogram chunks, 32 encode tickets and 128 decode
-// runs per CU (a launch keeps 8-16 wavefronts per CU busy and the queue
-// balances their tails), within the bounds of each.  4096 buffers of 8 GB
-// take the largest grain; one request of a few tens of MB the smallest.
+// still leave about 32 histogram chunks and 32 encode tickets per CU (a launch
+// keeps 8-16 wavefronts per CU busy and the queue balances their tails),
+// within the bounds of each.  4096 buffers of 8 GB take the largest grain; one
+// request of a few tens of MB the smallest.  Decode items: DecodeItems.
 BatchGrain batch_grain(uint64_t bytes, uint64_t units, int cu) {
   const uint64_t c = (uint64_t)std::max(cu, 1);
-  BatchGrain g{kBatchHistChunkMin, 1, 1};
+  BatchGrain g{kBatchHistChunkMin, 1, 0};
   while (g.hist_chunk < kBatchHistChunkMax && bytes / (2ull * g.hist_chunk) >= 32 * c) g.hist_chunk *= 2;
   while (g.rounds < 4 && units / (4ull * 2 * g.rounds) >= 32 * c) g.rounds *= 2;
-  if (units / (2ull * 4) >= 128 * c) g.run = 4;
   const uint32_t fc = g_force_chunk.load(), fr = g_force_rounds.load(), fu = g_force_run.load();
   if (fc) g.hist_chunk = fc;
   if (fr) g.rounds = fr;
@@ -1273,7 +1271,6 @@ mans_status batch_alloc(mans_batch* b, uint32_t cap_bufs, uint64_t cap_items, ui
   const uint32_t q0[4] = {0, 0, 1, 0};  // next item, exited waves, first generation, next chunk
   HIP_TRY(hipMemcpy(b->queue, q0, 16, hipMemcpyHostToDevice));
   if (b->decode) {
-    HIP_TRY(hipMalloc(&b->luts, nb1 * 4 * (4ull << b->pb)));
     HIP_TRY(hipMalloc(&b->bad, nb1 * 4));
     HIP_TRY(hipMemset(b->bad, 0, nb1 * 4));
   } else {
@@ -1296,6 +1293,34 @@ mans_status batch_alloc(mans_batch* b, uint32_t cap_bufs, uint64_t cap_items, ui
   return MANS_OK;
 }
 
+// Writes (or, with dst null, counts) the decode items of the planned buffers.
+// An item's tickets share one build of the LUTs, so items are large while
+// much of the batch is left, and small at the end, where they balance the
+// workgroups' finish: 16 tickets while every workgroup the chip holds (about
+// six a CU) has two items of that size before it, then 8, then 4.
+uint64_t decode_items(const std::vector<BatchBuf>& bufs, const BatchGrain& g, uint64_t nticks, int cu, uint2* dst) {
+  uint64_t k = 0, left = nticks;
+  const uint64_t wgs = 6ull * (uint64_t)std::max(cu, 1);
+  for (size_t i = 0; i < bufs.size(); ++i) {
+    const uint32_t pairs = bufs[i].eb == 4 ? 2u : 1u, nt = bufs[i].nticks / pairs;
+    if (nt == 0) {
+      if (dst) dst[k] = make_uint2((uint32_t)i, 0u);
+      ++k;
+    }
+    for (uint32_t q = 0; q < pairs; ++q)
+      for (uint32_t r = 0; r < nt;) {
+        uint32_t per = 4u * g.run;
+        if (per == 0) per = left >= 2 * 16 * wgs ? 16u : (left >= 2 * 8 * wgs ? 8u : 4u);
+        const uint32_t c = std::min(per, nt - r);
+        if (dst) dst[k] = make_uint2((uint32_t)i, (q * nt + r) | (c - 1u) << kItemFirstBits);
+        ++k;
+        r += c;
+        left -= c;
+      }
+  }
+  return k;
+}
+
 // Plans `count` buffers into b (which must hold them) and uploads the
 // descriptors: on stream s from the pinned staging when b has one (the
 // staging must not be in use by an earlier upload), else synchronously.
@@ -1305,7 +1330,8 @@ mans_status batch_plan(mans_batch* b, const mans_params* p, const mans_buffer* h
   const BatchGrain grain = grain_of(h_bufs, count, b->ws->cu, p->lanes);
   mans_status st = plan_batch(p, h_bufs, count, b->decode, grain, bufs, nhist, nticks);
   if (st != MANS_OK) return st;
-  const uint64_t nitems = (b->decode ? (uint64_t)count : nhist) + nticks;
+  const uint64_t nitems =
+      b->decode ? decode_items(bufs, grain, nticks, b->ws->cu, nullptr) : nhist + nticks;
   if ((uint32_t)count > b->cap_bufs || nitems > b->cap_items || nticks > b->cap_ticks) return MANS_ERR_TOO_LARGE;
   std::vector<uint2> items;
   const size_t items_off = round_up((uint64_t)count * sizeof(BatchBuf), 16);
@@ -1316,10 +1342,7 @@ mans_status batch_plan(mans_batch* b, const mans_params* p, const mans_buffer* h
   }
   uint64_t k = 0;
   if (b->decode) {
-    // every buffer's LUT item, then the tickets in buffer order
-    for (int32_t i = 0; i < count; ++i) dst[k++] = make_uint2((uint32_t)i, 0u);
-    for (int32_t i = 0; i < count; ++i)
-      for (uint32_t r = 0; r < bufs[(size_t)i].nticks; ++r) dst[k++] = make_uint2((uint32_t)i, 0u);
+    decode_items(bufs, grain, nticks, b->ws->cu, dst);
   } else {
     // histogram chunks in buffer order, then the tickets in buffer order
     // (the kernel takes each kind from its own counter)
@@ -1641,7 +1664,7 @@ mans_status mans_batch_decode_create(mans_batch** out, const mans_params* p, con
 
 mans_status mans_batch_decode_run(mans_batch* b, void* stream) {
   if (!b || !b->decode) return MANS_ERR_INVALID_ARG;
-  if (b->nitems == 0) return MANS_OK;
+  if (b->nbufs == 0) return MANS_OK;
   mans_workspace* ws = b->ws;
   DeviceGuard g(ws->device);
   hipStream_t s = (hipStream_t)stream;
@@ -1651,12 +1674,9 @@ mans_status mans_batch_decode_run(mans_batch* b, void* stream) {
   a.items = b->items_dev;
   a.nbufs = b->nbufs;
   a.nitems = b->nitems;
-  a.ready = b->ready;
-  a.luts = b->luts;
   a.queue = b->queue;
   a.err = ws->counters + 3;
   a.bad = b->bad;
-  a.run = b->grain.run;
   a.lanes = b->lanes;
   // per-buffer flags start at zero in every run (a kernel, so the run can
   // be captured)
@@ -1812,8 +1832,8 @@ mans_status mans_batch_tune(mans_batch* b, void* stream, int32_t reps, mans_tune
   for (int i = 0; i < ncand && st == MANS_OK; ++i) {
     const BatchShape c{kNws[i / nkb], kbs[i % nkb]};
     const bool fits = batch_shape_ok(c, b->pb, b->decode);
-    double ms = fits && b->nitems == 0 ? 0.0 : -1.0;
-    if (fits && b->nitems > 0) {
+    double ms = fits && b->nbufs == 0 ? 0.0 : -1.0;
+    if (fits && b->nbufs > 0) {
       b->shape = c;
       auto run = [&]() { return b->decode ? mans_batch_decode_run(b, s) : mans_batch_encode_run(b, d_sizes, s); };
       st = run();

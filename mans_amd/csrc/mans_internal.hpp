@@ -253,22 +253,21 @@ struct BatchEncodeArgs {
   uint32_t lanes;                // every buffer's frame: 64 or 32 lanes
   uint32_t hist_wgs;             // workgroups that start on histogram chunks (set at launch)
 };
-// Batched decode: BatchBuf.in is the frame, .out the elements; items
-// [0, nbufs) build buffer b's LUTs, then come the decode tickets.
+// Batched decode: BatchBuf.in is the frame, .out the elements.  A queue item
+// is up to 16 tickets of one buffer (of one plane pair of a uint32 buffer): {buffer,
+// first ticket | (tickets - 1) << kItemFirstBits}; a buffer without blocks has
+// one item too, which checks its frame.
+constexpr uint32_t kItemFirstBits = 28, kItemFirst = (1u << kItemFirstBits) - 1u;
 struct BatchDecodeArgs {
   const BatchBuf* bufs;
-  const uint2* items;            // [nitems] {buffer, 0}: LUT items, then tickets
+  const uint2* items;            // [nitems]
   uint32_t nbufs;
   uint32_t nitems;
-  uint32_t* ready;               // [nbufs] generation whose LUTs are built (| kBatchBad: frame rejected)
-  uint32_t* luts;                // [nbufs][4][2^p] packed LUT entries
-  uint32_t* queue;               // [4] as BatchEncodeArgs::queue (next item, exited, generation)
+  uint32_t* queue;               // [2] next item, exited workgroups (both left zeroed)
   uint32_t* err;
   uint32_t* bad;                 // [nbufs] the error flags of each buffer (zeroed before the launch)
-  uint32_t run;                  // items a wavefront takes per queue grab (BatchGrain)
   uint32_t lanes;                // every buffer's frame: 64 or 32 lanes
 };
-constexpr uint32_t kBatchBad = 1u << 31;
 constexpr uint32_t kBatchGenMask = 0x3fffu;     // 14-bit generations
 // Work-item grain of a batched launch, picked per plan from the batch's
 // size against the chip (batch_grain in capi.hip): a large batch takes big
@@ -280,7 +279,7 @@ constexpr uint32_t kBatchHistChunkMax = 1u << 19;
 struct BatchGrain {
   uint32_t hist_chunk;  // power of two in [kBatchHistChunkMin, kBatchHistChunkMax]
   uint32_t rounds;      // encode ticket rounds: 1, 2 or 4
-  uint32_t run;         // decode items per grab: 1 or 4
+  uint32_t run;         // a fourth of the tickets per decode item: 1 or 4, 0: by what is left of the batch
 };
 
 // ---- archive: the frames of a batch in one container (archive.hip) --------
@@ -351,8 +350,9 @@ struct BatchShape {
 };
 constexpr BatchShape kBatchEncodeDefault = {4, 16};
 constexpr BatchShape kBatchDecodeDefault = {4, 8};
-// LDS bytes per workgroup of a shape (encode: tables | stages per
-// wave; decode: two LUTs | two rings per wave)
+// LDS bytes per workgroup a shape is admitted by (encode: tables | stages
+// per wave; decode: two 4-byte LUTs and two rings a wave, more than the
+// launch takes)
 constexpr uint64_t batch_encode_lds(BatchShape sh) { return (uint64_t)sh.nw * (2u * 256u * 2u + 1024u) * 4u; }
 constexpr uint64_t batch_decode_lds(BatchShape sh, int pb) {
   return (uint64_t)sh.nw * (2ull * (1u << pb) * 4u +
