@@ -7,16 +7,16 @@
 // it alone (MANS_MODE_PLANES, in the batch's 64- or 32-lane format): the same
 // histogram and normalisation (GpuANSStatistics.h:23-151, :186-406), the
 // same rANS arithmetic and container (GpuANSEncode.h:24-164, :180-284).  What
-// changes is the schedule.  One queue of work items (an atomic counter) holds
-// the histogram chunks of every buffer and its encode tickets, the tickets of
-// a buffer queued a few hundred items after its last chunk; every wavefront
-// takes items one at a time:
-//  * a histogram item counts one chunk of one buffer (all its byte planes)
-//    into LDS and adds the counts to the buffer's accumulators; the wavefront
-//    that finishes a buffer's last chunk normalises its planes (one wavefront
-//    per buffer), writes the frame and plane headers and publishes the
+// changes is the schedule.  A persistent launch works through two queues
+// (atomic counters), the histogram chunks of every buffer and then its encode
+// tickets:
+//  * every workgroup counts chunks (all byte planes of one buffer's chunk)
+//    until none is left and adds the counts to the buffer's accumulators; the
+//    workgroup that declares a buffer's last chunk done normalises its planes
+//    (a wavefront each), writes the frame and plane headers and publishes the
 //    encoder tables, then marks the buffer ready;
-//  * a 64-lane encode ticket is 1, 2 or 4 rounds of four chains per lane (two
+//  * then every wavefront takes tickets one at a time:
+//    a 64-lane encode ticket is 1, 2 or 4 rounds of four chains per lane (two
 //    for uint32) with the single-buffer coder's step; a 32-lane ticket is two
 //    units, one per half-wave.  A ticket waits until its buffer is ready,
 //    codes its units and resolves its output offset by decoupled look-back
@@ -47,8 +47,12 @@ constexpr uint32_t kStageWords = 4 * 512 / 2;
 constexpr uint32_t kWaveWords = kTabWords + kStageWords;
 template <typename T>
 using gptr = const __attribute__((address_space(1))) T*;
+// a writable one.  (Frames and elements are reached through pointers read from
+// memory, which the compiler must take for generic: flat accesses, whose
+// completion every wait for LDS then includes.)
+template <typename T>
+using gout = __attribute__((address_space(1))) T*;
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ uint32_t wave_u32(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 
@@ -115,33 +119,42 @@ __device__ __forceinline__ void wg_hist_chunk(const uint8_t* in, uint64_t c0, ui
   const uint32_t ntiles = n / (16u * kTileU4);
   int32_t sum[EB][4] = {};
   count_tiles<(int)EB>((const uint4*)(in + c0), wave_u32(t >> 6), ntiles, NW, sum);
-  for (uint32_t i = 16u * kTileU4 * ntiles + t; i < n; i += 64u * NW) count_byte(cnt, i % EB, in[c0 + i]);
+  for (uint32_t i = 16u * kTileU4 * ntiles + t; i < n; i += 64u * NW) count_byte(cnt, i % EB, ((gptr<uint8_t>)in)[c0 + i]);
+  publish();  // the previous chunk's adds
   __syncthreads();
   flush_counts<(int)EB, 64 * NW>(sum, cnt, ghist);
 }
 
-// The histogram phase of a workgroup that starts on histograms: it takes
-// chunk items from their own counter (queue[3]) until none is left, one
-// workgroup barrier round per chunk (the next grab is taken while the
-// current chunk is counted); the workgroup that counts a buffer's last chunk
-// runs its finisher on wavefront 0.  LDS: the counts, the finisher's 256
-// keys, the two grabbed items and the finish flag.
-template <int PB>
+// The histogram phase: a workgroup takes chunk items from their own counter
+// until none is left, the next grab taken while the current chunk is counted.
+// Each chunk is declared done one chunk later, when its adds to the
+// accumulators have had the next chunk's counting time to complete; the
+// workgroup that declares a buffer's last one finishes the buffer.  LDS: the
+// counts, the finisher's keys, the two grabbed items and the finish flag.
+template <int PB, int NW>
 __device__ void finish_buffer(const BatchBuf& B, uint32_t b, const BatchEncodeArgs& a, uint32_t gen, uint32_t* keys);
 
 template <int PB, int NW>
 __device__ void hist_phase(const BatchEncodeArgs& a, uint32_t gen, uint32_t* lds) {
-  static_assert(kFlushWords + 256u + 4u <= NW * kWaveWords, "the histogram phase fits the workgroup's LDS");
+  constexpr uint32_t kKeys = kMaxPlanes * kNumSymbols;
+  static_assert(kFlushWords + kKeys + 4u <= NW * kWaveWords, "the histogram phase fits the workgroup's LDS");
   uint32_t* const cnt = lds;
   uint32_t* const keys = lds + kFlushWords;
-  uint32_t* const s_it = keys + 256;  // [0..1] grabbed items, [2] finish flag
+  uint32_t* const s_it = keys + kKeys;  // [0..1] grabbed items, [2] finish flag
   for (uint32_t i = threadIdx.x; i < kFlushWords; i += 64u * NW) cnt[i] = 0;
-  if (threadIdx.x == 0) s_it[0] = atomicAdd(a.queue + 3, 1u);
+  if (threadIdx.x == 0) s_it[0] = atomicAdd(a.queue + kQueueChunk, 1u);
   __syncthreads();
+  uint32_t prev = ~0u;  // the buffer of the chunk counted last
+  // with every wavefront past its publish() and a barrier
+  auto declare = [&]() {
+    if (threadIdx.x == 0) s_it[2] = atomicAdd(a.done + prev, 1u) + 1u == a.bufs[prev].nhist ? 1u : 0u;
+    __syncthreads();
+    if (s_it[2]) finish_buffer<PB, NW>(a.bufs[prev], prev, a, gen, keys);
+  };
   for (uint32_t k = 0;; ++k) {
     const uint32_t it = wave_u32(s_it[k & 1u]);
     if (it >= a.nhist_items) break;
-    if (threadIdx.x == 0) s_it[(k + 1) & 1u] = atomicAdd(a.queue + 3, 1u);
+    if (threadIdx.x == 0) s_it[(k + 1) & 1u] = atomicAdd(a.queue + kQueueChunk, 1u);
     const uint2 itm = a.items[it];
     const uint32_t b = wave_u32(itm.x), li = wave_u32(itm.y);
     const BatchBuf& B = a.bufs[b];
@@ -153,23 +166,28 @@ __device__ void hist_phase(const BatchEncodeArgs& a, uint32_t gen, uint32_t* lds
       if (B.eb == 1) wg_hist_chunk<1, NW>(B.in, c0, c1, cnt, ghist);
       else if (B.eb == 2) wg_hist_chunk<2, NW>(B.in, c0, c1, cnt, ghist);
       else wg_hist_chunk<4, NW>(B.in, c0, c1, cnt, ghist);
+    } else {
+      publish();  // (an empty buffer)
     }
+    __syncthreads();
+    if (prev != ~0u) declare();
+    prev = b;
+  }
+  if (prev != ~0u) {
     publish();
     __syncthreads();
-    if (threadIdx.x == 0) s_it[2] = atomicAdd(a.done + b, 1u) + 1u == B.nhist ? 1u : 0u;
-    __syncthreads();
-    if (s_it[2] && threadIdx.x < 64) finish_buffer<PB>(B, b, a, gen, keys);
+    declare();
   }
   __syncthreads();  // (the LDS becomes the wavefronts' ticket areas)
 }
 
-// ---- finisher: one wavefront normalises every plane of buffer b -----------
-template <int PB>
+// ---- finisher: a workgroup normalises buffer b, a wavefront per plane ------
+template <int PB, int NW>
 __device__ void finish_buffer(const BatchBuf& B, uint32_t b, const BatchEncodeArgs& a, uint32_t gen, uint32_t* keys) {
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t P = B.eb;
+  static_assert(NW >= (int)kMaxPlanes, "a wavefront per plane");
+  const uint32_t lane = threadIdx.x & 63u, k = wave_u32(threadIdx.x >> 6);
   bool bad = false;
-  for (uint32_t k = 0; k < P; ++k) {
+  if (k < B.eb) {
     uint32_t* h = a.hist + (uint64_t)b * 1024u + k * 256u;
     uint32_t c[4];
 #pragma unroll
@@ -178,7 +196,7 @@ __device__ void finish_buffer(const BatchBuf& B, uint32_t b, const BatchEncodeAr
       atomic_st32(h + 4 * lane + j, 0u);
     }
     uint4 e[4];
-    normalize_wave(c, (uint32_t)B.n, PB, keys, e, bad);
+    normalize_wave(c, (uint32_t)B.n, PB, keys + k * kNumSymbols, e, bad);
     uint64_t* t2 = (uint64_t*)(a.tables + ((uint64_t)b * 4u + k) * 256u);
     uint16_t pr[4];
 #pragma unroll
@@ -188,9 +206,9 @@ __device__ void finish_buffer(const BatchBuf& B, uint32_t b, const BatchEncodeAr
       atomic_st64(t2 + 4 * lane + j, ((uint64_t)f.y << 32) | f.x);
       pr[j] = (uint16_t)e[j].x;
     }
-    uint8_t* sec = B.out + B.section[k];
-    ((uint2*)(sec + kAnsHeaderBytes))[lane] =
-        make_uint2((uint32_t)pr[0] | ((uint32_t)pr[1] << 16), (uint32_t)pr[2] | ((uint32_t)pr[3] << 16));
+    const gout<uint8_t> sec = (gout<uint8_t>)B.out + B.section[k];
+    ((gout<u32x2>)(sec + kAnsHeaderBytes))[lane] =
+        u32x2{(uint32_t)pr[0] | ((uint32_t)pr[1] << 16), (uint32_t)pr[2] | ((uint32_t)pr[3] << 16)};
     if (lane < 8) {
       uint32_t f = 0;
       if (lane == 0) f = (kAnsMagic << 16) | (B.lanes == 32 ? 1u : 2u);  // reference / native format version
@@ -199,17 +217,19 @@ __device__ void finish_buffer(const BatchBuf& B, uint32_t b, const BatchEncodeAr
       if (lane == 4) f = (uint32_t)PB;
       // totalCompressedWords (field 3) is written by the buffer's last
       // ticket to finish; no other store may touch its bytes before that
-      if (lane != 3 || B.nticks == 0) ((uint32_t*)sec)[lane] = f;
+      if (lane != 3 || B.nticks == 0) ((gout<uint32_t>)sec)[lane] = f;
     }
-    if ((B.nb & 1) && lane < 2) ((uint32_t*)(sec + kSectionFixed + 4ull * B.lanes * B.nb + 8ull * B.nb))[lane] = 0;
+    if ((B.nb & 1) && lane < 2) ((gout<uint32_t>)(sec + kSectionFixed + 4ull * B.lanes * B.nb + 8ull * B.nb))[lane] = 0;
   }
   // frame header; data_words / total_size (bytes 48..63) belong to the
   // buffer's last ticket unless there is none
-  if (lane < 32 && (lane < 12 || lane >= 16 || B.nticks == 0)) ((uint32_t*)B.out)[lane] = B.frame_hdr[lane];
-  if (B.nticks == 0 && lane == 0) a.sizes[b] = B.data_off;
+  if (k == 0 && lane < 32 && (lane < 12 || lane >= 16 || B.nticks == 0))
+    ((gout<uint32_t>)B.out)[lane] = B.frame_hdr[lane];
+  if (B.nticks == 0 && threadIdx.x == 0) a.sizes[b] = B.data_off;
   if (bad && lane == 0) atomicOr(a.err, kErrTable);
   publish();
-  if (lane == 0) {
+  __syncthreads();
+  if (threadIdx.x == 0) {
     atomic_st32(a.done + b, 0u);
     atomic_st32(a.ready + b, gen);
   }
@@ -252,7 +272,6 @@ template <int PB, int EB, int KBB>
 __device__ uint64_t encode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, uint64_t tix, const BatchEncodeArgs& a,
                               uint32_t gen, uint32_t* wl, uint16_t* spill, uint64_t& tkey) {
   constexpr int CH = (int)enc_chains(EB);                    // chains per round
-  constexpr int UT = (int)enc_ticket_units(EB, kMaxRounds);  // units per ticket, at most
   const uint32_t R = a.rounds, UTR = R * (uint32_t)CH;      // rounds, units of this ticket
   constexpr int SPB = EB == 4 ? 2 : EB;          // chains per element block (planes coded together)
   constexpr int BPT = CH / SPB;                  // element blocks per round
@@ -267,10 +286,9 @@ __device__ uint64_t encode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, ui
   const uint64_t u0 = (uint64_t)UTR * lt;
   uint2* s_tab = (uint2*)wl;  // [SPB <= 2][256]
   uint16_t* wstage = (uint16_t*)(wl + kTabWords);
-  static_assert(UT <= kMaxTicketUnits, "a ticket's units fit its slot");
-  uint32_t padj[UT];  // per unit of the ticket (wave-uniform)
-#pragma unroll
-  for (int j = 0; j < UT; ++j) padj[j] = 0;
+  static_assert(enc_ticket_units(EB, kMaxRounds) <= kMaxTicketUnits, "a ticket's units fit its slot");
+  uint32_t pv = 0;  // lane j: unit j's padded words
+  uint32_t ptot[EB == 1 ? 1 : EB] = {};  // padded words per plane
 
 #pragma unroll 1
   for (uint32_t r = 0; r < R; ++r) {
@@ -326,7 +344,7 @@ __device__ uint64_t encode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, ui
         const uint32_t un = (sb[c] - cb[c]) >> 1;  // unspilled words
         if (un >= H) {
           uint16_t* st = wstage + c * REG;
-          if (lane < H4) ((uint4*)(rspill + c * CSTAGE + fl[c]))[lane] = ((const uint4*)st)[lane];
+          if (lane < H4) ((gout<u32x4>)(rspill + c * CSTAGE + fl[c]))[lane] = ((const u32x4*)st)[lane];
           if (4u * lane < un - H) ((uint2*)st)[lane] = ((const uint2*)(st + H))[lane];
           fl[c] += H;
           sb[c] -= 2u * H;
@@ -430,32 +448,33 @@ __device__ uint64_t encode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, ui
       uint16_t* st = wstage + c * REG;
       if (lane < padded - cnt) st[rem + lane] = 0;
       const uint32_t nr = padded > fl[c] ? (padded - fl[c]) / 8 : 0u;
-      for (uint32_t k = lane; k < nr; k += kL) ((uint4*)(rspill + c * CSTAGE + fl[c]))[k] = ((const uint4*)st)[k];
+      for (uint32_t k = lane; k < nr; k += kL) ((gout<u32x4>)(rspill + c * CSTAGE + fl[c]))[k] = ((const u32x4*)st)[k];
       const uint32_t kp = p0 + (uint32_t)(c % SPB);
       if (act[c]) {
-        ((uint32_t*)(B.out + B.section[kp] + kSectionFixed))[blk[c] * kL + lane] = x[c];
-        if (lane == 0) {
-          ((uint32_t*)(B.out + B.section[kp] + kSectionFixed + 4ull * kL * B.nb + 8ull * blk[c]))[0] =
+        ((gout<uint32_t>)(B.out + B.section[kp] + kSectionFixed))[blk[c] * kL + lane] = x[c];
+        if (lane == 0)
+          ((gout<uint32_t>)(B.out + B.section[kp] + kSectionFixed + 4ull * kL * B.nb + 8ull * blk[c]))[0] =
               (n[c] << 16) | cnt;
-          atomicAdd(a.ptot + 4ull * b + kp, padded);
-        }
       }
-#pragma unroll
-      for (int j = 0; j < UT; ++j)
-        if ((uint32_t)j == j0 + (uint32_t)c) padj[j] = padded;
+      pv = lane == j0 + (uint32_t)c ? padded : pv;
+      if constexpr (EB == 4) {
+        ptot[c] += p0 == 0 ? padded : 0u;
+        ptot[2 + c] += p0 == 0 ? 0u : padded;
+      } else {
+        ptot[c % SPB] += padded;
+      }
     }
   }
 
   // the units' padded sizes to the slot's tail, the aggregate to the
-  // ticket's status word
+  // ticket's status word, the planes' words to the buffer's sums
   uint64_t agg = 0;
-  uint32_t pv = 0;
 #pragma unroll
-  for (int j = 0; j < UT; ++j) {
-    agg += padj[j];
-    pv = lane == (uint32_t)j ? padj[j] : pv;
+  for (int k = 0; k < EB; ++k) {
+    agg += ptot[k];
+    if (lane == (uint32_t)k && ptot[k] > 0) atomicAdd(a.ptot + 4ull * b + k, ptot[k]);
   }
-  if (lane < kMaxTicketUnits) ((uint32_t*)(spill + kMaxTicketUnits * CSTAGE))[lane] = pv;
+  if (lane < kMaxTicketUnits) ((gout<uint32_t>)(spill + kMaxTicketUnits * CSTAGE))[lane] = pv;
   publish_agg_gen(a.status, tix, tix - lt, agg, gen, (int)lane);
   return agg;
 }
@@ -557,7 +576,7 @@ __device__ uint64_t encode_ticket32(const BatchBuf& B, uint32_t b, uint32_t lt, 
       const uint32_t un = wave_u32((sb[j] - cb[j]) >> 1);  // unspilled words
       if (un >= H) {
         uint16_t* st = wstage + j * REG;
-        if (lane < H4) ((uint4*)(spill + j * SSTAGE + fl[j]))[lane] = ((const uint4*)st)[lane];
+        if (lane < H4) ((gout<u32x4>)(spill + j * SSTAGE + fl[j]))[lane] = ((const u32x4*)st)[lane];
         if (4u * lane < un - H) ((uint2*)st)[lane] = ((const uint2*)(st + H))[lane];
         fl[j] += H;
         sb[j] = wave_u32(sb[j] - 2u * H);
@@ -648,17 +667,17 @@ __device__ uint64_t encode_ticket32(const BatchBuf& B, uint32_t b, uint32_t lt, 
     uint16_t* st = wstage + j * REG;
     if (lane < pad[j] - cnt[j]) st[rem + lane] = 0;
     const uint32_t nr = pad[j] > fl[j] ? (pad[j] - fl[j]) / 8 : 0u;
-    for (uint32_t k = lane; k < nr; k += 64) ((uint4*)(spill + j * SSTAGE + fl[j]))[k] = ((const uint4*)st)[k];
+    for (uint32_t k = lane; k < nr; k += 64) ((gout<u32x4>)(spill + j * SSTAGE + fl[j]))[k] = ((const u32x4*)st)[k];
   }
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     if (act[c]) {
-      uint8_t* sec = B.out + B.section[kp[c]] + kSectionFixed;
-      ((uint32_t*)sec)[blk[c] * L + lin] = x[c];
+      const gout<uint8_t> sec = (gout<uint8_t>)B.out + B.section[kp[c]] + kSectionFixed;
+      ((gout<uint32_t>)sec)[blk[c] * L + lin] = x[c];
       if (lin == 0) {
         const uint32_t cu = half ? cnt[NC + c] : cnt[c];
         const uint32_t pu = half ? pad[NC + c] : pad[c];
-        ((uint32_t*)(sec + 4ull * L * B.nb + 8ull * blk[c]))[0] = (n[c] << 16) | cu;
+        ((gout<uint32_t>)(sec + 4ull * L * B.nb + 8ull * blk[c]))[0] = (n[c] << 16) | cu;
         atomicAdd(a.ptot + 4ull * b + kp[c], pu);
       }
     }
@@ -714,16 +733,16 @@ __device__ void place_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, uint64_
     const uint64_t u = u0 + lane;
     if (lane < ut && u < U) {
       const uint32_t kp = (uint32_t)(u % P);
-      ((uint32_t*)(B.out + B.section[kp] + kSectionFixed + 4ull * L * B.nb + 8ull * (u / P)))[1] =
+      ((gout<uint32_t>)(B.out + B.section[kp] + kSectionFixed + 4ull * L * B.nb + 8ull * (u / P)))[1] =
           (uint32_t)(excl + 8ull * exq);
     }
   }
   {
-    const uint4* s4 = (const uint4*)slot;
-    uint4* dst = (uint4*)(B.out + B.data_off + 2ull * excl);
+    const gptr<u32x4> s4 = (gptr<u32x4>)slot;
+    const gout<u32x4> dst = (gout<u32x4>)(B.out + B.data_off + 2ull * excl);
     constexpr int CBQ = 8;
     for (uint32_t j0 = 0; j0 < nq; j0 += CBQ * 64) {
-      uint4 q[CBQ];
+      u32x4 q[CBQ];
 #pragma unroll
       for (int u = 0; u < CBQ; ++u) {
         const uint32_t j = j0 + u * 64 + lane;
@@ -744,16 +763,17 @@ __device__ void place_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, uint64_
     const uint64_t total_words = excl + agg;
     const uint64_t size = B.data_off + 2ull * total_words;
     a.sizes[b] = size;
-    ((uint64_t*)B.out)[6] = total_words;  // data_words at byte 48
-    ((uint64_t*)B.out)[7] = size;         // total_size at byte 56
+    ((gout<uint64_t>)B.out)[6] = total_words;  // data_words at byte 48
+    ((gout<uint64_t>)B.out)[7] = size;         // total_size at byte 56
   }
-  publish();
+  // (the ticket's adds to the planes' sums were complete before its words
+  // were read back)
   uint32_t f = 0;
   if (lane == 0) f = atomicAdd(a.fin + b, 1u);
   if (wave_u32(f) + 1 == B.nticks && lane < B.eb) {
     const uint32_t v = atomic_ld32(a.ptot + 4ull * b + lane);
     atomic_st32(a.ptot + 4ull * b + lane, 0u);
-    ((uint32_t*)(B.out + B.section[lane]))[3] = v;
+    ((gout<uint32_t>)(B.out + B.section[lane]))[3] = v;
     if (lane == 0) atomic_st32(a.fin + b, 0u);
   }
 }
@@ -775,11 +795,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
   uint16_t* const spill = a.spill + ((uint64_t)blockIdx.x * NW + wave) * (2ull * batch_slot_words<PB>());
   // this launch's generation (every wavefront reads it before the last one
   // out advances it)
-  const uint32_t gen = wave_u32(lane == 0 ? atomic_ld32(a.queue + 2) : 0u);
-  // the first hist_wgs workgroups count histogram chunks until none is left
-  // (the rest start on tickets, whose buffers become ready as their chunks
-  // are counted)
-  if (blockIdx.x < a.hist_wgs) hist_phase<PB, NW>(a, gen, lds);
+  const uint32_t gen = wave_u32(lane == 0 ? atomic_ld32(a.queue + kQueueGen) : 0u);
+  // every workgroup counts histogram chunks until none is left.  (A quarter of
+  // them, the rest starting on tickets: 920 us on 1024 buffers of 590 MB
+  // against 855.)
+  hist_phase<PB, NW>(a, gen, lds);
   uint64_t tkey = ~0ull;  // tables held in this wave's LDS
   // the ticket coded last if not resolved yet (wave-uniform), in the slot
   // other than `slot`
@@ -844,11 +864,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
   // the next launch (a replayed graph passes the same arguments every time)
   if (lane == 0) {
     const uint32_t total = gridDim.x * NW;
-    if (atomicAdd(a.queue + 1, 1u) + 1 == total) {
+    if (atomicAdd(a.queue + kQueueExit, 1u) + 1 == total) {
       atomic_st32(a.queue, 0u);
-      atomic_st32(a.queue + 1, 0u);
-      atomic_st32(a.queue + 3, 0u);
-      atomic_st32(a.queue + 2, gen % kBatchGenMask + 1u);
+      atomic_st32(a.queue + kQueueExit, 0u);
+      atomic_st32(a.queue + kQueueChunk, 0u);
+      atomic_st32(a.queue + kQueueGen, gen % kBatchGenMask + 1u);
     }
   }
 }
@@ -876,13 +896,8 @@ hipError_t launch_enc_shape(const BatchEncodeArgs& a, int cu, hipStream_t s, uin
       return hipSuccess;
     }
     if (spill_bytes > a.spill_bytes) return hipErrorInvalidValue;
-    // a quarter of the workgroups start on histogram chunks (at least one
-    // when there are any: the tickets wait for them).  (4096 buffers of
-    // 8.5 GB: 9.53 ms with a quarter, 9.65 with half or all of them.)
-    BatchEncodeArgs g = a;
-    g.hist_wgs = a.nhist_items == 0 ? 0u : (uint32_t)(grid > 3 ? grid / 4 : 1);
-    if (a.lanes == 32) hipLaunchKernelGGL((batch_encode_kernel<PB, NW, KB, 32>), dim3((uint32_t)grid), dim3(64 * NW), lds, s, g);
-    else hipLaunchKernelGGL((batch_encode_kernel<PB, NW, KB, 64>), dim3((uint32_t)grid), dim3(64 * NW), lds, s, g);
+    if (a.lanes == 32) hipLaunchKernelGGL((batch_encode_kernel<PB, NW, KB, 32>), dim3((uint32_t)grid), dim3(64 * NW), lds, s, a);
+    else hipLaunchKernelGGL((batch_encode_kernel<PB, NW, KB, 64>), dim3((uint32_t)grid), dim3(64 * NW), lds, s, a);
     return hipGetLastError();
   }
 }
@@ -1447,9 +1462,9 @@ __global__ __launch_bounds__(64 * NW) void batch_decode_kernel(BatchDecodeArgs a
   }
   // the last workgroup out resets the queue for the next launch
   if (threadIdx.x == 0) {
-    if (atomicAdd(a.queue + 1, 1u) + 1 == gridDim.x) {
+    if (atomicAdd(a.queue + kQueueExit, 1u) + 1 == gridDim.x) {
       atomic_st32(a.queue, 0u);
-      atomic_st32(a.queue + 1, 0u);
+      atomic_st32(a.queue + kQueueExit, 0u);
     }
   }
 }

@@ -1114,7 +1114,7 @@ struct mans_batch {
   uint64_t* status = nullptr; // [cap_ticks]
   uint32_t* ptot = nullptr;   // [cap_bufs][4]
   uint32_t* fin = nullptr;    // [cap_bufs]
-  uint32_t* queue = nullptr;  // [4] next item, exited waves, generation, next chunk
+  uint32_t* queue = nullptr;  // kQueue* words
   BatchBuf* h_bufs = nullptr; // pinned staging for asynchronous plans (or null):
                               // descriptors then items, one upload
   const uint2* items_dev = nullptr;  // the plan's items (item_buf, or after the
@@ -1266,10 +1266,11 @@ mans_status batch_alloc(mans_batch* b, uint32_t cap_bufs, uint64_t cap_items, ui
     b->items_dev = b->item_buf;
   }
   HIP_TRY(hipMalloc(&b->ready, nb1 * 4));
-  HIP_TRY(hipMalloc(&b->queue, 16));
+  HIP_TRY(hipMalloc(&b->queue, kQueueWords * 4));
   HIP_TRY(hipMemset(b->ready, 0, nb1 * 4));
-  const uint32_t q0[4] = {0, 0, 1, 0};  // next item, exited waves, first generation, next chunk
-  HIP_TRY(hipMemcpy(b->queue, q0, 16, hipMemcpyHostToDevice));
+  uint32_t q0[kQueueWords] = {};
+  q0[kQueueGen] = 1;  // the first generation
+  HIP_TRY(hipMemcpy(b->queue, q0, sizeof(q0), hipMemcpyHostToDevice));
   if (b->decode) {
     HIP_TRY(hipMalloc(&b->bad, nb1 * 4));
     HIP_TRY(hipMemset(b->bad, 0, nb1 * 4));

@@ -24,6 +24,7 @@
 
 namespace mans {
 
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef int32_t i32x8 __attribute__((ext_vector_type(8)));
 
@@ -126,9 +127,13 @@ __device__ __forceinline__ void count_tiles(const uint4* body, uint32_t t0, uint
   if (t0 >= t1) return;
   const uint32_t lane = threadIdx.x & 63u, m = (lane & 15u) * 0x11111111u;
   auto load = [&](uint4 (&q)[4], uint32_t t) {
-    const uint4* p = body + (uint64_t)t * kTileU4 + lane;
+    // (a global pointer: a batch's comes from memory)
+    const auto* p = (const __attribute__((address_space(1))) u32x4*)body + (uint64_t)t * kTileU4 + lane;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) q[u] = p[64 * u];
+    for (int u = 0; u < 4; ++u) {
+      const u32x4 v = p[64 * u];
+      q[u] = make_uint4(v.x, v.y, v.z, v.w);
+    }
   };
   f32x4 acc[S];
 #pragma unroll

@@ -225,6 +225,11 @@ struct BatchBuf {
   uint32_t frame_hdr[32];        // frame header (data_words / total_size set by the kernel)
 };
 
+// Words of a batch's queue, a cache line each (atomics on one line take turns):
+// [0] the next ticket, exited wavefronts (both left zeroed), the launch
+// generation 1 .. kBatchGenMask (advanced by the last wavefront out), the next
+// histogram chunk (left zeroed).
+constexpr uint32_t kQueueExit = 32, kQueueGen = 64, kQueueChunk = 96, kQueueWords = 128;
 // A queue item: {buffer, kItemTicket | ticket, or histogram chunk}.
 constexpr uint32_t kItemTicket = 1u << 31;
 struct BatchEncodeArgs {
@@ -240,10 +245,7 @@ struct BatchEncodeArgs {
   uint64_t* status;              // [tickets] look-back words tagged with gen
   uint32_t* ptot;                // [nbufs][4] words per plane (left zeroed)
   uint32_t* fin;                 // [nbufs] encode tickets finished (left zeroed)
-  uint32_t* queue;               // [4] next ticket, exited wavefronts (both left
-                                 // zeroed), launch generation 1 .. kBatchGenMask
-                                 // (advanced by the last wavefront out), next
-                                 // histogram chunk (left zeroed)
+  uint32_t* queue;               // kQueue* words
   uint32_t* err;
   uint64_t* sizes;               // [nbufs] frame sizes out
   uint16_t* spill;               // per-wave spill areas
@@ -251,7 +253,6 @@ struct BatchEncodeArgs {
   uint32_t hist_chunk;           // bytes per histogram item (BatchGrain)
   uint32_t rounds;               // rounds per encode ticket (BatchGrain; 64 lanes)
   uint32_t lanes;                // every buffer's frame: 64 or 32 lanes
-  uint32_t hist_wgs;             // workgroups that start on histogram chunks (set at launch)
 };
 // Batched decode: BatchBuf.in is the frame, .out the elements.  A queue item
 // is up to 16 tickets of one buffer (of one plane pair of a uint32 buffer): {buffer,
@@ -263,7 +264,7 @@ struct BatchDecodeArgs {
   const uint2* items;            // [nitems]
   uint32_t nbufs;
   uint32_t nitems;
-  uint32_t* queue;               // [2] next item, exited workgroups (both left zeroed)
+  uint32_t* queue;               // [0] next item, [kQueueExit] exited workgroups (both left zeroed)
   uint32_t* err;
   uint32_t* bad;                 // [nbufs] the error flags of each buffer (zeroed before the launch)
   uint32_t lanes;                // every buffer's frame: 64 or 32 lanes
