@@ -10,13 +10,13 @@
 // 0xFF >> (L % 8)), lanes without elements stay zero (mappingcpuV1.cpp:146);
 // lane l's bytes go to 32 O_g + l M_g with O = exclusive prefix of M.
 //
-// Structure: a wavefront takes 32 groups per ticket, two at a time (one
-// per half-wave).  Pass A writes codes and centers, finds each group's byte
-// length and publishes the ticket's sum; after pass A of the wave's next
-// ticket, the look-back gives the offset and pass B rebuilds the bits (lane
-// bit buffers in LDS, ds_or per element) and writes them at their offsets.
-// O_g is resolved by decoupled look-back over tickets (any number of groups;
-// the reference's fused path is limited to 1024 groups,
+// Structure: a workgroup takes 4 x 32 groups per ticket, a wavefront 32 of
+// them, two at a time (one per half-wave).  Each pair's codes and centers are
+// written, its bits built in registers and put into the wavefront's LDS area,
+// back to back; the workgroup publishes the ticket's byte total, and once its
+// next ticket is mapped the look-back gives the offset and the area is copied
+// out.  O_g is resolved by decoupled look-back over tickets (any number of
+// groups; the reference's fused path is limited to 1024 groups,
 // mappingV15_fused_uint16.cu:851), the whole wave reading 512 predecessors
 // per round trip.  Unmap parses each lane's bytes with clz over 32-bit words.
 #include "adm_device.hpp"
@@ -28,29 +28,37 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
 
+// Sum and maximum over a half-wave (every lane gets it): within rows of 16
+// lanes by DPP, then across the half's two rows.
+template <typename F>
+__device__ __forceinline__ uint32_t half_reduce(uint32_t v, F f) {
+  v = f(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1, 0xf, 0xf, true));   // quad_perm [1,0,3,2]
+  v = f(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4e, 0xf, 0xf, true));   // quad_perm [2,3,0,1]
+  v = f(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true));  // row_half_mirror
+  v = f(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, true));  // row_mirror
+  return f(v, (uint32_t)__shfl_xor(v, 16, 64));
+}
 __device__ __forceinline__ uint32_t half_sum(uint32_t v) {
-#pragma unroll
-  for (int o = 16; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  return half_reduce(v, [](uint32_t x, uint32_t y) { return x + y; });
 }
 __device__ __forceinline__ uint32_t half_max(uint32_t v) {
-#pragma unroll
-  for (int o = 16; o > 0; o >>= 1) {
-    uint32_t u = __shfl_xor(v, o, 64);
-    v = v > u ? v : u;
-  }
-  return v;
+  return half_reduce(v, [](uint32_t x, uint32_t y) { return x > y ? x : y; });
 }
 
-// Group pairs per ticket.  A ticket of 32 groups (16384 elements) keeps the
-// look-back chain short and the ticket counter's traffic low: 2-group
-// tickets (256K per 512 MiB) made the scan, not the data, the bound, and on
-// 512 MiB 16-group tickets took 0.55 ms, 32 0.50 ms, 64 0.53 ms.
+// Group pairs per wavefront and ticket.  One workgroup ticket (65536 elements)
+// is one add on the ticket counter (11 ns each, all on one address) and one
+// look-back entry: a ticket per wavefront cost 185 us in adds alone on
+// 512 MiB.
 constexpr uint32_t kPairs = kAdmTicketGroups / 2;
+constexpr uint32_t kTicketGroups = kWaves * kAdmTicketGroups;
 static_assert(kPairs % 2 == 0, "pairs are mapped two at a time");
-// Lane bit buffers are padded to 9 words so the 64 lanes' words of one
-// index fall in distinct LDS banks.
+// Bytes of a wavefront's area for its 32 groups' bits: 4 for each of the 1024
+// lanes.  Groups that need more are mapped a second time when their offset is
+// known, in the area itself (lane buffers of kLaneWords words, padded to 9 so
+// the lanes' words of one index fall in distinct LDS banks).
+constexpr uint32_t kAreaBytes = 4096;
 constexpr uint32_t kLaneWords = kAdmLaneBytes / 4 + 1;
+static_assert(64 * kLaneWords * 4 <= kAreaBytes, "the lane buffers fit the area");
 
 // The 16 elements of one lane (half-wave = one group): raw_lane loads them
 // (two 16-byte loads for a whole lane, element loads for the last, partial
@@ -108,7 +116,8 @@ __device__ __forceinline__ uint32_t unpack_center(const AdmMapArgs& a, const Lan
   }
   uint32_t lsum = 0;
 #pragma unroll
-  for (int i = 0; i < (int)kAdmChunk; ++i) lsum += (uint32_t)i < r.cnt ? v[i] : 0u;
+  for (int i = 0; i < (int)kAdmChunk; ++i) lsum += FULL || (uint32_t)i < r.cnt ? v[i] : 0u;
+  if constexpr (FULL) return half_sum(lsum) / kAdmGroup;
   const uint32_t gsum = half_sum(lsum), gcnt = half_sum(r.cnt);
   return gcnt ? gsum / gcnt : 0u;  // mappingcpuV1.cpp:60-66
 }
@@ -140,61 +149,84 @@ __device__ __forceinline__ uint32_t map_lane(const uint32_t (&v)[kAdmChunk], uin
   return bo;
 }
 
-// A wavefront resolves a ticket's offset only after pass A of its next
-// ticket (the byte lengths of two tickets in LDS, used in turn): by then the
-// predecessors have had a whole pass A to publish their lengths, so the
-// look-back sums published entries instead of waiting for the slowest wave
-// still in pass A.  A wave waits only on lower tickets, each of which
-// publishes its aggregate right after its pass A, so the launch drains.
+// map_lane for a whole lane whose bits fit 64: the same codes, and the bits
+// in `word` (first bit on top).  With q = len - 1 = (max(d, 1) - 1) / 126 (the
+// high word of a 24-bit product: exact for 16 bits) an element's string is a one and q zeros,
+// and its code 2 (d - 126 q) + 1, less one if x > c.  Each half of the
+// elements collects its bits in a 32-bit word; false if one does not fit.
+__device__ __forceinline__ bool map_lane_word(const uint32_t (&v)[kAdmChunk], uint32_t c, uint32_t (&codes)[4],
+                                              uint64_t& word, uint32_t& bo) {
+  uint32_t acc[2] = {0, 0}, len[2] = {8, 8};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) codes[i] = 0;
+#pragma unroll
+  for (int i = 0; i < (int)kAdmChunk; ++i) {
+    const int32_t e = (int32_t)c - (int32_t)v[i];
+    const uint32_t d = (uint32_t)(e < 0 ? -e : e);
+    const uint32_t y = ((d > 1u ? d : 1u) << 8) - 256u;
+    const uint32_t q = (uint32_t)(((uint64_t)(y & 0xffffffu) * 133153u) >> 32);
+    const uint32_t code = 2u * (d - __umul24(kAdmMod, q)) + (uint32_t)(e >> 31);
+    codes[i >> 2] |= code << (8 * (i & 3));
+    acc[i >> 3] = ((acc[i >> 3] << 1) | 1u) << (q & 31u);
+    len[i >> 3] += q;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) codes[i] += 0x01010101u;
+  bo = len[0] + len[1];
+  if (len[0] > 32u || len[1] > 32u) return false;
+  word = ((uint64_t)acc[0] << (64u - len[0])) | ((uint64_t)acc[1] << (64u - bo));
+  return true;
+}
+
+// A ticket's offset is resolved only after the workgroup's next ticket is
+// mapped (two areas, used in turn): by then the predecessors have had a whole
+// ticket's time to publish their totals, so the look-back sums published
+// entries instead of waiting for the slowest.  A workgroup waits only on lower
+// tickets, each of which publishes its total right after its mapping, so the
+// launch drains.
+// Bound by vector instructions (about 15 per element) and, from there, memory
+// traffic (input, codes and bits once): 512 MiB 285 us; with a second
+// pass over the input that built the bits by one LDS atomic per element, and
+// a ticket per wavefront, 460.
 __global__ __launch_bounds__(kThreads) void adm_map_kernel(AdmMapArgs a) {
-  __shared__ uint32_t s_bits[kWaves][64][kLaneWords];
-  __shared__ uint32_t s_m[kWaves][2][2 * kPairs];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  __shared__ uint4 s_area[2][kWaves][kAreaBytes / 16];
+  __shared__ uint32_t s_sum[2][kWaves], s_next[2];
+  const int t = threadIdx.x, lane = t & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane((uint32_t)t >> 6);
   const uint32_t half = (uint32_t)lane >> 5, lin = (uint32_t)lane & 31u;
-  uint32_t* mybits = s_bits[wave][lane];
-  const uint8_t* wavebytes = (const uint8_t*)s_bits[wave];
-  constexpr uint32_t kTicketGroups = 2 * kPairs;
 
-  // the ticket whose pass A is done and whose offset is not yet resolved
-  // (wave-uniform), its byte lengths in s_m[wave][slot ^ 1]; lane g < 16:
-  // group g's exclusive byte offset within it
-  bool pend = false;
-  uint32_t p_tk = 0, p_exlo = 0, slot = 0;
-  uint64_t p_agg = 0;
+  // the ticket mapped but not resolved (workgroup-uniform): its first group,
+  // byte total (in units of 32 bytes, as all offsets here); of this
+  // wavefront's groups the offset in the ticket, the total, whether they are
+  // in the area, and in lane g < 32 group g's offset
+  bool pend = false, p_kept = false;
+  uint32_t p_tk = 0, p_agg = 0, p_off = 0, p_sum = 0, p_exlo = 0;
 
-  // offsets and pass B of the pending ticket: each pair's bit plane, lane
-  // l's m bytes at 32 og + l m
-  auto finish_pending = [&]() {
-    const uint32_t* wm = s_m[wave][slot ^ 1u];
-    const uint64_t chain = p_tk / kTicketGroups;
-    uint64_t excl = resolve_prefix(a.status, chain, p_agg, lane);
-    excl = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(excl >> 32)) << 32) |
-           (uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)excl);
-    {
-      const uint64_t g = (uint64_t)p_tk + lane;
-      if ((uint32_t)lane < kTicketGroups && g < a.gsize) a.offsets[g] = (int32_t)(excl + p_exlo);
-    }
-    if ((uint64_t)p_tk + kTicketGroups >= a.gsize && lane == 0) a.offsets[a.gsize] = (int32_t)(excl + p_agg);
-    auto pair_b = [&](uint32_t pr, const LaneRaw& cur, auto full) {
-      constexpr bool FULL = decltype(full)::value;
-      const uint64_t g = (uint64_t)p_tk + 2 * pr + half;
+  // Groups that did not fit the area: mapped again from the input, pair by
+  // pair, with the lanes' bits in the area's lane buffers.
+  auto direct = [&](uint32_t* area, uint64_t excl, uint64_t g0) {
+    uint32_t* const mybits = area + lane * kLaneWords;
+    const uint8_t* const wavebytes = (const uint8_t*)area;
+    for (uint32_t pr = 0; pr < kPairs; ++pr) {
+      const uint64_t g = g0 + 2 * pr + half;
+      const LaneRaw cur = raw_lane<false>(a, g, lin);
       uint32_t v[kAdmChunk], codes[4];
       const uint32_t cnt = cur.cnt;
-      const uint32_t c = unpack_center<FULL>(a, cur, v);
+      const uint32_t c = unpack_center<false>(a, cur, v);
 #pragma unroll
       for (int i = 0; i < (int)kLaneWords; ++i) mybits[i] = 0;
       __threadfence_block();
       const uint32_t bo = map_lane<true>(v, cnt, c, codes, mybits);
-      const uint32_t m = wm[2 * pr + half];
+      const uint32_t ex0 = __shfl(p_exlo, (int)(2 * pr), 64), ex1 = __shfl(p_exlo, (int)(2 * pr + 1), 64);
+      const uint32_t ex2 = pr + 1 < kPairs ? __shfl(p_exlo, (int)((2 * pr + 2) & 63u), 64) : p_sum;
+      const uint32_t m = half ? ex2 - ex1 : ex1 - ex0;
       if (cnt && bo < 8u * m) {
         const uint32_t pad = (bo & 7u) == 0 ? 0xffu : (0xffu >> (bo & 7u));
         atomicOr(mybits + (bo >> 5), pad << (((bo >> 3) & 3u) * 8u));
       }
       __threadfence_block();
-      const uint32_t og_lo = __shfl(p_exlo, (int)(2 * pr), 64), og_hi = __shfl(p_exlo, (int)(2 * pr + 1), 64);
-      const uint64_t og = excl + (half ? og_hi : og_lo);
       if (g < a.gsize && m > 0) {
-        const uint64_t dst0 = 32ull * og;
+        const uint64_t dst0 = 32ull * (excl + (half ? ex1 : ex0));
         const uint32_t total = 32u * m;
         const uint32_t inv = (65536u + m - 1u) / m;
         const uint64_t valid_lanes = a.n > g * kAdmGroup ? div_up(a.n - g * kAdmGroup, kAdmChunk) : 0;
@@ -209,87 +241,142 @@ __global__ __launch_bounds__(kThreads) void adm_map_kernel(AdmMapArgs a) {
         }
       }
       __threadfence_block();
-    };
-    // two buffers used in turn (no register copy between them, so the next
-    // pair's loads stay in flight while a pair is mapped)
-    auto pass_b = [&](auto full) {
-      constexpr bool FULL = decltype(full)::value;
-      LaneRaw ra = raw_lane<FULL>(a, (uint64_t)p_tk + half, lin), rb;
-      for (uint32_t pr = 0; pr < kPairs; pr += 2) {
-        rb = raw_lane<FULL>(a, (uint64_t)p_tk + 2 * (pr + 1) + half, lin);
-        pair_b(pr, ra, full);
-        if (pr + 2 < kPairs) ra = raw_lane<FULL>(a, (uint64_t)p_tk + 2 * (pr + 2) + half, lin);
-        pair_b(pr + 1, rb, full);
-      }
-    };
-    if ((uint64_t)(p_tk + kTicketGroups) * kAdmGroup <= a.n) pass_b(std::true_type{});
-    else pass_b(std::false_type{});
+    }
   };
 
-  for (;;) {
-    uint32_t tk = 0;
-    if (lane == 0) tk = atomicAdd(a.ticket, kTicketGroups);
-    tk = __builtin_amdgcn_readfirstlane(tk);
+  // the pending ticket's offsets and bits
+  auto finish_pending = [&](uint32_t slot) {
+    // (every wavefront resolves; all write the same prefix)
+    uint64_t excl = resolve_prefix(a.status, p_tk / kTicketGroups, p_agg, lane);
+    excl = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(excl >> 32)) << 32) |
+           (uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)excl);
+    if ((uint64_t)p_tk + kTicketGroups >= a.gsize && t == 0) a.offsets[a.gsize] = (int32_t)(excl + p_agg);
+    excl += p_off;
+    const uint64_t g0 = (uint64_t)p_tk + wave * kAdmTicketGroups;
+    if ((uint32_t)lane < kAdmTicketGroups && g0 + lane < a.gsize) a.offsets[g0 + lane] = (int32_t)(excl + p_exlo);
+    if (p_kept && 32ull * (excl + p_sum) <= a.bits_capacity) {
+      uint8_t* const dst = a.bits + 32ull * excl;
+      if (((uintptr_t)a.bits & 15u) == 0) {
+        const uint4* const src = s_area[slot][wave];
+        for (uint32_t q = (uint32_t)lane; q < 2u * p_sum; q += 64u) ((uint4*)dst)[q] = src[q];
+      } else {
+        const uint8_t* const src = (const uint8_t*)s_area[slot][wave];
+        for (uint32_t q = (uint32_t)lane; q < 32u * p_sum; q += 64u) dst[q] = src[q];
+      }
+      __threadfence_block();  // (the area is written again)
+    } else if (p_sum > 0) {
+      direct((uint32_t*)s_area[slot][wave], excl, g0);
+    }
+  };
+
+  if (t == 0) s_next[0] = atomicAdd(a.ticket, kTicketGroups);
+  __syncthreads();
+  for (uint32_t k = 0;; ++k) {
+    const uint32_t slot = k & 1u;
+    const uint32_t tk = __builtin_amdgcn_readfirstlane(s_next[slot]);
     const bool more = (uint64_t)tk < a.gsize;
-    uint32_t exlo = 0;
-    uint64_t agg = 0;
+    uint32_t ex = 0, exlo = 0;
+    bool kept = true;
     if (more) {
-      // ---- pass A: codes, centers and each group's byte length M_g -------
-      uint32_t* wm = s_m[wave][slot];
+      const uint64_t g0 = (uint64_t)tk + wave * kAdmTicketGroups;
+      uint8_t* const area = (uint8_t*)s_area[slot][wave];
       bool over = false;
-      auto pair_a = [&](uint32_t pr, const LaneRaw& cur, auto full) {
+      auto pair = [&](uint32_t pr, const LaneRaw& cur, auto full) {
         constexpr bool FULL = decltype(full)::value;
-        const uint64_t g = (uint64_t)tk + 2 * pr + half;
+        const uint64_t g = g0 + 2 * pr + half;
         uint32_t v[kAdmChunk], codes[4];
         const uint32_t cnt = cur.cnt;
-        const uint64_t base = cur.base;
         const uint32_t c = unpack_center<FULL>(a, cur, v);
-        const uint32_t bo = map_lane<false>(v, cnt, c, codes, nullptr);
+        uint64_t word = 0;
+        uint32_t bo;
+        bool narrow = false;
+        if constexpr (FULL) narrow = __ballot(!map_lane_word(v, c, codes, word, bo)) == 0;
+        else bo = map_lane<false>(v, cnt, c, codes, nullptr);
         if (bo > 8 * kAdmLaneBytes) over = true;
         uint32_t m = half_max(cnt ? (bo + 7u) / 8u : 0u);
         if (m > kAdmLaneBytes) m = kAdmLaneBytes;
         if (cnt == kAdmChunk) {
-          *(uint4*)(a.codes + base) = make_uint4(codes[0], codes[1], codes[2], codes[3]);
+          *(uint4*)(a.codes + cur.base) = make_uint4(codes[0], codes[1], codes[2], codes[3]);
         } else {
-          for (uint32_t i = 0; i < cnt; ++i) a.codes[base + i] = (uint8_t)(codes[i >> 2] >> (8 * (i & 3)));
+          for (uint32_t i = 0; i < cnt; ++i) a.codes[cur.base + i] = (uint8_t)(codes[i >> 2] >> (8 * (i & 3)));
         }
         if (g < a.gsize && lin == 0) a.centers[g] = (uint16_t)c;
-        if (lin == 0) wm[2 * pr + half] = m;
+        const uint32_t m0 = __builtin_amdgcn_readlane(m, 0), m1 = __builtin_amdgcn_readlane(m, 32);
+        const uint32_t at = 32u * (ex + (half ? m0 : 0u)) + lin * m;  // this lane's bytes in the area
+        if (32u * (ex + m0 + m1) > kAreaBytes) {
+          kept = false;
+        } else if (kept && narrow) {
+          // the byte that holds bit bo, if the lane has one: ones from there
+          if (bo < 8u * m) word |= ((1ull << (8u - (bo & 7u))) - 1u) << (63u - (bo | 7u));
+          word = __builtin_bswap64(word);
+          const uint32_t mm = m0 > m1 ? m0 : m1;
+          for (uint32_t j = 0; j < mm; ++j) {
+            if (j < m) area[at + j] = (uint8_t)word;
+            word >>= 8;
+          }
+        } else if (kept) {
+          for (uint32_t i = (uint32_t)lane; i < 8u * (m0 + m1); i += 64u) ((uint32_t*)area)[8u * ex + i] = 0;
+          __threadfence_block();
+          uint32_t p = 0;  // bit of the lane, `at` bytes into the area
+          auto set = [&](uint32_t bit, uint32_t byte_bits) {
+            const uint32_t y = at + (bit >> 3);
+            atomicOr((uint32_t*)area + (y >> 2), byte_bits << (8u * (y & 3u)));
+          };
+#pragma unroll
+          for (int i = 0; i < (int)kAdmChunk; ++i) {
+            const bool ok = (uint32_t)i < cnt;
+            const uint32_t d = v[i] > c ? v[i] - c : c - v[i];
+            if (ok && p < 8u * m) set(p, 128u >> (p & 7u));
+            p += ok ? (d == 0 ? 1u : (d + kAdmMod - 1) / kAdmMod) : 0u;
+          }
+          if (cnt && p < 8u * m) set(p, 0xffu >> (p & 7u));
+        }
+        exlo = (uint32_t)lane == 2 * pr ? ex : exlo;
+        exlo = (uint32_t)lane == 2 * pr + 1 ? ex + m0 : exlo;
+        ex += m0 + m1;
       };
-      auto pass_a = [&](auto full) {
+      // two buffers used in turn (no register copy between them, so the next
+      // pair's loads stay in flight while a pair is mapped)
+      auto pass = [&](auto full) {
         constexpr bool FULL = decltype(full)::value;
-        LaneRaw ra = raw_lane<FULL>(a, (uint64_t)tk + half, lin), rb;
+        LaneRaw ra = raw_lane<FULL>(a, g0 + half, lin), rb;
         for (uint32_t pr = 0; pr < kPairs; pr += 2) {
-          rb = raw_lane<FULL>(a, (uint64_t)tk + 2 * (pr + 1) + half, lin);
-          pair_a(pr, ra, full);
-          if (pr + 2 < kPairs) ra = raw_lane<FULL>(a, (uint64_t)tk + 2 * (pr + 2) + half, lin);
-          pair_a(pr + 1, rb, full);
+          rb = raw_lane<FULL>(a, g0 + 2 * (pr + 1) + half, lin);
+          pair(pr, ra, full);
+          if (pr + 2 < kPairs) ra = raw_lane<FULL>(a, g0 + 2 * (pr + 2) + half, lin);
+          pair(pr + 1, rb, full);
         }
       };
-      // (tickets before the input's end: whole lanes only)
-      if ((uint64_t)(tk + kTicketGroups) * kAdmGroup <= a.n) pass_a(std::true_type{});
-      else pass_a(std::false_type{});
+      // (before the input's end: whole lanes only)
+      if ((g0 + kAdmTicketGroups) * kAdmGroup <= a.n) pass(std::true_type{});
+      else pass(std::false_type{});
       if (__ballot(over) && lane == 0) atomicOr(a.err, kErrAdmDomain);
-      __threadfence_block();
-      // the ticket's groups: exclusive byte offsets within it, and their sum
-      const uint32_t mine = (uint32_t)lane < kTicketGroups ? wm[lane] : 0u;
-      uint32_t incl = mine;
-#pragma unroll
-      for (int o = 1; o < (int)kTicketGroups; o <<= 1) {
-        const uint32_t u = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += u;
-      }
-      agg = __builtin_amdgcn_readlane(incl, kTicketGroups - 1);
-      exlo = incl - mine;
-      publish_aggregate(a.status, tk / kTicketGroups, agg, lane);
+      if (lane == 0) s_sum[slot][wave] = ex;
+      // (not earlier: a ticket held long before it is mapped keeps those
+      // after it waiting)
+      if (t == 0) s_next[slot ^ 1u] = atomicAdd(a.ticket, kTicketGroups);
     }
-    if (pend) finish_pending();
+    __threadfence_block();
+    __syncthreads();
+    uint32_t agg = 0, off = 0;
+    if (more) {
+#pragma unroll
+      for (uint32_t w = 0; w < (uint32_t)kWaves; ++w) {
+        const uint32_t v = __builtin_amdgcn_readfirstlane(s_sum[slot][w]);
+        off += w < wave ? v : 0u;
+        agg += v;
+      }
+      if (wave == 0) publish_aggregate(a.status, tk / kTicketGroups, agg, lane);
+    }
+    if (pend) finish_pending(slot ^ 1u);
     if (!more) break;
     pend = true;
     p_tk = tk;
-    p_exlo = exlo;
     p_agg = agg;
-    slot ^= 1u;
+    p_off = off;
+    p_sum = ex;
+    p_exlo = exlo;
+    p_kept = kept;
   }
 }
 
@@ -322,7 +409,7 @@ hipError_t launch_adm_map(const AdmMapArgs& a, int cu, hipStream_t s) {
   hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, adm_map_kernel, kThreads, 0);
   if (e != hipSuccess) return e;
   if (per_cu < 1) per_cu = 1;
-  uint64_t grid = div_up(div_up(a.gsize, kAdmTicketGroups), kWaves);
+  uint64_t grid = div_up(a.gsize, kTicketGroups);
   const uint64_t cap = (uint64_t)cu * per_cu;
   if (grid > cap) grid = cap;
   hipLaunchKernelGGL(adm_map_kernel, dim3((uint32_t)grid), dim3(kThreads), 0, s, a);
