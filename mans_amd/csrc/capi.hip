@@ -808,7 +808,17 @@ mans_status mans_lorenzo_reconstruct(const uint16_t* d_codes, const uint32_t* d_
   DeviceGuard g(ws->device);
   hipStream_t s = (hipStream_t)stream;
   note_capture(ws, s);
-  mans_status st = ensure_scratch(ws, 4 * n);
+  // By tiles the outliers wait in the out array, which is written while the
+  // codes are read: only where it shares no byte with them or the outlier
+  // lists.
+  auto apart = [&](const void* p, uint64_t bytes) {
+    const uintptr_t f = (uintptr_t)d_field, b = (uintptr_t)p;
+    return b + bytes <= f || f + 4 * n <= b;
+  };
+  const LorenzoScratch l = lorenzo_inverse_scratch(nz, ny, nx, ws->cu);
+  const bool tiles = l.fits && apart(d_codes, 2 * n) && apart(d_outlier_idx, outlier_count * 4) &&
+                     apart(d_outlier_val, outlier_count * 4);
+  mans_status st = ensure_scratch(ws, tiles ? 4 * l.words : 4 * n);
   if (st != MANS_OK) return st;
   LorenzoArgs a;
   memset(&a, 0, sizeof(a));
@@ -820,8 +830,14 @@ mans_status mans_lorenzo_reconstruct(const uint16_t* d_codes, const uint32_t* d_
   a.in_idx = d_outlier_idx;
   a.in_val = d_outlier_val;
   a.n_out = outlier_count;
-  a.q = (int32_t*)ws->scratch;
+  a.q = tiles ? (int32_t*)d_field : (int32_t*)ws->scratch;
   a.recon = d_field;
+  if (tiles) {
+    a.slab = (int32_t*)ws->scratch;
+    a.band = a.slab + l.band;
+    a.corner = a.slab + l.corner;
+    a.ty = l.ty;
+  }
   a.err = ws->counters + 3;
   prof_mark(ws, s, "lorenzo_inverse");
   HIP_TRY(launch_lorenzo_inverse(a, ws->cu, s));

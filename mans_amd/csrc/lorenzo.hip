@@ -251,9 +251,17 @@ __global__ __launch_bounds__(kTX * kFixGroups) void lorenzo_fixup_kernel(Lorenzo
 }
 
 // ---- inverse ---------------------------------------------------------------
-// q of outliers first (scattered), then per plane: x-prefix of each row plus
-// the y-prefix (running per column), then per column: the z-prefix and
-// f' = q * 2 eb.
+// The outliers' residuals are scattered first.  Then either
+//  * by tiles of `ty` rows x TZ planes x whole rows of x: the sums of the
+//    residuals r over each tile's planes (per row), its rows (per plane) and
+//    both; their prefixes over the tiles; then each tile from those, the
+//    x-prefix last.  All sums are of 32-bit integers, so their order does not
+//    matter.  The codes are read twice, the field is written once and the
+//    sums are a tenth of it; or
+//  * (buffers that overlap) per plane the x-prefix of each row plus the
+//    y-prefix (running per column), then per column the z-prefix and
+//    f' = q * 2 eb, with every q through memory.
+// 500 x 499 x 900: by tiles 515 us, through q 820.
 __global__ void lorenzo_scatter_kernel(LorenzoArgs a) {
   for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < a.n_out; k += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t i = a.in_idx[k];
@@ -398,6 +406,258 @@ __global__ __launch_bounds__(256) void lorenzo_column_kernel(LorenzoArgs a) {
   }
 }
 
+// The codes of planes z0 .. z0 + TZ - 1 at (y, x), and the residuals they
+// stand for (FULL: every plane is in the field; else 0 past its end).
+template <uint32_t TZ, bool FULL>
+__device__ __forceinline__ void load_codes(const LorenzoArgs& a, uint32_t z0, uint32_t y, uint32_t x,
+                                           uint32_t (&code)[TZ]) {
+  const uint64_t plane = (uint64_t)a.ny * a.nx;
+  const uint16_t* p = a.codes + z0 * plane + (uint64_t)y * a.nx + x;
+#pragma unroll
+  for (uint32_t k = 0; k < TZ; ++k) code[k] = FULL || z0 + k < a.nz ? p[k * plane] : 32768u;
+}
+template <uint32_t TZ>
+__device__ __forceinline__ void residuals(const LorenzoArgs& a, uint32_t z0, uint32_t y, uint32_t x,
+                                          const uint32_t (&code)[TZ], int32_t (&r)[TZ]) {
+  const uint64_t plane = (uint64_t)a.ny * a.nx;
+  const int32_t* q = a.q + z0 * plane + (uint64_t)y * a.nx + x;
+#pragma unroll
+  for (uint32_t k = 0; k < TZ; ++k) {
+    r[k] = (int32_t)code[k] - 32768;
+    if (code[k] == 0) r[k] = q[k * plane];
+  }
+}
+
+// A tile's sums: over its planes for each row (slab), over its rows for each
+// plane (band), over both (corner[0 .. ]).  A thread per x, the next row's
+// codes loaded ahead; the last slab's and the last band's are not needed.
+// Memory bound: 154 us for 500 x 499 x 900.  (Workgroups of 256 columns, which
+// share lines of a row across XCDs: 167.)
+template <uint32_t TZ>
+__global__ __launch_bounds__(1024) void lorenzo_sums_kernel(LorenzoArgs a) {
+  const uint32_t nxc = (uint32_t)div_up(a.nx, 1024), nyt = gridDim.x / nxc, nzt = gridDim.y;
+  const uint32_t yt = blockIdx.x / nxc, zt = blockIdx.y;
+  const uint32_t y0 = yt * a.ty, y1 = a.ny - y0 < a.ty ? a.ny : y0 + a.ty, z0 = zt * TZ;
+  auto columns = [&](uint32_t x, auto full) {
+    constexpr bool FULL = decltype(full)::value;
+    int32_t v[TZ];
+#pragma unroll
+    for (uint32_t k = 0; k < TZ; ++k) v[k] = 0;
+    uint32_t code[TZ];
+    load_codes<TZ, FULL>(a, z0, y0, x, code);
+    for (uint32_t y = y0; y < y1; ++y) {
+      uint32_t next[TZ];
+      load_codes<TZ, FULL>(a, z0, y + 1 < y1 ? y + 1 : y, x, next);
+      int32_t r[TZ], s = 0;
+      residuals<TZ>(a, z0, y, x, code, r);
+#pragma unroll
+      for (uint32_t k = 0; k < TZ; ++k) {
+        v[k] += r[k];
+        s += r[k];
+        code[k] = next[k];
+      }
+      if (zt + 1 < nzt) a.slab[((uint64_t)zt * a.ny + y) * a.nx + x] = s;
+    }
+    int32_t all = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < TZ; ++k) {
+      all += v[k];
+      if (yt + 1 < nyt && (FULL || z0 + k < a.nz)) a.band[((uint64_t)yt * a.nz + z0 + k) * a.nx + x] = v[k];
+    }
+    a.corner[((uint64_t)zt * nyt + yt) * a.nx + x] = all;
+  };
+  const uint32_t x = blockIdx.x % nxc * 1024u + threadIdx.x;
+  if (x >= a.nx) return;
+  if (z0 + TZ <= a.nz) columns(x, std::true_type{});
+  else columns(x, std::false_type{});
+}
+
+// Prefixes over the tiles, a thread a column: of slab over the slabs and of
+// band over the bands (inclusive, in place), of corner over both (exclusive,
+// into corner[nzt nyt nx ..]).
+__global__ __launch_bounds__(256) void lorenzo_prefix_kernel(LorenzoArgs a, uint32_t nzt, uint32_t nyt) {
+  constexpr uint32_t B = 16;  // entries loaded before any is summed
+  const uint64_t per_slab = (uint64_t)a.ny * a.nx, per_band = (uint64_t)a.nz * a.nx, per_row = (uint64_t)nyt * a.nx;
+  auto scan = [&](int32_t* p, uint64_t step, uint32_t n) {
+    int32_t s = 0;
+    for (uint32_t k0 = 0; k0 < n; k0 += B) {
+      int32_t v[B];
+#pragma unroll
+      for (uint32_t k = 0; k < B; ++k) v[k] = k0 + k < n ? p[(k0 + k) * step] : 0;
+#pragma unroll
+      for (uint32_t k = 0; k < B; ++k) {
+        s += v[k];
+        if (k0 + k < n) p[(k0 + k) * step] = s;
+      }
+    }
+  };
+  // (the corners first: each takes up to nzt nyt reads)
+  const uint64_t nc = per_row, ns = nzt > 1 ? per_slab : 0, nb = nyt > 1 ? per_band : 0;
+  for (uint64_t j = (uint64_t)blockIdx.x * 256 + threadIdx.x; j < nc + ns + nb; j += (uint64_t)gridDim.x * 256) {
+    if (j < nc) {
+      const uint32_t yt = (uint32_t)(j / a.nx), x = (uint32_t)(j % a.nx);
+      int32_t run = 0;
+      for (uint32_t zt = 0; zt < nzt; ++zt) {
+        a.corner[(nzt + (uint64_t)zt) * per_row + j] = run;
+        const int32_t* p = a.corner + zt * per_row + x;
+        for (uint32_t k0 = 0; k0 < yt; k0 += B) {
+#pragma unroll
+          for (uint32_t k = 0; k < B; ++k) run += k0 + k < yt ? p[(uint64_t)(k0 + k) * a.nx] : 0;
+        }
+      }
+    } else if (j < nc + ns) {
+      scan(a.slab + (j - nc), per_slab, nzt - 1);
+    } else {
+      scan(a.band + (j - nc - ns), per_band, nyt - 1);
+    }
+  }
+}
+
+// Inclusive sum over the 64 lanes.
+__device__ __forceinline__ int32_t wave_scan(int32_t v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return v;
+}
+// Sum over each row of 16 lanes (every lane gets it).
+__device__ __forceinline__ int32_t row_sum(int32_t v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, true);   // quad_perm [1,0,3,2]
+  v += __builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, true);   // quad_perm [2,3,0,1]
+  v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true);  // row_half_mirror
+  v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true);  // row_mirror
+  return v;
+}
+
+// A tile of the field.  A thread keeps, for its x of each 1024-column chunk
+// and each of the tile's planes, the sum w of r over the planes and rows up
+// to here; a row adds its r, summed over the planes so far, and its x-prefix
+// is the row of q.  One barrier a row and chunk; the next row's codes are
+// loaded before it and their outliers after it.  Threads past the end of a
+// row repeat its last column: nothing reads their sums.  Memory bound: 307 us
+// for 500 x 499 x 900 (1.43 GB, 4.7 TB/s; with every load waited for in its
+// own row 413).
+template <uint32_t C, uint32_t TZ, bool FULL>
+__device__ __forceinline__ void write_tile(const LorenzoArgs& a, int32_t (&s_w)[2][TZ][16]) {
+  static_assert(TZ % 4 == 0, "four planes a row sum");
+  const uint32_t yt = blockIdx.x, zt = blockIdx.y, nyt = gridDim.x, nzt = gridDim.y;
+  const uint32_t y0 = yt * a.ty, y1 = a.ny - y0 < a.ty ? a.ny : y0 + a.ty, z0 = zt * TZ;
+  const uint32_t t = threadIdx.x, lane = t & 63u, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const uint64_t plane = (uint64_t)a.ny * a.nx;
+  auto column = [&](uint32_t c) {
+    const uint32_t x = c * 1024u + t;
+    return x < a.nx ? x : a.nx - 1u;
+  };
+  int32_t cz[C][TZ];
+#pragma unroll
+  for (uint32_t c = 0; c < C; ++c) {
+    const uint32_t x = column(c);
+    int32_t run = a.corner[((uint64_t)(nzt + zt) * nyt + yt) * a.nx + x];
+#pragma unroll
+    for (uint32_t k = 0; k < TZ; ++k) {
+      if (yt > 0 && (FULL || z0 + k < a.nz)) run += a.band[((uint64_t)(yt - 1) * a.nz + z0 + k) * a.nx + x];
+      cz[c][k] = run;
+    }
+  }
+  uint32_t code[TZ];
+  int32_t r[TZ], u = 0;
+  auto load = [&](uint32_t y, uint32_t c) {
+    load_codes<TZ, FULL>(a, z0, y, column(c), code);
+    if (zt > 0) u = a.slab[((uint64_t)(zt - 1) * a.ny + y) * a.nx + column(c)];
+  };
+  load(y0, 0);
+  residuals<TZ>(a, z0, y0, column(0), code, r);
+  uint32_t buf = 0;
+  for (uint32_t y = y0; y < y1; ++y) {
+    int32_t carry[TZ];
+#pragma unroll
+    for (uint32_t k = 0; k < TZ; ++k) carry[k] = 0;
+#pragma unroll
+    for (uint32_t c = 0; c < C; ++c) {
+      const uint32_t x = c * 1024u + t;
+      int32_t inc[TZ], s = u;
+#pragma unroll
+      for (uint32_t k = 0; k < TZ; ++k) {
+        s += r[k];
+        cz[c][k] += s;
+        inc[k] = wave_scan(cz[c][k]);
+      }
+      if (lane == 63) {
+#pragma unroll
+        for (uint32_t k = 0; k < TZ; ++k) s_w[buf][k][w] = inc[k];
+      }
+      // (the last row is loaded again after itself)
+      const uint32_t cn = c + 1 < C ? c + 1 : 0u, yn = c + 1 < C || y + 1 == y1 ? y : y + 1;
+      load(yn, cn);
+      __syncthreads();
+      float* const out = a.recon + z0 * plane + (uint64_t)y * a.nx + x;
+#pragma unroll
+      for (uint32_t k0 = 0; k0 < TZ; k0 += 4) {
+        // lane 16 p + v: wavefront v's total of plane k0 + p
+        const int32_t v = s_w[buf][k0 + (lane >> 4)][lane & 15u];
+        const int32_t before = row_sum((lane & 15u) < w ? v : 0);
+        const int32_t all = C > 1 ? row_sum(v) : 0;
+#pragma unroll
+        for (uint32_t p = 0; p < 4; ++p) {
+          const uint32_t k = k0 + p;
+          inc[k] += carry[k] + __builtin_amdgcn_readlane(before, 16 * p);
+          if (C > 1) carry[k] += __builtin_amdgcn_readlane(all, 16 * p);
+        }
+      }
+      // the next row's outliers, before this row is written: the threads past
+      // the end of the row read their last column's from where its own thread
+      // may be writing (and use none of them)
+      residuals<TZ>(a, z0, yn, column(cn), code, r);
+      if (x < a.nx) {
+#pragma unroll
+        for (uint32_t k = 0; k < TZ; ++k)
+          if (FULL || z0 + k < a.nz) out[k * plane] = (float)inc[k] * a.twoeb;
+      }
+      buf ^= 1u;
+    }
+  }
+}
+
+template <uint32_t C, uint32_t TZ>
+__global__ __launch_bounds__(1024) void lorenzo_tile_kernel(LorenzoArgs a) {
+  __shared__ int32_t s_w[2][TZ][16];  // the wavefronts' row totals
+  for (uint32_t i = threadIdx.x; i < 2 * TZ * 16; i += blockDim.x) ((int32_t*)s_w)[i] = 0;
+  __syncthreads();
+  if ((blockIdx.y + 1) * TZ <= a.nz) write_tile<C, TZ, true>(a, s_w);
+  else write_tile<C, TZ, false>(a, s_w);
+}
+
+// Planes of a tile: as many as a thread's sums of all its columns fit in
+// registers.  Rows: 32, fewer (not under 2, nor so few that a column has more
+// than 256 tiles: the prefixes take time for each) while the tiles would not
+// give every compute unit two workgroups.
+uint32_t tile_planes(uint32_t nx) { return nx <= 1024 ? 16u : (nx <= 2048 ? 8u : 4u); }
+uint32_t tile_rows(uint32_t nz, uint32_t ny, uint32_t nx, int cu) {
+  uint32_t ty = 32;
+  while (ty > 2 && div_up(ny, ty / 2) <= 256 && div_up(nz, tile_planes(nx)) * div_up(ny, ty) < 2ull * (uint64_t)cu)
+    ty /= 2;
+  return ty;
+}
+
+template <uint32_t C, uint32_t TZ>
+hipError_t launch_tiles(const LorenzoArgs& a, int cu, hipStream_t s) {
+  const uint32_t nyt = (uint32_t)div_up(a.ny, a.ty), nzt = (uint32_t)div_up(a.nz, TZ);
+  const uint32_t threads = a.nx > 1024 ? 1024u : (uint32_t)round_up(a.nx, 64);
+  hipLaunchKernelGGL(lorenzo_sums_kernel<TZ>, dim3(nyt * (uint32_t)div_up(a.nx, 1024), nzt), dim3(threads), 0, s, a);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const uint64_t cols = ((uint64_t)nyt + a.ny + a.nz) * a.nx;
+  const uint32_t g = (uint32_t)std::min<uint64_t>(div_up(cols, 256), (uint64_t)cu * 16);
+  hipLaunchKernelGGL(lorenzo_prefix_kernel, dim3(g), dim3(256), 0, s, a, nzt, nyt);
+  e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((lorenzo_tile_kernel<C, TZ>), dim3(nyt, nzt), dim3(threads), 0, s, a);
+  return hipGetLastError();
+}
+
 }  // namespace
 
 hipError_t launch_lorenzo(const LorenzoArgs& a, hipStream_t s) {
@@ -419,6 +679,17 @@ uint32_t lorenzo_tiles(uint32_t nz, uint32_t ny, uint32_t nx) {
   return (uint32_t)(div_up(nx, kTX) * div_up(ny, kTY) * div_up(nz, kTZ));
 }
 
+LorenzoScratch lorenzo_inverse_scratch(uint32_t nz, uint32_t ny, uint32_t nx, int cu) {
+  LorenzoScratch l;
+  l.ty = tile_rows(nz, ny, nx, cu);
+  const uint64_t nzt = div_up(nz, tile_planes(nx)), nyt = div_up(ny, l.ty);
+  l.fits = nzt <= 65535;  // (the grid's second dimension)
+  l.band = round_up((nzt - 1) * ny * nx, 64);
+  l.corner = l.band + round_up((nyt - 1) * nz * nx, 64);
+  l.words = l.corner + 2 * nzt * nyt * nx;
+  return l;
+}
+
 hipError_t launch_lorenzo_inverse(const LorenzoArgs& a, int cu, hipStream_t s) {
   const uint64_t n = (uint64_t)a.nx * a.ny * a.nz;
   if (n == 0) return hipSuccess;
@@ -427,6 +698,12 @@ hipError_t launch_lorenzo_inverse(const LorenzoArgs& a, int cu, hipStream_t s) {
     hipLaunchKernelGGL(lorenzo_scatter_kernel, dim3(g), dim3(256), 0, s, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
+  }
+  if (a.slab) {
+    if (a.nx <= 1024) return launch_tiles<1, 16>(a, cu, s);
+    if (a.nx <= 2048) return launch_tiles<2, 8>(a, cu, s);
+    if (a.nx <= 4096) return launch_tiles<4, 4>(a, cu, s);
+    return launch_tiles<8, 4>(a, cu, s);
   }
   // two elements a thread where rows are even and the codes 4-byte aligned
   // (the q scratch is a whole allocation)

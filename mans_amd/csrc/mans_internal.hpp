@@ -330,9 +330,22 @@ struct LorenzoArgs {
   const uint32_t* in_idx;
   const int32_t* in_val;
   uint64_t n_out;
-  int32_t* q;                    // [n] scratch
+  int32_t* q;                    // [n] the outliers' residuals in their places (by tiles: the out array)
   float* recon;                  // [n] out
+  // inverse by tiles of ty rows (null: through q); LorenzoScratch
+  int32_t* slab;
+  int32_t* band;
+  int32_t* corner;
+  uint32_t ty;
 };
+// Scratch of the inverse by tiles, in 32-bit words: slab at 0, then band,
+// corner.
+struct LorenzoScratch {
+  bool fits;                     // the tiles fit a launch
+  uint32_t ty;
+  uint64_t band, corner, words;
+};
+LorenzoScratch lorenzo_inverse_scratch(uint32_t nz, uint32_t ny, uint32_t nx, int cu);
 hipError_t launch_lorenzo(const LorenzoArgs& a, hipStream_t s);
 hipError_t launch_lorenzo_inverse(const LorenzoArgs& a, int cu, hipStream_t s);
 uint32_t lorenzo_tiles(uint32_t nz, uint32_t ny, uint32_t nx);
