@@ -373,10 +373,11 @@ def frame_encode(x, p: Params, ws: Workspace, out=None, stream=None, sync_size: 
     cap = frame_max_size(n, p)
     if out is None:
         out = torch.empty(cap, dtype=torch.uint8, device=x.device)
-    if d_size is None:
+    if d_size is None and not sync_size:
         d_size = torch.zeros(1, dtype=torch.int64, device=x.device)
     h_size = C.c_uint64(0)
-    rc = lib().mans_frame_encode(C.byref(p), _ptr(x), n, out.data_ptr(), out.numel(), d_size.data_ptr(),
+    rc = lib().mans_frame_encode(C.byref(p), _ptr(x), n, out.data_ptr(), out.numel(),
+                                 None if d_size is None else d_size.data_ptr(),
                                  C.byref(h_size) if sync_size else None, ws.handle, _stream(stream))
     _check(rc, "mans_frame_encode")
     return (out, h_size.value) if sync_size else (out, d_size)

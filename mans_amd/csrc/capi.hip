@@ -37,7 +37,6 @@ struct mans_workspace {
   uint64_t scratch_cap = 0;
   uint16_t* spill = nullptr;     // encoder spill areas (one per resident wave)
   uint64_t spill_cap = 0;
-  uint64_t* d_u64 = nullptr;     // [4]
   uint64_t* h_pinned = nullptr;  // [32] host pinned
   // set once a call ran on a capturing stream: the buffers above may then
   // be referenced by a graph, so they are never freed or replaced again
@@ -283,7 +282,8 @@ mans_status run_encode(mans_workspace* ws, const CodecDesc& d, const HistSource*
 }
 
 mans_status read_u64(mans_workspace* ws, const uint64_t* d, uint64_t* h, hipStream_t s) {
-  HIP_TRY(hipMemcpyAsync(ws->h_pinned, d, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+  // (d may be h_pinned itself: the size stored there by the launch)
+  if (d != ws->h_pinned) HIP_TRY(launch_to_host(ws->h_pinned, d, 2, nullptr, 0, s));
   HIP_TRY(hipStreamSynchronize(s));
   *h = ws->h_pinned[0];
   return MANS_OK;
@@ -377,7 +377,6 @@ mans_status mans_workspace_create(mans_workspace** out, int32_t device) {
   }
   bool ok = hipMalloc(&ws->hist, 4 * 256 * 4) == hipSuccess && hipMalloc(&ws->counters, 64 * 4) == hipSuccess &&
             hipMalloc(&ws->table, 4 * 256 * 16) == hipSuccess && hipMalloc(&ws->hist_out, 4 * 256 * 4) == hipSuccess &&
-            hipMalloc(&ws->d_u64, 4 * 8) == hipSuccess &&
             hipHostMalloc((void**)&ws->h_pinned, 32 * 8, hipHostMallocDefault) == hipSuccess;
   ok = ok && hipMemset(ws->hist, 0, 4 * 256 * 4) == hipSuccess && hipMemset(ws->counters, 0, 64 * 4) == hipSuccess &&
        hipMemset(ws->table, 0, 4 * 256 * 16) == hipSuccess && hipDeviceSynchronize() == hipSuccess;
@@ -400,7 +399,6 @@ mans_status mans_workspace_destroy(mans_workspace* ws) {
   if (ws->status) (void)hipFree(ws->status);
   if (ws->scratch) (void)hipFree(ws->scratch);
   if (ws->spill) (void)hipFree(ws->spill);
-  if (ws->d_u64) (void)hipFree(ws->d_u64);
   if (ws->h_pinned) (void)hipHostFree(ws->h_pinned);
   for (hipEvent_t e : ws->ev) (void)hipEventDestroy(e);
   delete ws;
@@ -486,9 +484,9 @@ mans_status mans_encode(const mans_params* p, const void* d_in, uint64_t n, void
   d.total_units = d.plane[0].nb;
   d.data_off = section_bytes(d.plane[0].nb, f);
   HistSource src = {(const uint8_t*)d_in, n, 1u, 0u};
-  st = run_encode(ws, d, &src, n ? 1 : 0, (uint8_t*)d_out, d_out_size, h_out_size ? ws->d_u64 : nullptr, nullptr, s);
+  st = run_encode(ws, d, &src, n ? 1 : 0, (uint8_t*)d_out, d_out_size, h_out_size ? ws->h_pinned : nullptr, nullptr, s);
   if (st != MANS_OK) return st;
-  if (h_out_size) return read_u64(ws, ws->d_u64, h_out_size, s);
+  if (h_out_size) return read_u64(ws, ws->h_pinned, h_out_size, s);
   return MANS_OK;
 }
 
@@ -655,11 +653,9 @@ static mans_status adm_map_impl(const uint16_t* d_in, uint64_t n, int32_t* d_off
   const uint64_t chain = div_up(gsize, kAdmTicketGroups);
   mans_status st = ensure_status(ws, std::max<uint64_t>(chain, 1));
   if (st != MANS_OK) return st;
-  HIP_TRY(launch_fill_u64(ws->status, chain, 0, s));
   // counters[2] = ticket, counters[4] = this call's domain / capacity flags
   // (kept apart from the sticky stream-error word counters[3])
-  HIP_TRY(launch_fill_u32(ws->counters + 2, 1, 0, s));
-  HIP_TRY(launch_fill_u32(ws->counters + 4, 1, 0, s));
+  HIP_TRY(launch_zero(ws->status, chain, ws->counters + 2, 1, ws->counters + 4, 1, s));
   if (gsize == 0) HIP_TRY(launch_fill_u32((uint32_t*)d_offsets, 1, 0, s));
   AdmMapArgs a;
   memset(&a, 0, sizeof(a));
@@ -678,8 +674,7 @@ static mans_status adm_map_impl(const uint16_t* d_in, uint64_t n, int32_t* d_off
   HIP_TRY(launch_adm_map(a, ws->cu, s));
   if (h_bits_len || h_in_domain) {
     uint32_t* hp = (uint32_t*)ws->h_pinned;
-    HIP_TRY(hipMemcpyAsync(hp, d_offsets + gsize, 4, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(hp + 1, ws->counters + 4, 4, hipMemcpyDeviceToHost, s));
+    HIP_TRY(launch_to_host(hp, d_offsets + gsize, 1, ws->counters + 4, 1, s));
     HIP_TRY(hipStreamSynchronize(s));
     if (h_bits_len) *h_bits_len = 32ull * hp[0];
     if (h_in_domain) *h_in_domain = (hp[1] & kErrAdmDomain) ? 0 : 1;
@@ -752,9 +747,7 @@ mans_status mans_lorenzo_quantize(const float* d_field, uint32_t nz, uint32_t ny
   if (st == MANS_OK) st = ensure_scratch(ws, grp_off + 1024ull * fix_cap);
   if (st != MANS_OK) return st;
   // counters[5]: tile ticket; counters[4]: this call's flags
-  HIP_TRY(launch_fill_u64(ws->status, ntiles, 0, s));
-  HIP_TRY(launch_fill_u32(ws->counters + 4, 2, 0, s));
-  HIP_TRY(launch_fill_u32((uint32_t*)(ws->scratch + list_off), 1, 0, s));
+  HIP_TRY(launch_zero(ws->status, ntiles, ws->counters + 4, 2, (uint32_t*)(ws->scratch + list_off), 1, s));
   if (ntiles == 0) HIP_TRY(launch_fill_u64(d_outlier_count, 1, 0, s));
   LorenzoArgs a;
   memset(&a, 0, sizeof(a));
@@ -783,8 +776,7 @@ mans_status mans_lorenzo_quantize(const float* d_field, uint32_t nz, uint32_t ny
   HIP_TRY(launch_lorenzo(a, s));
   prof_mark(ws, s, nullptr);
   if (h_outlier_count) {
-    HIP_TRY(hipMemcpyAsync(ws->h_pinned, d_outlier_count, 8, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(ws->h_pinned + 1, ws->counters + 4, 4, hipMemcpyDeviceToHost, s));
+    HIP_TRY(launch_to_host(ws->h_pinned, d_outlier_count, 2, ws->counters + 4, 1, s));
     HIP_TRY(hipStreamSynchronize(s));
     *h_outlier_count = ws->h_pinned[0];
     const uint32_t flags = (uint32_t)ws->h_pinned[1];
@@ -934,7 +926,7 @@ mans_status mans_frame_encode(const mans_params* p, const void* d_in, uint64_t n
   d.data_off = off;
   uint32_t hdr[32];
   frame_header(hdr, n, eb, mode, f, p->prob_bits, d, gsize, meta_off);
-  uint64_t* dsz = d_size ? d_size : (h_size ? ws->d_u64 : nullptr);
+  uint64_t* dsz = d_size ? d_size : (h_size ? ws->h_pinned : nullptr);
   st = run_encode(ws, d, src, nsrc, out, nullptr, dsz, hdr, s);
   if (st != MANS_OK) return st;
   if (h_size) return read_u64(ws, dsz, h_size, s);
@@ -971,7 +963,7 @@ static mans_status frame_decode_impl(const void* d_in, uint64_t c, const void* h
   if (h_header) {
     memcpy(hcopy, h_header, kFrameHeaderBytes);
   } else {
-    HIP_TRY(hipMemcpyAsync(ws->h_pinned, d_in, kFrameHeaderBytes, hipMemcpyDeviceToHost, s));
+    HIP_TRY(launch_to_host(ws->h_pinned, d_in, kFrameHeaderBytes / 4, nullptr, 0, s));
     HIP_TRY(hipStreamSynchronize(s));
     memcpy(hcopy, ws->h_pinned, kFrameHeaderBytes);
   }

@@ -186,6 +186,20 @@ __global__ void fill_u32_kernel(uint32_t* p, uint64_t n, uint32_t v) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
     p[i] = v;
 }
+// Zeroes n words at p and na / nb at a / b: one launch before a call.
+__global__ void zero_kernel(uint64_t* p, uint64_t n, uint32_t* a, uint32_t na, uint32_t* b, uint32_t nb) {
+  const uint64_t i0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i0 < na) a[i0] = 0;
+  if (i0 < nb) b[i0] = 0;
+  for (uint64_t i = i0; i < n; i += (uint64_t)gridDim.x * blockDim.x) p[i] = 0;
+}
+// na words of a, then nb of b, to pinned host memory.  (An asynchronous copy
+// each is a kernel of the runtime's too, of 4-5 us, and 10 us of host time.)
+__global__ void to_host_kernel(uint32_t* dst, const uint32_t* a, uint32_t na, const uint32_t* b, uint32_t nb) {
+  const uint32_t i = threadIdx.x;
+  if (i < na) dst[i] = a[i];
+  else if (i < na + nb) dst[i] = b[i - na];
+}
 
 }  // namespace
 
@@ -220,6 +234,19 @@ hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s) {
   if (n == 0) return hipSuccess;
   uint32_t grid = (uint32_t)(div_up(n, 256) < 1024 ? div_up(n, 256) : 1024);
   hipLaunchKernelGGL(fill_u32_kernel, dim3(grid), dim3(256), 0, s, p, n, v);
+  return hipGetLastError();
+}
+hipError_t launch_zero(uint64_t* p, uint64_t n, uint32_t* a, uint32_t na, uint32_t* b, uint32_t nb, hipStream_t s) {
+  const uint64_t most = std::max<uint64_t>(std::max<uint64_t>(n, 1), std::max(na, nb));
+  const uint32_t grid = (uint32_t)std::min<uint64_t>(div_up(most, 256), 1024);
+  if (std::max(na, nb) > grid * 256u) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(zero_kernel, dim3(grid), dim3(256), 0, s, p, n, a, na, b, nb);
+  return hipGetLastError();
+}
+hipError_t launch_to_host(void* dst, const void* a, uint32_t na, const void* b, uint32_t nb, hipStream_t s) {
+  if (na + nb > 256) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(to_host_kernel, dim3(1), dim3(64 * (uint32_t)div_up(na + nb, 64)), 0, s, (uint32_t*)dst,
+                     (const uint32_t*)a, na, (const uint32_t*)b, nb);
   return hipGetLastError();
 }
 

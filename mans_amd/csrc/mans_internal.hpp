@@ -397,5 +397,9 @@ hipError_t launch_adm_map(const AdmMapArgs& a, int cu, hipStream_t s);
 hipError_t launch_adm_unmap(const AdmUnmapArgs& a, hipStream_t s);
 hipError_t launch_fill_u64(uint64_t* p, uint64_t n, uint64_t v, hipStream_t s);
 hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s);
+// n 8-byte words at p, na / nb 4-byte words at a / b (at most 2^18) to zero
+hipError_t launch_zero(uint64_t* p, uint64_t n, uint32_t* a, uint32_t na, uint32_t* b, uint32_t nb, hipStream_t s);
+// na 4-byte words of a, then nb of b (at most 256) to pinned host memory
+hipError_t launch_to_host(void* dst, const void* a, uint32_t na, const void* b, uint32_t nb, hipStream_t s);
 
 }  // namespace mans
