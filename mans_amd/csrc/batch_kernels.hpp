@@ -258,7 +258,7 @@ __host__ __device__ constexpr uint32_t enc_ticket_units(uint32_t eb, uint32_t ro
 
 // Ticket lt of buffer B: units u0 .. u0 + UT - 1, u0 = UT lt, UT = rounds x
 // chains, coded round by round with the single-buffer launch's multi-chain
-// step (enc_step64f, a linear LDS stage of H + 256 words per chain, spilled
+// step (enc_steps64, a linear LDS stage of H + 256 words per chain, spilled
 // to the wave's slot in chunks of H; unit j of the ticket has slot area j).
 // uint32 tickets of four rounds code planes 0-1 of both blocks, then planes
 // 2-3, so the tables change once; of two rounds, planes 0-1 then 2-3 of one
@@ -484,7 +484,7 @@ __device__ uint64_t encode_ticket(const BatchBuf& B, uint32_t b, uint32_t lt, ui
 // 2 NC consecutive units u0 = 2 NC lt, ..., lanes 0-31 coding units u0 ..
 // u0 + NC - 1 and lanes 32-63 the next NC, NC chains per lane (unit
 // u0 + NC h + c is chain c of half h), with the single-buffer 32-lane step
-// (enc_step32f: one ballot per chain, words compacted per half).  NC = 2
+// (enc_steps32: one ballot per chain, words compacted per half).  NC = 2
 // for uint8 (two blocks per half) and uint16 (both planes of one block per
 // half: one element load feeds both chains); uint32 tickets are the two
 // units u0, u0 + 1 (planes p0, p0 + 1 of one block), one chain per lane,
@@ -828,9 +828,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3))) vo
     uint16_t* const sl = spill + slot * batch_slot_words<PB>();
     uint64_t agg;
     if constexpr (L == 32) {
-      if (B.eb == 1) agg = encode_ticket32<PB, 1, KB>(B, b, lt, tix, a, gen, wl, sl, tkey);
-      else if (B.eb == 2) agg = encode_ticket32<PB, 2, KB>(B, b, lt, tix, a, gen, wl, sl, tkey);
-      else agg = encode_ticket32<PB, 4, KB>(B, b, lt, tix, a, gen, wl, sl, tkey);
+      // (16 elements of two blocks ahead need 160 bytes of scratch a lane: 16.3
+      // ms on 4096 buffers of 8.5 GB against 11.9)
+      constexpr int KB32 = KB > 8 ? 8 : KB;
+      if (B.eb == 1) agg = encode_ticket32<PB, 1, KB32>(B, b, lt, tix, a, gen, wl, sl, tkey);
+      else if (B.eb == 2) agg = encode_ticket32<PB, 2, KB32>(B, b, lt, tix, a, gen, wl, sl, tkey);
+      else agg = encode_ticket32<PB, 4, KB32>(B, b, lt, tix, a, gen, wl, sl, tkey);
     } else {
       if (B.eb == 1) agg = encode_ticket<PB, 1, (KB / 4 < 4 ? 4 : KB / 4)>(B, b, lt, tix, a, gen, wl, sl, tkey);
       else if (B.eb == 2) agg = encode_ticket<PB, 2, (KB / 2 < 4 ? 4 : KB / 2)>(B, b, lt, tix, a, gen, wl, sl, tkey);

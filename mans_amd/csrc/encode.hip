@@ -38,11 +38,14 @@ namespace {
 constexpr int kBatch = 16;  // steps per prefetch batch
 // encode_mc_kernel: spill slots of a coding wavefront (on 1 GiB of uint16
 // codes 3 slots and more take the same time, 2 a third more: with one ticket
-// of slack every workgroup waits for the slowest), and workgroups per CU (5:
-// 0.59 ms, 4: 0.61, more no less; with four chains a lane 3 are enough).  Each
-// has its slots: 320 and 390 MB at p = 10 on 256 CUs.
+// of slack every workgroup waits for the slowest), and workgroups per CU (two
+// chains: 5 take 0.59 ms, 4 0.61, more no less; four chains: 3 are enough.  In
+// the 32-lane format 4 and 5 take the same; four chains 2 groups 0.157 ms on
+// 128 MiB of uint32, 3 0.144, but each group has its slots, whose allocation
+// a workspace pays for: 260 to 390 MB at p = 10 on 256 CUs, and 3 would make
+// them half as large again as two slots of four chains were).
 constexpr uint32_t kEncSlots = 3;
-constexpr int enc_groups(int chains) { return chains >= 4 ? 3 : 5; }
+constexpr int enc_groups(int lanes, int chains) { return lanes == 32 ? (chains >= 4 ? 2 : 4) : (chains >= 4 ? 3 : 5); }
 
 template <typename T>
 using gptr = const __attribute__((address_space(1))) T*;
@@ -845,7 +848,7 @@ hipError_t launch_mc(const EncodeArgs& a, int cu, hipStream_t s, uint64_t* need_
                                                               64 * (NW + 1), lds);
   if (e != hipSuccess) return e;
   if (per_cu < 1) per_cu = 1;
-  if (per_cu > enc_groups(CH)) per_cu = enc_groups(CH);
+  if (per_cu > enc_groups(L, CH)) per_cu = enc_groups(L, CH);
   const uint64_t waves = div_up(a.d.total_units, NS);
   uint64_t grid = div_up(waves, NW);
   const uint64_t cap = (uint64_t)cu * (uint64_t)per_cu;
