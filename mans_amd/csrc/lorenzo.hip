@@ -257,11 +257,13 @@ __global__ __launch_bounds__(kTX * kFixGroups) void lorenzo_fixup_kernel(Lorenzo
 //    both; their prefixes over the tiles; then each tile from those, the
 //    x-prefix last.  All sums are of 32-bit integers, so their order does not
 //    matter.  The codes are read twice, the field is written once and the
-//    sums are a tenth of it; or
+//    sums take 0.4 bytes an element where tiles are 16 planes x 32 rows, 1.1
+//    where they are 4 x 32 (rows over 2048) and up to 3.5 where they are
+//    small (fields of few tiles); or
 //  * (buffers that overlap) per plane the x-prefix of each row plus the
 //    y-prefix (running per column), then per column the z-prefix and
 //    f' = q * 2 eb, with every q through memory.
-// 500 x 499 x 900: by tiles 515 us, through q 820.
+// 500 x 499 x 900: by tiles 489 us, through q 820.
 __global__ void lorenzo_scatter_kernel(LorenzoArgs a) {
   for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < a.n_out; k += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t i = a.in_idx[k];
@@ -429,8 +431,8 @@ __device__ __forceinline__ void residuals(const LorenzoArgs& a, uint32_t z0, uin
 }
 
 // A tile's sums: over its planes for each row (slab), over its rows for each
-// plane (band), over both (corner[0 .. ]).  A thread per x, the next row's
-// codes loaded ahead; the last slab's and the last band's are not needed.
+// plane (band), over both (corner).  A thread per x, the next row's codes
+// loaded ahead; the last slab's and the last band's are not needed.
 // Memory bound: 154 us for 500 x 499 x 900.  (Workgroups of 256 columns, which
 // share lines of a row across XCDs: 167.)
 template <uint32_t TZ>
@@ -464,7 +466,7 @@ __global__ __launch_bounds__(1024) void lorenzo_sums_kernel(LorenzoArgs a) {
       all += v[k];
       if (yt + 1 < nyt && (FULL || z0 + k < a.nz)) a.band[((uint64_t)yt * a.nz + z0 + k) * a.nx + x] = v[k];
     }
-    a.corner[((uint64_t)zt * nyt + yt) * a.nx + x] = all;
+    if (zt + 1 < nzt && yt + 1 < nyt) a.corner[((uint64_t)zt * (nyt - 1) + yt) * a.nx + x] = all;
   };
   const uint32_t x = blockIdx.x % nxc * 1024u + threadIdx.x;
   if (x >= a.nx) return;
@@ -472,12 +474,17 @@ __global__ __launch_bounds__(1024) void lorenzo_sums_kernel(LorenzoArgs a) {
   else columns(x, std::false_type{});
 }
 
-// Prefixes over the tiles, a thread a column: of slab over the slabs and of
-// band over the bands (inclusive, in place), of corner over both (exclusive,
-// into corner[nzt nyt nx ..]).
+// Prefixes over the tiles, a thread a column, all inclusive and in place: of
+// slab over the slabs, of band over the bands, of corner over the bands and,
+// once those are complete (AXIS 1, a launch of its own), over the slabs.  Every
+// entry is read and written once an axis, whatever the shape.  (Each corner's
+// prefix summed from all corners before it, in one launch: 502 us for 500 x 499
+// x 900 against 489, 351 ms for 1 x 1,000,000 x 1000 against 14.)
+template <int AXIS>
 __global__ __launch_bounds__(256) void lorenzo_prefix_kernel(LorenzoArgs a, uint32_t nzt, uint32_t nyt) {
   constexpr uint32_t B = 16;  // entries loaded before any is summed
-  const uint64_t per_slab = (uint64_t)a.ny * a.nx, per_band = (uint64_t)a.nz * a.nx, per_row = (uint64_t)nyt * a.nx;
+  const uint64_t per_slab = (uint64_t)a.ny * a.nx, per_band = (uint64_t)a.nz * a.nx;
+  const uint64_t per_row = (uint64_t)(nyt - 1) * a.nx;  // corners of a slab
   auto scan = [&](int32_t* p, uint64_t step, uint32_t n) {
     int32_t s = 0;
     for (uint32_t k0 = 0; k0 < n; k0 += B) {
@@ -491,20 +498,12 @@ __global__ __launch_bounds__(256) void lorenzo_prefix_kernel(LorenzoArgs a, uint
       }
     }
   };
-  // (the corners first: each takes up to nzt nyt reads)
-  const uint64_t nc = per_row, ns = nzt > 1 ? per_slab : 0, nb = nyt > 1 ? per_band : 0;
+  const uint64_t nc = AXIS == 1 ? per_row : (nyt > 1 ? (uint64_t)(nzt - 1) * a.nx : 0);
+  const uint64_t ns = AXIS == 0 && nzt > 1 ? per_slab : 0, nb = AXIS == 0 && nyt > 1 ? per_band : 0;
   for (uint64_t j = (uint64_t)blockIdx.x * 256 + threadIdx.x; j < nc + ns + nb; j += (uint64_t)gridDim.x * 256) {
     if (j < nc) {
-      const uint32_t yt = (uint32_t)(j / a.nx), x = (uint32_t)(j % a.nx);
-      int32_t run = 0;
-      for (uint32_t zt = 0; zt < nzt; ++zt) {
-        a.corner[(nzt + (uint64_t)zt) * per_row + j] = run;
-        const int32_t* p = a.corner + zt * per_row + x;
-        for (uint32_t k0 = 0; k0 < yt; k0 += B) {
-#pragma unroll
-          for (uint32_t k = 0; k < B; ++k) run += k0 + k < yt ? p[(uint64_t)(k0 + k) * a.nx] : 0;
-        }
-      }
+      if (AXIS == 1) scan(a.corner + j, per_row, nzt - 1);
+      else scan(a.corner + j / a.nx * per_row + j % a.nx, a.nx, nyt - 1);
     } else if (j < nc + ns) {
       scan(a.slab + (j - nc), per_slab, nzt - 1);
     } else {
@@ -543,7 +542,7 @@ __device__ __forceinline__ int32_t row_sum(int32_t v) {
 template <uint32_t C, uint32_t TZ, bool FULL>
 __device__ __forceinline__ void write_tile(const LorenzoArgs& a, int32_t (&s_w)[2][TZ][16]) {
   static_assert(TZ % 4 == 0, "four planes a row sum");
-  const uint32_t yt = blockIdx.x, zt = blockIdx.y, nyt = gridDim.x, nzt = gridDim.y;
+  const uint32_t yt = blockIdx.x, zt = blockIdx.y, nyt = gridDim.x;
   const uint32_t y0 = yt * a.ty, y1 = a.ny - y0 < a.ty ? a.ny : y0 + a.ty, z0 = zt * TZ;
   const uint32_t t = threadIdx.x, lane = t & 63u, w = __builtin_amdgcn_readfirstlane(t >> 6);
   const uint64_t plane = (uint64_t)a.ny * a.nx;
@@ -555,7 +554,7 @@ __device__ __forceinline__ void write_tile(const LorenzoArgs& a, int32_t (&s_w)[
 #pragma unroll
   for (uint32_t c = 0; c < C; ++c) {
     const uint32_t x = column(c);
-    int32_t run = a.corner[((uint64_t)(nzt + zt) * nyt + yt) * a.nx + x];
+    int32_t run = zt > 0 && yt > 0 ? a.corner[((uint64_t)(zt - 1) * (nyt - 1) + yt - 1) * a.nx + x] : 0;
 #pragma unroll
     for (uint32_t k = 0; k < TZ; ++k) {
       if (yt > 0 && (FULL || z0 + k < a.nz)) run += a.band[((uint64_t)(yt - 1) * a.nz + z0 + k) * a.nx + x];
@@ -631,14 +630,17 @@ __global__ __launch_bounds__(1024) void lorenzo_tile_kernel(LorenzoArgs a) {
 }
 
 // Planes of a tile: as many as a thread's sums of all its columns fit in
-// registers.  Rows: 32, fewer (not under 2, nor so few that a column has more
+// registers.  Rows: 32; fewer (not under 2, nor so few that a column has more
 // than 256 tiles: the prefixes take time for each) while the tiles would not
-// give every compute unit two workgroups.
+// give every compute unit two workgroups; more while a column has over 4096
+// and every compute unit would still have four (1 x 1,000,000 x 1000: 14.1 ms
+// from 128 rows on, 16.2 with 32).
 uint32_t tile_planes(uint32_t nx) { return nx <= 1024 ? 16u : (nx <= 2048 ? 8u : 4u); }
 uint32_t tile_rows(uint32_t nz, uint32_t ny, uint32_t nx, int cu) {
+  const uint64_t nzt = div_up(nz, tile_planes(nx));
   uint32_t ty = 32;
-  while (ty > 2 && div_up(ny, ty / 2) <= 256 && div_up(nz, tile_planes(nx)) * div_up(ny, ty) < 2ull * (uint64_t)cu)
-    ty /= 2;
+  while (ty > 2 && div_up(ny, ty / 2) <= 256 && nzt * div_up(ny, ty) < 2ull * (uint64_t)cu) ty /= 2;
+  while (div_up(ny, ty) > 4096 && nzt * div_up(ny, 2 * ty) >= 4ull * (uint64_t)cu) ty *= 2;
   return ty;
 }
 
@@ -649,11 +651,16 @@ hipError_t launch_tiles(const LorenzoArgs& a, int cu, hipStream_t s) {
   hipLaunchKernelGGL(lorenzo_sums_kernel<TZ>, dim3(nyt * (uint32_t)div_up(a.nx, 1024), nzt), dim3(threads), 0, s, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const uint64_t cols = ((uint64_t)nyt + a.ny + a.nz) * a.nx;
-  const uint32_t g = (uint32_t)std::min<uint64_t>(div_up(cols, 256), (uint64_t)cu * 16);
-  hipLaunchKernelGGL(lorenzo_prefix_kernel, dim3(g), dim3(256), 0, s, a, nzt, nyt);
+  auto grid = [&](uint64_t cols) { return dim3((uint32_t)std::min<uint64_t>(div_up(cols, 256), (uint64_t)cu * 16)); };
+  const uint64_t cols = ((uint64_t)nzt - 1 + a.ny + a.nz) * a.nx;
+  hipLaunchKernelGGL(lorenzo_prefix_kernel<0>, grid(cols), dim3(256), 0, s, a, nzt, nyt);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
+  if (nzt > 2 && nyt > 1) {
+    hipLaunchKernelGGL(lorenzo_prefix_kernel<1>, grid((uint64_t)(nyt - 1) * a.nx), dim3(256), 0, s, a, nzt, nyt);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
   hipLaunchKernelGGL((lorenzo_tile_kernel<C, TZ>), dim3(nyt, nzt), dim3(threads), 0, s, a);
   return hipGetLastError();
 }
@@ -683,10 +690,10 @@ LorenzoScratch lorenzo_inverse_scratch(uint32_t nz, uint32_t ny, uint32_t nx, in
   LorenzoScratch l;
   l.ty = tile_rows(nz, ny, nx, cu);
   const uint64_t nzt = div_up(nz, tile_planes(nx)), nyt = div_up(ny, l.ty);
-  l.fits = nzt <= 65535;  // (the grid's second dimension)
-  l.band = round_up((nzt - 1) * ny * nx, 64);
-  l.corner = l.band + round_up((nyt - 1) * nz * nx, 64);
-  l.words = l.corner + 2 * nzt * nyt * nx;
+  l.fits = nzt <= 65535;  // (the grid's second dimension; tile_rows keeps the first small)
+  l.band = (nzt - 1) * ny * nx;
+  l.corner = l.band + (nyt - 1) * nz * nx;
+  l.words = l.corner + (nzt - 1) * (nyt - 1) * nx;
   return l;
 }
 

@@ -1,0 +1,50 @@
+"""The plan of the Lorenzo inverse by tiles (lorenzo_inverse_scratch in
+mans_amd/csrc/lorenzo.hip), on the CPU: its scratch never exceeds the 4 bytes
+an element that the route through q takes (so a workspace sized by one serves
+the other), a column has at most 4096 bands whatever the field's shape (the
+prefixes walk them one after another), and every launch fits a grid."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import mans_amd
+
+
+class Scratch(ctypes.Structure):
+    _fields_ = [("fits", ctypes.c_bool), ("ty", ctypes.c_uint32), ("band", ctypes.c_uint64),
+                ("corner", ctypes.c_uint64), ("words", ctypes.c_uint64)]
+
+
+def plan(nz, ny, nx, cu=256):
+    f = mans_amd.lib()._ZN4mans23lorenzo_inverse_scratchEjjji
+    f.restype = Scratch
+    f.argtypes = [ctypes.c_uint32] * 3 + [ctypes.c_int]
+    return f(nz, ny, nx, cu)
+
+
+def shapes():
+    rng = np.random.default_rng(5)
+    out = [(1, 1, 1), (1, 2, 1), (2, 2, 2), (5, 3, 8192), (1, 500, 1000), (1, 512, 8192), (24, 500, 900),
+           (512, 24, 1024), (64, 512, 1024), (500, 499, 900), (1, 1_000_000, 1000), (1, 4_000_000, 1000),
+           (17, 100_000, 64), (1, (1 << 32) - 1, 1), (1, 1 << 31, 1), (2, 1 << 30, 1), ((1 << 32) - 1, 1, 1),
+           (1_000_000, 64, 64)]
+    for _ in range(2000):
+        nx = int(np.exp(rng.uniform(0, np.log(8193))))
+        ny = int(np.exp(rng.uniform(0, np.log((1 << 32) / nx))))
+        nz = int(np.exp(rng.uniform(0, np.log((1 << 32) / nx / ny))))
+        out.append((max(nz, 1), max(ny, 1), max(nx, 1)))
+    return out
+
+
+@pytest.mark.parametrize("cu", [64, 256, 304])
+def test_plan_is_bounded(cu):
+    for nz, ny, nx in shapes():
+        n = nz * ny * nx
+        if n >= 1 << 32:
+            continue
+        s = plan(nz, ny, nx, cu)
+        bands = -(-ny // s.ty)
+        assert s.words <= n, (nz, ny, nx, s.words / n)
+        assert bands <= 4096, (nz, ny, nx, s.ty)
+        assert bands * -(-nx // 1024) * 1024 < 1 << 32, (nz, ny, nx, s.ty)
