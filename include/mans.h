@@ -179,8 +179,8 @@ mans_status mans_lorenzo_quantize(const float* d_field, uint32_t nz, uint32_t ny
 /* The inverse: q as the 3-D prefix sum of the residuals (codes and
  * outliers), d_field = q * float32(2 eb).  Needs up to 3.5 bytes of
  * workspace per element (0.4 in large fields with rows of up to 1024, 1.1
- * with longer ones; 4 where d_field overlaps an input or nz is above
- * 262,140); d_field holds the outliers in between. */
+ * with longer ones; 4 where d_field overlaps an input, in fields of few
+ * rows, and with nz above 262,140); d_field holds the outliers in between. */
 mans_status mans_lorenzo_reconstruct(const uint16_t* d_codes, const uint32_t* d_outlier_idx,
                                      const int32_t* d_outlier_val, uint64_t outlier_count, uint32_t nz, uint32_t ny,
                                      uint32_t nx, double error_bound, float* d_field, mans_workspace* ws,

@@ -808,7 +808,7 @@ mans_status mans_lorenzo_reconstruct(const uint16_t* d_codes, const uint32_t* d_
     return b + bytes <= f || f + 4 * n <= b;
   };
   const LorenzoScratch l = lorenzo_inverse_scratch(nz, ny, nx, ws->cu);
-  const bool tiles = l.fits && apart(d_codes, 2 * n) && apart(d_outlier_idx, outlier_count * 4) &&
+  const bool tiles = l.tiles && apart(d_codes, 2 * n) && apart(d_outlier_idx, outlier_count * 4) &&
                      apart(d_outlier_val, outlier_count * 4);
   mans_status st = ensure_scratch(ws, tiles ? 4 * l.words : 4 * n);
   if (st != MANS_OK) return st;

@@ -260,7 +260,7 @@ __global__ __launch_bounds__(kTX * kFixGroups) void lorenzo_fixup_kernel(Lorenzo
 //    sums take 0.4 bytes an element where tiles are 16 planes x 32 rows, 1.1
 //    where they are 4 x 32 (rows over 2048) and up to 3.5 where they are
 //    small (fields of few tiles); or
-//  * (buffers that overlap) per plane the x-prefix of each row plus the
+//  * (buffers that overlap, fields of few rows) per plane the x-prefix of each row plus the
 //    y-prefix (running per column), then per column the z-prefix and
 //    f' = q * 2 eb, with every q through memory.
 // 500 x 499 x 900: by tiles 489 us, through q 820.
@@ -648,14 +648,19 @@ template <uint32_t C, uint32_t TZ>
 hipError_t launch_tiles(const LorenzoArgs& a, int cu, hipStream_t s) {
   const uint32_t nyt = (uint32_t)div_up(a.ny, a.ty), nzt = (uint32_t)div_up(a.nz, TZ);
   const uint32_t threads = a.nx > 1024 ? 1024u : (uint32_t)round_up(a.nx, 64);
-  hipLaunchKernelGGL(lorenzo_sums_kernel<TZ>, dim3(nyt * (uint32_t)div_up(a.nx, 1024), nzt), dim3(threads), 0, s, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  hipError_t e;
+  if (nzt > 1 || nyt > 1) {  // (a single tile needs no sums)
+    hipLaunchKernelGGL(lorenzo_sums_kernel<TZ>, dim3(nyt * (uint32_t)div_up(a.nx, 1024), nzt), dim3(threads), 0, s, a);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
   auto grid = [&](uint64_t cols) { return dim3((uint32_t)std::min<uint64_t>(div_up(cols, 256), (uint64_t)cu * 16)); };
-  const uint64_t cols = ((uint64_t)nzt - 1 + a.ny + a.nz) * a.nx;
-  hipLaunchKernelGGL(lorenzo_prefix_kernel<0>, grid(cols), dim3(256), 0, s, a, nzt, nyt);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if (nzt > 2 || nyt > 2) {  // (one entry is its own prefix)
+    const uint64_t cols = ((uint64_t)nzt - 1 + a.ny + a.nz) * a.nx;
+    hipLaunchKernelGGL(lorenzo_prefix_kernel<0>, grid(cols), dim3(256), 0, s, a, nzt, nyt);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
   if (nzt > 2 && nyt > 1) {
     hipLaunchKernelGGL(lorenzo_prefix_kernel<1>, grid((uint64_t)(nyt - 1) * a.nx), dim3(256), 0, s, a, nzt, nyt);
     e = hipGetLastError();
@@ -686,11 +691,25 @@ uint32_t lorenzo_tiles(uint32_t nz, uint32_t ny, uint32_t nx) {
   return (uint32_t)(div_up(nx, kTX) * div_up(ny, kTY) * div_up(nz, kTZ));
 }
 
+// Fields of few rows and planes go through q: with up to three row groups a
+// plane its two launches are shorter than the tiles' three or four (1 x 16 x
+// 1024 13 us against 21, 16 x 16 x 16 13 against 16, 64 x 8 x 512 13 against
+// 22, 128 x 16 x 64 20 against 20).  From there on the time of a workgroup a
+// plane, or of a thread a column, grows past them (1 x 64 x 64 35 against 16,
+// 256 x 8 x 64 25 against 20; a row's second chunk counts as a row: 16 x 16 x
+// 2048 21 against 23).  Fields of one row have few tiles' sums or none (16 x 1
+// x 512: 9 us against 4).
+static bool few_rows(uint32_t nz, uint32_t ny, uint32_t nx) {
+  if (ny == 1 || nz > 128 || nx > 2048) return false;
+  return ny <= (nx > 1024 ? 8u : (nx > 512 ? 32u : 25u - nz / 16u));
+}
+
 LorenzoScratch lorenzo_inverse_scratch(uint32_t nz, uint32_t ny, uint32_t nx, int cu) {
   LorenzoScratch l;
   l.ty = tile_rows(nz, ny, nx, cu);
   const uint64_t nzt = div_up(nz, tile_planes(nx)), nyt = div_up(ny, l.ty);
-  l.fits = nzt <= 65535;  // (the grid's second dimension; tile_rows keeps the first small)
+  // (65535: the grid's second dimension; tile_rows keeps the first small)
+  l.tiles = nzt <= 65535 && !few_rows(nz, ny, nx);
   l.band = (nzt - 1) * ny * nx;
   l.corner = l.band + (nyt - 1) * nz * nx;
   l.words = l.corner + (nzt - 1) * (nyt - 1) * nx;

@@ -341,7 +341,7 @@ struct LorenzoArgs {
 // Scratch of the inverse by tiles, in 32-bit words: slab at 0, then band,
 // corner.
 struct LorenzoScratch {
-  bool fits;                     // the tiles fit a launch
+  bool tiles;                    // by tiles (else through q): they fit a launch and are the faster
   uint32_t ty;
   uint64_t band, corner, words;
 };

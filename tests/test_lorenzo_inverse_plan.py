@@ -48,3 +48,12 @@ def test_plan_is_bounded(cu):
         assert s.words <= n, (nz, ny, nx, s.words / n)
         assert bands <= 4096, (nz, ny, nx, s.ty)
         assert bands * -(-nx // 1024) * 1024 < 1 << 32, (nz, ny, nx, s.ty)
+
+
+@pytest.mark.parametrize("shape,tiles", [((4, 4, 4), False), ((16, 16, 16), False), ((24, 24, 32), False),
+                                         ((1, 16, 1024), False), ((128, 16, 64), False), ((64, 8, 512), False),
+                                         ((1, 1, 8192), True), ((16, 1, 512), True), ((1, 64, 64), True),
+                                         ((129, 8, 64), True), ((16, 16, 2048), True), ((64, 64, 64), True),
+                                         ((500, 499, 900), True)])
+def test_fields_of_few_rows_take_the_shorter_route(shape, tiles):
+    assert plan(*shape).fits == tiles
