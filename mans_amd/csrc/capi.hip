@@ -33,8 +33,12 @@ struct mans_workspace {
   uint32_t* hist_out = nullptr;  // [4][256]
   uint64_t* status = nullptr;
   uint64_t status_cap = 0;
-  uint8_t* scratch = nullptr;    // ADM planes of frames
+  uint8_t* scratch = nullptr;    // ADM planes of frames, sums and lists of the Lorenzo front end
   uint64_t scratch_cap = 0;
+  // what the calls before the freeze entitle a later one to (ensure_scratch),
+  // and the scratch that a larger one replaced after it
+  uint64_t scratch_promised = 0;
+  uint8_t* scratch_retired = nullptr;
   uint16_t* spill = nullptr;     // encoder spill areas (one per resident wave)
   uint64_t spill_cap = 0;
   uint64_t* h_pinned = nullptr;  // [32] host pinned
@@ -96,9 +100,29 @@ mans_status ensure_status(mans_workspace* ws, uint64_t n) {
   return MANS_OK;
 }
 
-mans_status ensure_scratch(mans_workspace* ws, uint64_t n) {
+// `size`, if larger than n, is what a call of this kind and size takes at most:
+// a frozen workspace that has served it serves any call that takes no more,
+// whichever of its routes (of different scratch) either takes.  It then gets
+// scratch of the promised size, at most once, beside the one that a graph may
+// use.
+mans_status ensure_scratch(mans_workspace* ws, uint64_t n, uint64_t size = 0) {
+  if (!ws->frozen) ws->scratch_promised = std::max({ws->scratch_promised, n, size});
   if (n <= ws->scratch_cap) return MANS_OK;
-  if (ws->frozen) return MANS_ERR_CAPACITY;
+  if (ws->frozen) {
+    if (n > ws->scratch_promised || ws->scratch_retired) return MANS_ERR_CAPACITY;
+    // (the stream may be under capture, which allows an allocation only in
+    // this mode; a new buffer is part of no graph)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+    uint8_t* more = nullptr;
+    const hipError_t e = hipMalloc(&more, ws->scratch_promised);
+    HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+    HIP_TRY(e);
+    ws->scratch_retired = ws->scratch;
+    ws->scratch = more;
+    ws->scratch_cap = ws->scratch_promised;
+    return MANS_OK;
+  }
   if (ws->scratch) (void)hipFree(ws->scratch);
   ws->scratch = nullptr;
   ws->scratch_cap = 0;
@@ -398,6 +422,7 @@ mans_status mans_workspace_destroy(mans_workspace* ws) {
   if (ws->hist_out) (void)hipFree(ws->hist_out);
   if (ws->status) (void)hipFree(ws->status);
   if (ws->scratch) (void)hipFree(ws->scratch);
+  if (ws->scratch_retired) (void)hipFree(ws->scratch_retired);
   if (ws->spill) (void)hipFree(ws->spill);
   if (ws->h_pinned) (void)hipHostFree(ws->h_pinned);
   for (hipEvent_t e : ws->ev) (void)hipEventDestroy(e);
@@ -810,7 +835,7 @@ mans_status mans_lorenzo_reconstruct(const uint16_t* d_codes, const uint32_t* d_
   const LorenzoScratch l = lorenzo_inverse_scratch(nz, ny, nx, ws->cu);
   const bool tiles = l.tiles && apart(d_codes, 2 * n) && apart(d_outlier_idx, outlier_count * 4) &&
                      apart(d_outlier_val, outlier_count * 4);
-  mans_status st = ensure_scratch(ws, tiles ? 4 * l.words : 4 * n);
+  mans_status st = ensure_scratch(ws, tiles ? 4 * l.words : 4 * n, 4 * n);
   if (st != MANS_OK) return st;
   LorenzoArgs a;
   memset(&a, 0, sizeof(a));
