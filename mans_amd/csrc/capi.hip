@@ -131,9 +131,16 @@ mans_status ensure_scratch(mans_workspace* ws, uint64_t n, uint64_t size = 0) {
   return MANS_OK;
 }
 
-mans_status ensure_spill(mans_workspace* ws, uint64_t bytes) {
-  if (bytes <= ws->spill_cap) return MANS_OK;
-  if (ws->frozen) return MANS_ERR_CAPACITY;
+// A frozen workspace keeps its spill area and serves an encode that would take
+// up to twice the workgroups it holds (elements of another width, whose
+// workgroups take other amounts), with those it holds.
+mans_status ensure_spill(mans_workspace* ws, const SpillNeed& need) {
+  if (need.bytes() <= ws->spill_cap) return MANS_OK;
+  if (ws->frozen) {
+    const uint64_t held = ws->spill_cap / need.group_bytes;
+    return held >= 1 && 2 * held >= need.groups ? MANS_OK : MANS_ERR_CAPACITY;
+  }
+  const uint64_t bytes = std::max(need.bytes(), need.least_bytes);
   if (ws->spill) (void)hipFree(ws->spill);
   ws->spill = nullptr;
   ws->spill_cap = 0;
@@ -143,7 +150,7 @@ mans_status ensure_spill(mans_workspace* ws, uint64_t bytes) {
 }
 
 // Spill area the encoder needs on a large input of P planes of stride S.
-uint64_t spill_for(mans_workspace* ws, int lanes, int pb, int P, uint32_t S, int order) {
+SpillNeed spill_for(mans_workspace* ws, int lanes, int pb, int P, uint32_t S, int order) {
   EncodeArgs e;
   memset(&e, 0, sizeof(e));
   e.d.lanes = lanes;
@@ -152,9 +159,9 @@ uint64_t spill_for(mans_workspace* ws, int lanes, int pb, int P, uint32_t S, int
   e.d.order = order;
   for (int k = 0; k < P; ++k) e.d.plane[k].stride = S;
   e.d.total_units = 1ull << 30;
-  uint64_t bytes = 0;
-  if (encode_spill_bytes(e, ws->cu, &bytes) != hipSuccess) return 0;
-  return bytes;
+  SpillNeed need;
+  if (encode_spill(e, ws->cu, &need) != hipSuccess) return SpillNeed{};
+  return need;
 }
 
 // Profiling: events recorded around launches when enabled.
@@ -297,8 +304,8 @@ mans_status run_encode(mans_workspace* ws, const CodecDesc& d, const HistSource*
   EncodeArgs probe;
   memset(&probe, 0, sizeof(probe));
   probe.d = d;
-  uint64_t spill = 0;
-  HIP_TRY(encode_spill_bytes(probe, ws->cu, &spill));
+  SpillNeed spill;
+  HIP_TRY(encode_spill(probe, ws->cu, &spill));
   st = ensure_spill(ws, spill);
   if (st != MANS_OK) return st;
   const EncodeScratch sc{ws->hist, ws->counters, ws->table, ws->status, ws->spill, ws->spill_cap};
@@ -447,10 +454,12 @@ mans_status mans_workspace_reserve(mans_workspace* ws, uint64_t max_bytes, const
     // the encoder's spill areas for this element width (byte planes) and for
     // single byte streams (single streams, ADM planes)
     const int eb = p->elem_bytes == 4 ? 4 : (p->elem_bytes == 2 ? 2 : 1);
-    const uint64_t need = std::max({spill_for(ws, lanes, p->prob_bits, eb, (uint32_t)eb, 0),
-                                    spill_for(ws, lanes, p->prob_bits, 1, 1u, 0),
-                                    spill_for(ws, lanes, p->prob_bits, 1, 1u, 1)});
-    st = ensure_spill(ws, need);
+    SpillNeed need[3] = {spill_for(ws, lanes, p->prob_bits, eb, (uint32_t)eb, 0),
+                         spill_for(ws, lanes, p->prob_bits, 1, 1u, 0), spill_for(ws, lanes, p->prob_bits, 1, 1u, 1)};
+    // (the largest first: one allocation)
+    std::sort(need, need + 3, [](const SpillNeed& a, const SpillNeed& b) { return a.bytes() > b.bytes(); });
+    for (const SpillNeed& n : need)
+      if (st == MANS_OK) st = ensure_spill(ws, n);
   }
   return st;
 }

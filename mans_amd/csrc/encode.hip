@@ -816,7 +816,7 @@ __global__ __launch_bounds__(64 * (NW + 1), 5) void encode_mc_kernel(EncodeArgs 
 // spill areas.  The multi-chain kernel (encode_mc_kernel): BPT blocks per
 // half-wave ticket, spill areas.
 template <int L, int PB, int S, int CH, int NW>
-hipError_t launch_staged(const EncodeArgs& a, int cu, hipStream_t s, uint64_t* need_spill) {
+hipError_t launch_staged(const EncodeArgs& a, int cu, hipStream_t s, SpillNeed* need_spill) {
   constexpr uint32_t CSTAGE = chain_stage_words<PB>();
   const size_t lds = (size_t)a.d.num_planes * kNumSymbols * sizeof(uint4) + (size_t)NW * (CH * CSTAGE + 128) * 2u;
   int per_cu = 0;
@@ -829,7 +829,7 @@ hipError_t launch_staged(const EncodeArgs& a, int cu, hipStream_t s, uint64_t* n
   if (grid > cap) grid = cap;
   if (grid < 1) grid = 1;
   if (need_spill) {
-    *need_spill = 0;
+    *need_spill = SpillNeed{};
     return hipSuccess;
   }
   hipLaunchKernelGGL((encode_kernel<L, PB, S, CH, NW>), dim3((uint32_t)grid), dim3(64 * NW), lds, s, a);
@@ -837,7 +837,7 @@ hipError_t launch_staged(const EncodeArgs& a, int cu, hipStream_t s, uint64_t* n
 }
 
 template <int L, int PB, int S, int BPT, int NW, int HB>
-hipError_t launch_mc(const EncodeArgs& a, int cu, hipStream_t s, uint64_t* need_spill) {
+hipError_t launch_mc(const EncodeArgs& a, int cu, hipStream_t s, SpillNeed* need_spill) {
   constexpr uint32_t CSTAGE = chain_stage_words<PB>();
   constexpr int CH = S * BPT, NS = CH * (L == 32 ? 2 : 1);
   constexpr uint32_t REG = (1u << HB) + 256u;
@@ -855,12 +855,15 @@ hipError_t launch_mc(const EncodeArgs& a, int cu, hipStream_t s, uint64_t* need_
   if (grid > cap) grid = cap;
   if (grid < 1) grid = 1;
   // kEncSlots slots per coding wavefront of CH chains of 64 lanes
-  const uint64_t spill_bytes = grid * NW * kEncSlots * CH * CSTAGE * 2ull;
+  const uint64_t group_bytes = (uint64_t)NW * kEncSlots * CH * CSTAGE * 2ull;
   if (need_spill) {
-    *need_spill = spill_bytes;
+    *need_spill = SpillNeed{grid, group_bytes, (uint64_t)NW * kEncSlots * 4u * CSTAGE * 2ull};
     return hipSuccess;
   }
-  if (!a.spill || spill_bytes > a.spill_bytes) return hipErrorInvalidValue;
+  // as many workgroups as the area holds (tickets go to any number of them)
+  const uint64_t held = a.spill ? a.spill_bytes / group_bytes : 0;
+  if (held < 1) return hipErrorInvalidValue;
+  if (grid > held) grid = held;
   hipLaunchKernelGGL((encode_mc_kernel<L, PB, S, BPT, NW, HB>), dim3((uint32_t)grid), dim3(64 * (NW + 1)), lds, s, a);
   return hipGetLastError();
 }
@@ -868,7 +871,7 @@ hipError_t launch_mc(const EncodeArgs& a, int cu, hipStream_t s, uint64_t* need_
 // staged: the 32-lane whole-unit kernel (no spill areas: the allocation-free
 // entry point, and ADM planes concatenated at 32 lanes).
 template <int L, int PB>
-hipError_t launch_s(const EncodeArgs& a, int cu, hipStream_t s, uint64_t* need_spill, bool staged) {
+hipError_t launch_s(const EncodeArgs& a, int cu, hipStream_t s, SpillNeed* need_spill, bool staged) {
   const int P = a.d.num_planes;
   const uint32_t S = a.d.plane[0].stride;
   if constexpr (L == 64) {
@@ -892,7 +895,7 @@ hipError_t launch_s(const EncodeArgs& a, int cu, hipStream_t s, uint64_t* need_s
 }
 
 template <int L>
-hipError_t launch_p(const EncodeArgs& a, int cu, hipStream_t s, uint64_t* need_spill, bool staged) {
+hipError_t launch_p(const EncodeArgs& a, int cu, hipStream_t s, SpillNeed* need_spill, bool staged) {
   switch (a.d.prob_bits) {
     case 9: return launch_s<L, 9>(a, cu, s, need_spill, staged);
     case 10: return launch_s<L, 10>(a, cu, s, need_spill, staged);
@@ -903,10 +906,10 @@ hipError_t launch_p(const EncodeArgs& a, int cu, hipStream_t s, uint64_t* need_s
 
 }  // namespace
 
-hipError_t encode_spill_bytes(const EncodeArgs& a, int cu, uint64_t* bytes) {
-  *bytes = 0;
+hipError_t encode_spill(const EncodeArgs& a, int cu, SpillNeed* need) {
+  *need = SpillNeed{};
   if (a.d.total_units == 0) return hipSuccess;
-  return a.d.lanes == 64 ? launch_p<64>(a, cu, nullptr, bytes, false) : launch_p<32>(a, cu, nullptr, bytes, false);
+  return a.d.lanes == 64 ? launch_p<64>(a, cu, nullptr, need, false) : launch_p<32>(a, cu, nullptr, need, false);
 }
 
 // a.spill == nullptr selects the 32-lane whole-unit kernel (no spill areas).

@@ -387,8 +387,14 @@ hipError_t launch_batch_decode_p9(const BatchDecodeArgs&, BatchShape, int, hipSt
 hipError_t launch_batch_decode_p10(const BatchDecodeArgs&, BatchShape, int, hipStream_t);
 hipError_t launch_batch_decode_p11(const BatchDecodeArgs&, BatchShape, int, hipStream_t);
 hipError_t launch_encode(const EncodeArgs& a, int cu, hipStream_t s);
-// bytes of spill area launch_encode needs for a (0 for the 32-lane format)
-hipError_t encode_spill_bytes(const EncodeArgs& a, int cu, uint64_t* bytes);
+// The spill area of a multi-chain encode: of `groups` workgroups (0: none
+// needed), `group_bytes` each; one workgroup of the widest elements takes
+// `least_bytes`.  The launch takes fewer workgroups where the area is smaller.
+struct SpillNeed {
+  uint64_t groups = 0, group_bytes = 0, least_bytes = 0;
+  uint64_t bytes() const { return groups * group_bytes; }
+};
+hipError_t encode_spill(const EncodeArgs& a, int cu, SpillNeed* need);
 hipError_t launch_decode(const DecodeArgs& a, int cu, hipStream_t s);
 // 64-lane ADM frames: decodes plane 0 (the code plane) and restores each
 // block's elements from a.adm (bit plane already decoded) in the same wave.
