@@ -383,8 +383,13 @@ mans_status mans_server_submit(mans_server* s, const mans_request* r, uint64_t* 
 mans_status mans_server_submit_many(mans_server* s, const mans_request* r, int32_t count, uint64_t* ids);
 /* Waits up to timeout_ms (< 0: no limit); MANS_ERR_BUSY if not done yet. */
 mans_status mans_server_wait(mans_server* s, uint64_t id, int32_t timeout_ms, mans_result* out);
-/* Frees a finished request's output. */
+/* Frees a finished request's output: a request waiting for memory may be
+ * launched into it at once, so every read of it must have run. */
 mans_status mans_server_release(mans_server* s, uint64_t id);
+/* The same once the work enqueued so far on `stream` has run (it may be given
+ * back later than that).  Does not wait.  The stream has to exist until the
+ * server is destroyed. */
+mans_status mans_server_release_after(mans_server* s, uint64_t id, void* stream);
 mans_status mans_server_stats(mans_server* s, uint64_t* arena_bytes, uint64_t* arena_used, uint64_t* batches,
                               uint64_t* waiting);
 /* Finishes every submitted request, then frees everything. */

@@ -111,6 +111,7 @@ SIGNATURES = {
     "mans_server_submit_many": (C.c_int, [_vp, C.POINTER(Request), _i32, C.POINTER(_u64)]),
     "mans_server_wait": (C.c_int, [_vp, _u64, _i32, C.POINTER(Result)]),
     "mans_server_release": (C.c_int, [_vp, _u64]),
+    "mans_server_release_after": (C.c_int, [_vp, _u64, _vp]),
     "mans_server_stats": (C.c_int, [_vp, C.POINTER(_u64), C.POINTER(_u64), C.POINTER(_u64), C.POINTER(_u64)]),
     "mans_server_destroy": (C.c_int, [_vp]),
     "mans_set_profiling": (C.c_int, [_vp, _i32]),
@@ -589,6 +590,7 @@ class Server:
         h = C.c_void_p()
         _check(lib().mans_server_create(C.byref(h), C.byref(p), memory_budget, device), "mans_server_create")
         self.handle = h
+        self._reads: dict[int, int] = {}  # request id: the stream a copy of its result is enqueued on
 
     @staticmethod
     def compress_request(x) -> Request:
@@ -624,21 +626,32 @@ class Server:
         if rc == 11:  # MANS_ERR_BUSY
             return None
         _check(rc, "mans_server_wait")
+        res.id = rid
         return res
 
     def fetch(self, res: Result, dtype=None):
         """Copy a result out of the arena into a new CUDA tensor (uint8, or
-        viewed as dtype)."""
+        viewed as dtype), on the current stream.  The result may be released
+        at once: its memory is kept until the copy has run."""
         torch = _torch()
         out = torch.empty(max(1, res.out_bytes), dtype=torch.uint8, device="cuda")
         if res.out_bytes:
             t = _torch_from_ptr(res.d_out, res.out_bytes)
             out[:res.out_bytes].copy_(t)
+            # (torch.cuda.current_stream() takes 3 us, this 0.1)
+            s = torch._C._cuda_getCurrentRawStream(out.get_device())
+            rid = getattr(res, "id", None)
+            if rid is None or self._reads.setdefault(rid, s) != s:  # not from wait(), or on two streams
+                torch.cuda.current_stream().synchronize()
         out = out[:res.out_bytes]
         return out.view(dtype) if dtype is not None else out
 
     def release(self, rid: int) -> None:
-        _check(lib().mans_server_release(self.handle, rid), "mans_server_release")
+        s = self._reads.pop(rid, None)
+        if s is None:
+            _check(lib().mans_server_release(self.handle, rid), "mans_server_release")
+        else:
+            _check(lib().mans_server_release_after(self.handle, rid, s), "mans_server_release_after")
 
     def stats(self) -> dict:
         v = [C.c_uint64(0) for _ in range(4)]

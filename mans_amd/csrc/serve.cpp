@@ -120,6 +120,15 @@ struct Slot {
   bool busy = false;
 };
 
+// Released outputs that work on a client's stream still reads
+// (mans_server_release_after), and the event recorded behind it, which is when
+// somebody first waits for memory: one for all that were released by then.
+struct Leaving {
+  hipStream_t stream = nullptr;
+  hipEvent_t read = nullptr;                          // (null: not recorded yet)
+  std::vector<std::pair<uint64_t, uint64_t>> blocks;  // offset, bytes
+};
+
 double ms_between(Clock::time_point a, Clock::time_point b) {
   return std::chrono::duration<double, std::milli>(b - a).count();
 }
@@ -136,6 +145,7 @@ struct mans_server {
   std::condition_variable cv_work, cv_done;
   std::deque<Req*> waiting;
   std::unordered_map<uint64_t, Req*> reqs;
+  std::vector<Leaving> leaving;
   uint64_t next_id = 1;
   bool stop = false;
   std::thread worker;
@@ -152,6 +162,52 @@ uint64_t out_bytes_for(const mans_params& p, const mans_request& r) {
     return mans_frame_max_size(r.n_elems, &q);
   }
   return r.n_elems * (uint64_t)r.elem_bytes;
+}
+
+// Gives back the released outputs whose reads have run (lock held).  With
+// `idle`, also those of a stream that has run out of work by now: an event
+// recorded now would say so only later.
+void reap(mans_server* S, bool idle) {
+  int dev = -1;
+  (void)hipGetDevice(&dev);
+  if (dev != S->device) (void)hipSetDevice(S->device);
+  // (a stream that is not ready leaves an error with the calling thread, which
+  // may be the client's)
+  auto ok = [](hipError_t e) {
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
+  };
+  size_t k = 0;
+  for (size_t i = 0; i < S->leaving.size(); ++i) {
+    Leaving& l = S->leaving[i];
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    bool read = false;
+    if (l.read && ok(hipEventQuery(l.read))) {
+      read = true;
+    } else if (!ok(hipStreamIsCapturing(l.stream, &cs)) || cs != hipStreamCaptureStatusNone) {
+      // (nothing can be asked of the stream until the capture ends)
+    } else if (idle && ok(hipStreamQuery(l.stream))) {
+      read = true;
+    } else if (!l.read) {
+      if (!ok(hipEventCreateWithFlags(&l.read, hipEventDisableTiming))) {
+        l.read = nullptr;
+        read = ok(hipStreamSynchronize(l.stream));
+      } else if (!ok(hipEventRecord(l.read, l.stream))) {  // (another device's stream)
+        (void)hipEventDestroy(l.read);
+        l.read = nullptr;
+        read = ok(hipStreamSynchronize(l.stream));
+      }
+    }
+    if (read) {
+      for (const auto& b : l.blocks) S->arena.release(b.first, b.second);
+      if (l.read) (void)hipEventDestroy(l.read);
+    } else {
+      if (k != i) S->leaving[k] = std::move(l);
+      ++k;
+    }
+  }
+  S->leaving.resize(k);
+  if (dev >= 0 && dev != S->device) (void)hipSetDevice(dev);
 }
 
 // Launches the requests admitted into `sl` (called without the lock; the
@@ -274,6 +330,7 @@ void worker_loop(mans_server* S) {
       }
     }
     if (progress) S->cv_done.notify_all();
+    if (!S->leaving.empty() && !S->waiting.empty()) reap(S, false);
     for (Slot& sl : S->slot) {
       if (sl.busy || S->waiting.empty()) continue;
       if (!admit(S, sl)) continue;
@@ -287,8 +344,9 @@ void worker_loop(mans_server* S) {
     const bool any_busy = S->slot[0].busy || S->slot[1].busy;
     if (S->stop && S->waiting.empty() && !any_busy) break;
     if (!progress) {
-      if (any_busy) {
-        // poll the in-flight batches without holding the lock
+      if (any_busy || (!S->leaving.empty() && !S->waiting.empty())) {
+        // poll the in-flight batches, and the reads that a request waiting
+        // for memory waits for, without holding the lock
         lk.unlock();
         std::this_thread::sleep_for(std::chrono::microseconds(20));
         lk.lock();
@@ -421,14 +479,27 @@ mans_status mans_server_wait(mans_server* S, uint64_t id, int32_t timeout_ms, ma
   return MANS_OK;
 }
 
-mans_status mans_server_release(mans_server* S, uint64_t id) {
+// Frees a finished request's output, after the work on *stream unless null.
+static mans_status release_req(mans_server* S, uint64_t id, const hipStream_t* stream) {
   if (!S) return MANS_ERR_INVALID_ARG;
   {
     std::lock_guard<std::mutex> g(S->mu);
     auto it = S->reqs.find(id);
     if (it == S->reqs.end() || it->second->state != 2) return MANS_ERR_INVALID_ARG;
     Req* q = it->second;
-    S->arena.release(q->out_off, q->out_cap);
+    if (stream) {
+      Leaving* l = nullptr;
+      for (Leaving& o : S->leaving)
+        if (o.stream == *stream && !o.read) l = &o;
+      if (!l) {
+        S->leaving.emplace_back();
+        l = &S->leaving.back();
+        l->stream = *stream;
+      }
+      l->blocks.emplace_back(q->out_off, q->out_cap);
+    } else {
+      S->arena.release(q->out_off, q->out_cap);
+    }
     S->reqs.erase(it);
     delete q;
   }
@@ -436,10 +507,18 @@ mans_status mans_server_release(mans_server* S, uint64_t id) {
   return MANS_OK;
 }
 
+mans_status mans_server_release(mans_server* S, uint64_t id) { return release_req(S, id, nullptr); }
+
+mans_status mans_server_release_after(mans_server* S, uint64_t id, void* stream) {
+  const hipStream_t s = (hipStream_t)stream;
+  return release_req(S, id, &s);
+}
+
 mans_status mans_server_stats(mans_server* S, uint64_t* arena_bytes, uint64_t* arena_used, uint64_t* batches,
                               uint64_t* waiting) {
   if (!S) return MANS_ERR_INVALID_ARG;
   std::lock_guard<std::mutex> g(S->mu);
+  reap(S, true);
   if (arena_bytes) *arena_bytes = S->arena.total();
   if (arena_used) *arena_used = S->arena.used();
   if (batches) *batches = S->batches;
@@ -468,6 +547,8 @@ mans_status mans_server_destroy(mans_server* S) {
     if (sl.done) (void)hipEventDestroy(sl.done);
     if (sl.stream) (void)hipStreamDestroy(sl.stream);
   }
+  for (Leaving& l : S->leaving)
+    if (l.read) (void)hipEventDestroy(l.read);
   if (S->arena_base) (void)hipFree(S->arena_base);
   for (auto& kv : S->reqs) delete kv.second;
   delete S;
