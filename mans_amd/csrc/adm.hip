@@ -53,9 +53,11 @@ constexpr uint32_t kPairs = kAdmTicketGroups / 2;
 constexpr uint32_t kTicketGroups = kWaves * kAdmTicketGroups;
 static_assert(kPairs % 2 == 0, "pairs are mapped two at a time");
 // Bytes of a wavefront's area for its 32 groups' bits: 4 for each of the 1024
-// lanes.  Groups that need more are mapped a second time when their offset is
-// known, in the area itself (lane buffers of kLaneWords words, padded to 9 so
-// the lanes' words of one index fall in distinct LDS banks).
+// lanes.  The pairs from the first on that does not fit are mapped a second
+// time when their offset is known and the area has been copied out, in the area
+// itself (lane buffers of kLaneWords words, padded to 9 so the lanes' words of
+// one index fall in distinct LDS banks).  (All pairs mapped again: 4 M elements
+// of 0.43 bytes of bits 66 us; a second pass over everything 59; so 48.)
 constexpr uint32_t kAreaBytes = 4096;
 constexpr uint32_t kLaneWords = kAdmLaneBytes / 4 + 1;
 static_assert(64 * kLaneWords * 4 <= kAreaBytes, "the lane buffers fit the area");
@@ -197,17 +199,17 @@ __global__ __launch_bounds__(kThreads) void adm_map_kernel(AdmMapArgs a) {
 
   // the ticket mapped but not resolved (workgroup-uniform): its first group,
   // byte total (in units of 32 bytes, as all offsets here); of this
-  // wavefront's groups the offset in the ticket, the total, whether they are
-  // in the area, and in lane g < 32 group g's offset
-  bool pend = false, p_kept = false;
+  // wavefront's groups the offset in the ticket, the total, and in lane g < 32
+  // group g's offset
+  bool pend = false;
   uint32_t p_tk = 0, p_agg = 0, p_off = 0, p_sum = 0, p_exlo = 0;
 
-  // Groups that did not fit the area: mapped again from the input, pair by
-  // pair, with the lanes' bits in the area's lane buffers.
-  auto direct = [&](uint32_t* area, uint64_t excl, uint64_t g0) {
+  // Pairs pr0 on, which did not fit the area: mapped again from the input,
+  // pair by pair, with the lanes' bits in the area's lane buffers.
+  auto direct = [&](uint32_t* area, uint64_t excl, uint64_t g0, uint32_t pr0) {
     uint32_t* const mybits = area + lane * kLaneWords;
     const uint8_t* const wavebytes = (const uint8_t*)area;
-    for (uint32_t pr = 0; pr < kPairs; ++pr) {
+    for (uint32_t pr = pr0; pr < kPairs; ++pr) {
       const uint64_t g = g0 + 2 * pr + half;
       const LaneRaw cur = raw_lane<false>(a, g, lin);
       uint32_t v[kAdmChunk], codes[4];
@@ -254,19 +256,27 @@ __global__ __launch_bounds__(kThreads) void adm_map_kernel(AdmMapArgs a) {
     excl += p_off;
     const uint64_t g0 = (uint64_t)p_tk + wave * kAdmTicketGroups;
     if ((uint32_t)lane < kAdmTicketGroups && g0 + lane < a.gsize) a.offsets[g0 + lane] = (int32_t)(excl + p_exlo);
-    if (p_kept && 32ull * (excl + p_sum) <= a.bits_capacity) {
+    // the pairs in the area (each ends where the next begins) and their bytes
+    uint32_t pairs = kPairs, held = p_sum;
+    if (32u * p_sum > kAreaBytes) {
+      pairs = (uint32_t)__popcll(__ballot((lane & 1) == 0 && lane >= 2 && (uint32_t)lane < kAdmTicketGroups &&
+                                          32u * p_exlo <= kAreaBytes));
+      held = __builtin_amdgcn_readlane(p_exlo, 2u * pairs);
+    }
+    uint32_t pr0 = 0;
+    if (32ull * (excl + held) <= a.bits_capacity) {
       uint8_t* const dst = a.bits + 32ull * excl;
       if (((uintptr_t)a.bits & 15u) == 0) {
         const uint4* const src = s_area[slot][wave];
-        for (uint32_t q = (uint32_t)lane; q < 2u * p_sum; q += 64u) ((uint4*)dst)[q] = src[q];
+        for (uint32_t q = (uint32_t)lane; q < 2u * held; q += 64u) ((uint4*)dst)[q] = src[q];
       } else {
         const uint8_t* const src = (const uint8_t*)s_area[slot][wave];
-        for (uint32_t q = (uint32_t)lane; q < 32u * p_sum; q += 64u) dst[q] = src[q];
+        for (uint32_t q = (uint32_t)lane; q < 32u * held; q += 64u) dst[q] = src[q];
       }
       __threadfence_block();  // (the area is written again)
-    } else if (p_sum > 0) {
-      direct((uint32_t*)s_area[slot][wave], excl, g0);
+      pr0 = pairs;
     }
+    if (pr0 < kPairs && p_sum > 0) direct((uint32_t*)s_area[slot][wave], excl, g0, pr0);
   };
 
   if (t == 0) s_next[0] = atomicAdd(a.ticket, kTicketGroups);
@@ -276,7 +286,6 @@ __global__ __launch_bounds__(kThreads) void adm_map_kernel(AdmMapArgs a) {
     const uint32_t tk = __builtin_amdgcn_readfirstlane(s_next[slot]);
     const bool more = (uint64_t)tk < a.gsize;
     uint32_t ex = 0, exlo = 0;
-    bool kept = true;
     if (more) {
       const uint64_t g0 = (uint64_t)tk + wave * kAdmTicketGroups;
       uint8_t* const area = (uint8_t*)s_area[slot][wave];
@@ -303,9 +312,9 @@ __global__ __launch_bounds__(kThreads) void adm_map_kernel(AdmMapArgs a) {
         if (g < a.gsize && lin == 0) a.centers[g] = (uint16_t)c;
         const uint32_t m0 = __builtin_amdgcn_readlane(m, 0), m1 = __builtin_amdgcn_readlane(m, 32);
         const uint32_t at = 32u * (ex + (half ? m0 : 0u)) + lin * m;  // this lane's bytes in the area
-        if (32u * (ex + m0 + m1) > kAreaBytes) {
-          kept = false;
-        } else if (kept && narrow) {
+        // (the pairs that fit are the first ones: the sum only grows)
+        const bool fits = 32u * (ex + m0 + m1) <= kAreaBytes;
+        if (fits && narrow) {
           // the byte that holds bit bo, if the lane has one: ones from there
           if (bo < 8u * m) word |= ((1ull << (8u - (bo & 7u))) - 1u) << (63u - (bo | 7u));
           word = __builtin_bswap64(word);
@@ -314,7 +323,7 @@ __global__ __launch_bounds__(kThreads) void adm_map_kernel(AdmMapArgs a) {
             if (j < m) area[at + j] = (uint8_t)word;
             word >>= 8;
           }
-        } else if (kept) {
+        } else if (fits) {
           for (uint32_t i = (uint32_t)lane; i < 8u * (m0 + m1); i += 64u) ((uint32_t*)area)[8u * ex + i] = 0;
           __threadfence_block();
           uint32_t p = 0;  // bit of the lane, `at` bytes into the area
@@ -376,7 +385,6 @@ __global__ __launch_bounds__(kThreads) void adm_map_kernel(AdmMapArgs a) {
     p_off = off;
     p_sum = ex;
     p_exlo = exlo;
-    p_kept = kept;
   }
 }
 
