@@ -972,17 +972,19 @@ __device__ bool frame_bad(const BatchBuf& B) {
 }
 
 // The LUTs of planes p0 .. p0 + np - 1 of buffer B into lut[2^p each], by the
-// whole workgroup: wavefront k scans plane p0 + k's frequencies into cdf[k],
-// then every thread searches its slots, all of them at once (one after
-// another a slot's eight dependent reads took most of the build).  Returns
-// true if a table does not sum to 2^p.
+// whole workgroup: wavefront k scans plane p0 + k's (of all planes, in turn)
+// frequencies into cdf[k], then every thread searches its slots, all of them
+// at once (one after another a slot's eight dependent reads took most of the
+// build).  Returns true if a table of any plane does not sum to 2^p: the
+// buffer's other items reject it too, and nothing of it is decoded.
 template <int PB, int NW>
 __device__ __forceinline__ bool build_luts(const BatchBuf& B, uint32_t p0, uint32_t np, uint32_t* lut,
                                            uint32_t (*cdf)[kNumSymbols + 1]) {
   constexpr uint32_t W = 1u << PB, T = 64u * NW;
-  const uint32_t t = threadIdx.x, lane = t & 63u, wave = wave_u32(t >> 6);
-  if (wave < np) {
-    const u32x2 q = ((gptr<u32x2>)(B.in + B.section[p0 + wave] + kAnsHeaderBytes))[lane];
+  const uint32_t t = threadIdx.x, lane = t & 63u, wave = wave_u32(t >> 6), P = B.eb;
+  static_assert(NW >= (int)kMaxPlanes, "a wavefront per plane");
+  if (wave < P) {
+    const u32x2 q = ((gptr<u32x2>)(B.in + B.section[(p0 + wave) & (P - 1u)] + kAnsHeaderBytes))[lane];
     const uint32_t v[4] = {q.x & 0xffffu, q.x >> 16, q.y & 0xffffu, q.y >> 16};
     const uint32_t ls = v[0] + v[1] + v[2] + v[3];
     uint32_t inc = ls;
@@ -1000,12 +1002,9 @@ __device__ __forceinline__ bool build_luts(const BatchBuf& B, uint32_t p0, uint3
     if (lane == 63) cdf[wave][kNumSymbols] = run;
   }
   __syncthreads();
-  bool bad = false;
+  for (uint32_t k = 0; k < P; ++k)
+    if (B.n > 0 && cdf[k][kNumSymbols] != W) return true;
   for (uint32_t k = 0; k < np; ++k) {
-    if (B.n > 0 && cdf[k][kNumSymbols] != W) {
-      bad = true;
-      continue;
-    }
     constexpr uint32_t PER = W > T ? W / T : 1u;
     uint32_t lo[PER];
 #pragma unroll
@@ -1024,7 +1023,7 @@ __device__ __forceinline__ bool build_luts(const BatchBuf& B, uint32_t p0, uint3
       }
     }
   }
-  return bad;
+  return false;
 }
 
 // Decode ticket lt of buffer B with the 64-lane ring decoder: two blocks (2
@@ -1426,7 +1425,7 @@ __global__ __launch_bounds__(64 * NW) void batch_decode_kernel(BatchDecodeArgs a
   uint16_t* const wstage = rings + wave * (2 * DecRing<KB>::WORDS);
   // (the build's cumulative sums take the rings' place)
   uint32_t (*const cdf)[kNumSymbols + 1] = (uint32_t(*)[kNumSymbols + 1]) rings;
-  static_assert(sizeof(uint32_t) * 2 * (kNumSymbols + 1) <= NW * 4 * DecRing<KB>::WORDS, "cdf in the rings");
+  static_assert(sizeof(uint32_t) * kMaxPlanes * (kNumSymbols + 1) <= NW * 4 * DecRing<KB>::WORDS, "cdf in the rings");
   // (the first item is the workgroup's number: the queue's atomics take 11 ns
   // each, 17 us for a launch's first ones)
   for (uint32_t k = 0, it = blockIdx.x; it < a.nitems; it = wave_u32(s_item[k++ & 1u])) {
