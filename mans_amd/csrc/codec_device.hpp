@@ -4,9 +4,6 @@
 #pragma once
 #include "mans_internal.hpp"
 
-#ifndef SLEEPX
-#define SLEEPX 1
-#endif
 namespace mans {
 
 template <int S> struct ElemOf;
@@ -289,7 +286,7 @@ __device__ __forceinline__ uint64_t look_back_window(const uint64_t* status, int
     excl += wave_sum(part);
     if (found) return excl;
     j -= 64 * groups;
-    if (groups < K) __builtin_amdgcn_s_sleep(SLEEPX);
+    if (groups < K) __builtin_amdgcn_s_sleep(1);
   }
 }
 
