@@ -476,10 +476,12 @@ __global__ __launch_bounds__(1024) void lorenzo_sums_kernel(LorenzoArgs a) {
 
 // Prefixes over the tiles, a thread a column, all inclusive and in place: of
 // slab over the slabs, of band over the bands, of corner over the bands and,
-// once those are complete (AXIS 1, a launch of its own), over the slabs.  Every
-// entry is read and written once an axis, whatever the shape.  (Each corner's
+// once those are complete (AXIS 1, a launch of its own), over the slabs; of few
+// slabs each tile sums them itself instead.  Every entry is read and written
+// once an axis, whatever the shape.  (Each corner's
 // prefix summed from all corners before it, in one launch: 502 us for 500 x 499
 // x 900 against 489, 351 ms for 1 x 1,000,000 x 1000 against 14.)
+constexpr uint32_t kCornerSlabs = 8;  // (48 x 29 x 246: 21.5 us with the launch, 20.4 without)
 template <int AXIS>
 __global__ __launch_bounds__(256) void lorenzo_prefix_kernel(LorenzoArgs a, uint32_t nzt, uint32_t nyt) {
   constexpr uint32_t B = 16;  // entries loaded before any is summed
@@ -554,7 +556,10 @@ __device__ __forceinline__ void write_tile(const LorenzoArgs& a, int32_t (&s_w)[
 #pragma unroll
   for (uint32_t c = 0; c < C; ++c) {
     const uint32_t x = column(c);
-    int32_t run = zt > 0 && yt > 0 ? a.corner[((uint64_t)(zt - 1) * (nyt - 1) + yt - 1) * a.nx + x] : 0;
+    int32_t run = 0;
+    if (yt > 0)
+      for (uint32_t z = zt > 0 && gridDim.y > kCornerSlabs ? zt - 1 : 0; z < zt; ++z)
+        run += a.corner[((uint64_t)z * (nyt - 1) + yt - 1) * a.nx + x];
 #pragma unroll
     for (uint32_t k = 0; k < TZ; ++k) {
       if (yt > 0 && (FULL || z0 + k < a.nz)) run += a.band[((uint64_t)(yt - 1) * a.nz + z0 + k) * a.nx + x];
@@ -630,17 +635,33 @@ __global__ __launch_bounds__(1024) void lorenzo_tile_kernel(LorenzoArgs a) {
 }
 
 // Planes of a tile: as many as a thread's sums of all its columns fit in
-// registers.  Rows: 32; fewer (not under 2, nor so few that a column has more
-// than 256 tiles: the prefixes take time for each) while the tiles would not
-// give every compute unit two workgroups; more while a column has over 4096
-// and every compute unit would still have four (1 x 1,000,000 x 1000: 14.1 ms
-// from 128 rows on, 16.2 with 32).
+// registers.
 uint32_t tile_planes(uint32_t nx) { return nx <= 1024 ? 16u : (nx <= 2048 ? 8u : 4u); }
+// Rows of a tile: those of 2 .. 32 with the least time, in rows: the rounds of
+// resident tiles (16 wavefronts a compute unit, four tiles at most) times a
+// tile's rows and two for its start, and a 32nd for each band, which the
+// prefixes walk one after another (at most 256 bands under 32 rows).  Within 2 %
+// of the best of the five over 105 shapes, where two tiles a compute unit
+// whatever their size were 10 % (256 x 48 x 1024: 44 us against 60, through q
+// 51; 500 x 100 x 900: 100 against 142).  More rows while a column has over
+// 4096 bands and every compute unit would still have four tiles (1 x 1,000,000
+// x 1000: 14.1 ms from 128 rows on, 16.2 with 32).
 uint32_t tile_rows(uint32_t nz, uint32_t ny, uint32_t nx, int cu) {
-  const uint64_t nzt = div_up(nz, tile_planes(nx));
+  const uint64_t nzt = div_up(nz, tile_planes(nx)), chip = (uint64_t)std::max(cu, 1);
+  const uint64_t waves = div_up(std::min(nx, 1024u), 64);
+  const uint64_t held = chip * std::max<uint64_t>(1, std::min<uint64_t>(4, 16 / waves));
   uint32_t ty = 32;
-  while (ty > 2 && div_up(ny, ty / 2) <= 256 && nzt * div_up(ny, ty) < 2ull * (uint64_t)cu) ty /= 2;
-  while (div_up(ny, ty) > 4096 && nzt * div_up(ny, 2 * ty) >= 4ull * (uint64_t)cu) ty *= 2;
+  uint64_t least = ~0ull;
+  for (uint32_t r = 32; r >= 2; r /= 2) {
+    const uint64_t bands = div_up(ny, r);
+    if (r < 32 && bands > 256) break;
+    const uint64_t cost = 32 * div_up(nzt * bands, held) * (r + 2) + bands;
+    if (cost < least) {
+      least = cost;
+      ty = r;
+    }
+  }
+  while (div_up(ny, ty) > 4096 && nzt * div_up(ny, 2ull * ty) >= 4 * chip) ty *= 2;
   return ty;
 }
 
@@ -661,7 +682,7 @@ hipError_t launch_tiles(const LorenzoArgs& a, int cu, hipStream_t s) {
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  if (nzt > 2 && nyt > 1) {
+  if (nzt > kCornerSlabs && nyt > 1) {
     hipLaunchKernelGGL(lorenzo_prefix_kernel<1>, grid((uint64_t)(nyt - 1) * a.nx), dim3(256), 0, s, a, nzt, nyt);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -691,17 +712,28 @@ uint32_t lorenzo_tiles(uint32_t nz, uint32_t ny, uint32_t nx) {
   return (uint32_t)(div_up(nx, kTX) * div_up(ny, kTY) * div_up(nz, kTZ));
 }
 
-// Fields of few rows and planes go through q: with up to three row groups a
-// plane its two launches are shorter than the tiles' three or four (1 x 16 x
-// 1024 13 us against 21, 16 x 16 x 16 13 against 16, 64 x 8 x 512 13 against
-// 22, 128 x 16 x 64 20 against 20).  From there on the time of a workgroup a
-// plane, or of a thread a column, grows past them (1 x 64 x 64 35 against 16,
-// 256 x 8 x 64 25 against 20; a row's second chunk counts as a row: 16 x 16 x
-// 2048 21 against 23).  Fields of one row have few tiles' sums or none (16 x 1
-// x 512: 9 us against 4).
-static bool few_rows(uint32_t nz, uint32_t ny, uint32_t nx) {
-  if (ny == 1 || nz > 128 || nx > 2048) return false;
-  return ny <= (nx > 1024 ? 8u : (nx > 512 ? 32u : 25u - nz / 16u));
+// Whether the field goes through q, by what the two routes take (in 10 ns,
+// fitted to 2092 shapes of up to 1024 planes and 64 rows on 256 compute units:
+// within 5 % of the faster route on all but 59).  Through q are two launches
+// whose time grows with the planes and, in steps of eight, with the rows; rows of
+// odd length are taken an element a thread, rows over 1024 in two chunks.  By
+// tiles are one launch (a single tile), two or three, of about the same time
+// whatever the planes.  1 x 16 x 1024: 13 us through q, 21 by tiles; 64 x 8 x
+// 512 13 and 22; 24 x 24 x 32 17 and 19; 256 x 16 x 1024 34 and 38; 1 x 64 x
+// 64 35 and 16; 256 x 48 x 1024 51 and 44; 128 x 16 x 33 23 and 20.
+static bool through_q(uint32_t nz, uint32_t ny, uint32_t nx) {
+  const bool odd = nx % 2 != 0, one_slab = nz <= tile_planes(nx);
+  if (nx > 2048 || ny > 64 || nz > 1024 || (ny == 1 && one_slab)) return false;
+  const uint32_t groups = (ny + 7) / 8 - 1;  // beyond the first
+  if (nx > 1024) {
+    const uint32_t q = (odd ? 1450u : 1200u) + 10u * nz + (odd ? 900u : 750u) * groups;
+    if (ny <= 2) return q < (one_slab ? 550u + nx / 4u : (ny == 1 ? 1300u : 1700u));
+    return q < 2100u + 6u * nz;
+  }
+  const uint32_t q = (odd ? 1000u : 800u) + (odd ? 9u : 8u) * nz + (odd ? 550u : 420u) * groups;
+  if (ny == 1) return q < 900u + nx / 2u;
+  if (ny == 2) return q < (one_slab ? 550u + nx / 2u : 1100u + nx * 3u / 4u + nz);
+  return q < (ny == 3 ? 1450u : 1740u) + nx * 3u / 4u + 3u * nz;
 }
 
 LorenzoScratch lorenzo_inverse_scratch(uint32_t nz, uint32_t ny, uint32_t nx, int cu) {
@@ -709,7 +741,7 @@ LorenzoScratch lorenzo_inverse_scratch(uint32_t nz, uint32_t ny, uint32_t nx, in
   l.ty = tile_rows(nz, ny, nx, cu);
   const uint64_t nzt = div_up(nz, tile_planes(nx)), nyt = div_up(ny, l.ty);
   // (65535: the grid's second dimension; tile_rows keeps the first small)
-  l.tiles = nzt <= 65535 && !few_rows(nz, ny, nx);
+  l.tiles = nzt <= 65535 && !through_q(nz, ny, nx);
   l.band = (nzt - 1) * ny * nx;
   l.corner = l.band + (nyt - 1) * nz * nx;
   l.words = l.corner + (nzt - 1) * (nyt - 1) * nx;

@@ -33,8 +33,9 @@ def field(shape, seed):
 
 
 # shape, and the rows of a tile on 256 compute units
-SHAPES = [((130, 500, 66), 8), ((250, 500, 33), 16), ((500, 499, 70), 32), ((100, 330, 1030), 8),
-          ((100, 330, 2050), 16), ((124, 130, 4100), 8), ((1, 200_001, 7), 64), ((33, 200_003, 5), 64),
+SHAPES = [((64, 64, 64), 2), ((128, 130, 400), 4), ((130, 500, 66), 8), ((500, 499, 70), 16), ((700, 330, 400), 32),
+          ((100, 330, 1030), 8), ((200, 301, 1500), 32), ((60, 90, 2050), 8), ((100, 333, 2050), 8),
+          ((24, 130, 4100), 4), ((64, 90, 4100), 8), ((1, 200_001, 7), 64), ((33, 200_003, 5), 64),
           ((1, 600_001, 3), 256)]
 
 

@@ -50,10 +50,21 @@ def test_plan_is_bounded(cu):
         assert bands * -(-nx // 1024) * 1024 < 1 << 32, (nz, ny, nx, s.ty)
 
 
+# (shapes on which the two routes' times differ by a tenth and more)
 @pytest.mark.parametrize("shape,tiles", [((4, 4, 4), False), ((16, 16, 16), False), ((24, 24, 32), False),
-                                         ((1, 16, 1024), False), ((128, 16, 64), False), ((64, 8, 512), False),
-                                         ((1, 1, 8192), True), ((16, 1, 512), True), ((1, 64, 64), True),
-                                         ((129, 8, 64), True), ((16, 16, 2048), True), ((64, 64, 64), True),
-                                         ((500, 499, 900), True)])
-def test_fields_of_few_rows_take_the_shorter_route(shape, tiles):
+                                         ((1, 16, 1024), False), ((16, 16, 1500), False), ((64, 8, 512), False),
+                                         ((33, 1, 1024), False), ((24, 2, 1024), False), ((160, 8, 1024), False),
+                                         ((1, 1, 8192), True), ((16, 1, 512), True), ((16, 2, 100), True),
+                                         ((1, 64, 64), True), ((256, 8, 64), True), ((128, 16, 33), True),
+                                         ((16, 24, 247), True), ((60, 26, 643), True), ((256, 48, 1024), True),
+                                         ((64, 64, 64), True), ((1024, 3, 32), True), ((500, 499, 900), True)])
+def test_the_shorter_route_is_taken(shape, tiles):
     assert plan(*shape).fits == tiles
+
+
+# (shapes on which the rows of a tile make a difference of a fifth and more)
+@pytest.mark.parametrize("shape,rows", [((256, 48, 1024), 4), ((500, 100, 900), 16), ((64, 512, 1024), 8),
+                                        ((128, 512, 300), 8), ((24, 500, 900), 4), ((768, 32, 1024), 8),
+                                        ((500, 499, 900), 32), ((200, 300, 1500), 32), ((1, 1_000_000, 1000), 256)])
+def test_tiles_fill_the_chip_in_whole_rounds(shape, rows):
+    assert plan(*shape).ty == rows
