@@ -540,7 +540,8 @@ _NP_DT = {1: "int8", 2: "int16", 4: "int32"}
 def set_batch_grain(hist_chunk: int = 0, rounds: int = 0, run: int = 0) -> None:
     """Force the work-item grain of batches planned from now on (process-wide;
     0 = the planner's pick): histogram item bytes (power of two, 64 KiB ..
-    512 KiB), encode ticket rounds (1, 2, 4), decode items per grab (1, 4).
+    512 KiB), encode ticket rounds (1, 2, 4), a fourth of the tickets of a
+    decode item (1, 4).
     Output bytes do not depend on it."""
     _check(lib().mans_batch_set_grain(hist_chunk, rounds, run), "mans_batch_set_grain")
 

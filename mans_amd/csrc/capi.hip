@@ -28,7 +28,7 @@ struct mans_workspace {
   int cu = 0;
   uint32_t* hist = nullptr;      // [4][256] self-cleaning accumulators
   uint32_t* counters = nullptr;  // 0 done, 1 encode ticket, 2 adm ticket, 3 err, 4-5 scratch scalars,
-                                 // 8-9 histogram row grabs
+                                 // 8-9 histogram chunk grabs
   uint4* table = nullptr;        // [4][256]
   uint32_t* hist_out = nullptr;  // [4][256]
   uint64_t* status = nullptr;
@@ -330,7 +330,7 @@ constexpr uint64_t kNoAllocMaxBytes = 1ull << 30;
 constexpr uint64_t kNoAllocStatus = kNoAllocMaxBytes / 4096 / 2;  // one look-back word per two blocks
 struct NoAllocLayout {
   uint32_t hist[4 * 256];    // histogram accumulators (cleared by each call)
-  uint32_t counters[64];     // 0 done, 1 ticket, 3 error flags, 8-9 row grabs (cleared by each call)
+  uint32_t counters[64];     // 0 done, 1 ticket, 3 error flags, 8-9 histogram chunk grabs (cleared by each call)
   uint4 table[4 * 256];      // normalised tables
   uint64_t status[kNoAllocStatus];  // look-back words (cleared by the histogram launch)
 };
@@ -1197,7 +1197,7 @@ std::atomic<uint32_t> g_force_chunk{0}, g_force_rounds{0}, g_force_run{0};
 // still leave about 32 histogram chunks and 32 encode tickets per CU (a launch
 // keeps 8-16 wavefronts per CU busy and the queue balances their tails),
 // within the bounds of each.  4096 buffers of 8 GB take the largest grain; one
-// request of a few tens of MB the smallest.  Decode items: DecodeItems.
+// request of a few tens of MB the smallest.  Decode items: decode_items.
 BatchGrain batch_grain(uint64_t bytes, uint64_t units, int cu) {
   const uint64_t c = (uint64_t)std::max(cu, 1);
   BatchGrain g{kBatchHistChunkMin, 1, 0};

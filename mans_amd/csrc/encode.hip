@@ -335,7 +335,7 @@ __global__ __launch_bounds__(64 * NW) void encode_kernel(EncodeArgs a) {
 //
 // What bounds it: memory.  A unit's words are written to the slot, read back
 // and written out (2.6 GB for 1 GiB of codes of ratio 2.1, the 1.6 GB of input
-// and output and twice the output): 0.56 ms, 4.6 TB/s against the 4.7 of a
+// and output and twice the output): 0.58-0.59 ms, 4.6 TB/s against the 4.7 of a
 // large copy; with every load and store taken out of the loop the steps take
 // 0.39 ms.  (Before: a ticket per wavefront, its look-back and the next
 // ticket's atomic in the coding wavefronts' way, the chains' steps one after
@@ -653,7 +653,7 @@ __global__ __launch_bounds__(64 * (NW + 1), 5) void encode_mc_kernel(EncodeArgs 
       // Whole chunks: CK steps of each block are 1 KiB (512 B per half), read
       // with one 16-byte load per lane and passed through LDS, where each
       // lane then finds its element of every step.  (Elements loaded one by
-      // one, 128 B a load and 8 steps ahead: 0.58 ms on 1 GiB of uint16
+      // one, 128 B a load and 8 steps ahead: 4 % slower on 1 GiB of uint16
       // codes.)
       using EL = typename ElemOf<S>::T;
       typedef uint32_t u32x4a __attribute__((ext_vector_type(4), aligned(4)));  // inputs are 4-byte aligned

@@ -26,7 +26,7 @@ constexpr int kMaxPlanes = 4;
 constexpr uint32_t kAdmLanes = 32;
 constexpr uint32_t kAdmChunk = 16;
 constexpr uint32_t kAdmGroup = kAdmLanes * kAdmChunk;  // 512 elements
-constexpr uint32_t kAdmTicketGroups = 32;              // groups per wavefront and map ticket
+constexpr uint32_t kAdmTicketGroups = 32;              // groups of a map ticket that a wavefront maps
 constexpr uint32_t kAdmMod = 126;
 constexpr uint32_t kAdmLaneBytes = 32;                 // 256-bit lane buffer
 
@@ -161,7 +161,7 @@ struct EncodeArgs {
   uint32_t* d_out_size32;
   uint64_t* d_out_size64;
   int32_t frame;                 // 1: patch data_words / total_size in the frame header
-  uint16_t* spill;               // per-wave spill areas of the 64-lane encoder
+  uint16_t* spill;               // spill areas, per workgroup (null: the 32-lane whole-unit kernel)
   uint64_t spill_bytes;          // their capacity
 };
 
