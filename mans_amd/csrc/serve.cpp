@@ -164,10 +164,10 @@ uint64_t out_bytes_for(const mans_params& p, const mans_request& r) {
   return r.n_elems * (uint64_t)r.elem_bytes;
 }
 
-// Gives back the released outputs whose reads have run (lock held).  With
-// `idle`, also those of a stream that has run out of work by now: an event
-// recorded now would say so only later.
-void reap(mans_server* S, bool idle) {
+// Gives back the released outputs whose reads have run (lock held); true if
+// there were any.  With `idle`, also those of a stream that has run out of
+// work by now: an event recorded now would say so only later.
+bool reap(mans_server* S, bool idle) {
   int dev = -1;
   (void)hipGetDevice(&dev);
   if (dev != S->device) (void)hipSetDevice(S->device);
@@ -206,8 +206,10 @@ void reap(mans_server* S, bool idle) {
       ++k;
     }
   }
+  const bool any = k < S->leaving.size();
   S->leaving.resize(k);
   if (dev >= 0 && dev != S->device) (void)hipSetDevice(dev);
+  return any;
 }
 
 // Launches the requests admitted into `sl` (called without the lock; the
@@ -330,7 +332,7 @@ void worker_loop(mans_server* S) {
       }
     }
     if (progress) S->cv_done.notify_all();
-    if (!S->leaving.empty() && !S->waiting.empty()) reap(S, false);
+    bool launched = false;
     for (Slot& sl : S->slot) {
       if (sl.busy || S->waiting.empty()) continue;
       if (!admit(S, sl)) continue;
@@ -339,8 +341,10 @@ void worker_loop(mans_server* S) {
       lk.unlock();
       launch_slot(S, sl);
       lk.lock();
-      progress = true;
+      progress = launched = true;
     }
+    // (behind a launch, or when requests wait: not on their way to one)
+    if (!S->leaving.empty() && (launched || !S->waiting.empty()) && reap(S, false)) progress = true;
     const bool any_busy = S->slot[0].busy || S->slot[1].busy;
     if (S->stop && S->waiting.empty() && !any_busy) break;
     if (!progress) {
