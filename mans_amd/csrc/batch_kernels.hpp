@@ -1002,8 +1002,14 @@ __device__ __forceinline__ bool build_luts(const BatchBuf& B, uint32_t p0, uint3
     if (lane == 63) cdf[wave][kNumSymbols] = run;
   }
   __syncthreads();
-  for (uint32_t k = 0; k < P; ++k)
-    if (B.n > 0 && cdf[k][kNumSymbols] != W) return true;
+  // (the four sums are read together, those past P not looked at, and acted on
+  // after the build, which a bad table leads nowhere out of the LUT)
+  uint32_t off = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < kMaxPlanes; ++k) {
+    const uint32_t sum = cdf[k][kNumSymbols];
+    off |= k < P ? sum ^ W : 0u;
+  }
   for (uint32_t k = 0; k < np; ++k) {
     constexpr uint32_t PER = W > T ? W / T : 1u;
     uint32_t lo[PER];
@@ -1023,7 +1029,7 @@ __device__ __forceinline__ bool build_luts(const BatchBuf& B, uint32_t p0, uint3
       }
     }
   }
-  return false;
+  return B.n > 0 && off != 0;
 }
 
 // Decode ticket lt of buffer B with the 64-lane ring decoder: two blocks (2
