@@ -671,11 +671,14 @@ class Server:
             pass
 
 
+class _View:
+    """Device memory owned by the library, as torch takes it.  (A class made a
+    call: 3 us more of a fetch.)"""
+
+    def __init__(self, ptr: int, nbytes: int):
+        self.__cuda_array_interface__ = {"shape": (nbytes,), "typestr": "|u1", "data": (ptr, False), "version": 3}
+
+
 def _torch_from_ptr(ptr: int, nbytes: int):
     """A uint8 CUDA tensor aliasing device memory owned by the library."""
-    torch = _torch()
-
-    class _Arr:
-        __cuda_array_interface__ = {"shape": (nbytes,), "typestr": "|u1", "data": (ptr, False), "version": 3}
-
-    return torch.as_tensor(_Arr(), device="cuda")
+    return _torch().as_tensor(_View(ptr, nbytes), device="cuda")

@@ -165,9 +165,11 @@ uint64_t out_bytes_for(const mans_params& p, const mans_request& r) {
 }
 
 // Gives back the released outputs whose reads have run (lock held); true if
-// there were any.  With `idle`, also those of a stream that has run out of
-// work by now: an event recorded now would say so only later.
-bool reap(mans_server* S, bool idle) {
+// there were any.  kRecorded asks only the events there are; kRecord records
+// the missing ones; kIdle also gives back those of a stream that has run out of
+// work by now (an event recorded now would say so only later).
+enum class Reap { kRecorded, kRecord, kIdle };
+bool reap(mans_server* S, Reap how) {
   int dev = -1;
   (void)hipGetDevice(&dev);
   if (dev != S->device) (void)hipSetDevice(S->device);
@@ -184,9 +186,10 @@ bool reap(mans_server* S, bool idle) {
     bool read = false;
     if (l.read && ok(hipEventQuery(l.read))) {
       read = true;
+    } else if (how == Reap::kRecorded) {
     } else if (!ok(hipStreamIsCapturing(l.stream, &cs)) || cs != hipStreamCaptureStatusNone) {
       // (nothing can be asked of the stream until the capture ends)
-    } else if (idle && ok(hipStreamQuery(l.stream))) {
+    } else if (how == Reap::kIdle && ok(hipStreamQuery(l.stream))) {
       read = true;
     } else if (!l.read) {
       if (!ok(hipEventCreateWithFlags(&l.read, hipEventDisableTiming))) {
@@ -332,6 +335,7 @@ void worker_loop(mans_server* S) {
       }
     }
     if (progress) S->cv_done.notify_all();
+    if (!S->leaving.empty() && !S->waiting.empty()) (void)reap(S, Reap::kRecorded);
     bool launched = false;
     for (Slot& sl : S->slot) {
       if (sl.busy || S->waiting.empty()) continue;
@@ -343,8 +347,9 @@ void worker_loop(mans_server* S) {
       lk.lock();
       progress = launched = true;
     }
-    // (behind a launch, or when requests wait: not on their way to one)
-    if (!S->leaving.empty() && (launched || !S->waiting.empty()) && reap(S, false)) progress = true;
+    // (events are recorded behind a launch, or when requests wait for memory:
+    // not on their way to a launch)
+    if (!S->leaving.empty() && (launched || !S->waiting.empty()) && reap(S, Reap::kRecord)) progress = true;
     const bool any_busy = S->slot[0].busy || S->slot[1].busy;
     if (S->stop && S->waiting.empty() && !any_busy) break;
     if (!progress) {
@@ -522,7 +527,7 @@ mans_status mans_server_stats(mans_server* S, uint64_t* arena_bytes, uint64_t* a
                               uint64_t* waiting) {
   if (!S) return MANS_ERR_INVALID_ARG;
   std::lock_guard<std::mutex> g(S->mu);
-  reap(S, true);
+  reap(S, Reap::kIdle);
   if (arena_bytes) *arena_bytes = S->arena.total();
   if (arena_used) *arena_used = S->arena.used();
   if (batches) *batches = S->batches;
