@@ -186,7 +186,8 @@ bool reap(mans_server* S, Reap how) {
     bool read = false;
     if (l.read && ok(hipEventQuery(l.read))) {
       read = true;
-    } else if (how == Reap::kRecorded) {
+    } else if (how == Reap::kRecorded || l.stream == hipStreamPerThread) {
+      // (the releasing thread's stream: its event was recorded there)
     } else if (!ok(hipStreamIsCapturing(l.stream, &cs)) || cs != hipStreamCaptureStatusNone) {
       // (nothing can be asked of the stream until the capture ends)
     } else if (how == Reap::kIdle && ok(hipStreamQuery(l.stream))) {
@@ -496,7 +497,27 @@ static mans_status release_req(mans_server* S, uint64_t id, const hipStream_t* s
     auto it = S->reqs.find(id);
     if (it == S->reqs.end() || it->second->state != 2) return MANS_ERR_INVALID_ARG;
     Req* q = it->second;
-    if (stream) {
+    if (stream && *stream == hipStreamPerThread) {
+      // this thread's own stream: no other thread can record on it
+      Leaving l;
+      l.stream = *stream;
+      int dev = -1;
+      (void)hipGetDevice(&dev);
+      if (dev != S->device) (void)hipSetDevice(S->device);
+      const bool recorded = hipEventCreateWithFlags(&l.read, hipEventDisableTiming) == hipSuccess &&
+                            hipEventRecord(l.read, l.stream) == hipSuccess;
+      if (!recorded) {
+        if (l.read) (void)hipEventDestroy(l.read);
+        (void)hipStreamSynchronize(l.stream);
+      }
+      if (dev >= 0 && dev != S->device) (void)hipSetDevice(dev);
+      if (recorded) {
+        l.blocks.emplace_back(q->out_off, q->out_cap);
+        S->leaving.push_back(std::move(l));
+      } else {
+        S->arena.release(q->out_off, q->out_cap);
+      }
+    } else if (stream) {
       Leaving* l = nullptr;
       for (Leaving& o : S->leaving)
         if (o.stream == *stream && !o.read) l = &o;

@@ -76,3 +76,19 @@ def test_frozen_workspace_serves_any_shape_of_its_size():
         assert torch.equal(got.view(torch.int32).reshape(-1), want.view(torch.int32).reshape(-1)), shape
     del graph
     ws.close()
+
+
+# rows over 2048: tiles of 4 planes and 2 rows.  Tiles an axis of 1, 2 (no
+# prefixes), 3, and 8 and 9 slabs (a tile sums its corners, or a launch does)
+@pytest.mark.parametrize("shape", [(4, 2, 3000), (4, 4, 3000), (8, 2, 3000), (8, 4, 3000), (7, 3, 2049), (9, 6, 3000),
+                                   (5, 5, 8192), (32, 6, 2500), (30, 5, 2500), (36, 6, 2500), (33, 3, 2051),
+                                   (36, 1, 2500), (1, 6, 2500), (130, 70, 33), (113, 61, 200)],
+                         ids=lambda v: "x".join(map(str, v)))
+def test_inverse_of_few_tiles(shape):
+    assert plan(*shape).fits
+    codes, idx, val, want = field(shape, sum(shape))
+    ws = mans_amd.Workspace(0)
+    got = mans_amd.lorenzo_reconstruct(codes, idx, val, shape, EB, ws)
+    ws.check()
+    assert torch.equal(got.view(torch.int32).reshape(-1), want.view(torch.int32).reshape(-1))
+    ws.close()

@@ -51,3 +51,21 @@ def test_release_with_the_copy_enqueued(room):
     srv.close()
     ws.check()
     ws.close()
+
+
+@pytest.mark.parametrize("stream", ["default", "own", "thread"])
+def test_release_after_gives_the_memory_back(stream):
+    # (2: hipStreamPerThread, which only the releasing thread can record on)
+    own = torch.cuda.Stream()
+    handle = {"default": 0, "own": own.cuda_stream, "thread": 2}[stream]
+    srv = mans_amd.Server(mans_amd.params(10, 64), 4 << 30)
+    x = values(1 << 20, 3)
+    torch.cuda.synchronize()
+    rid = srv.submit_compress(x)
+    assert srv.wait(rid, 60_000).status == 0
+    assert srv.stats()["arena_used"] > 0
+    assert mans_amd.lib().mans_server_release_after(srv.handle, rid, handle) == 0
+    assert mans_amd.lib().mans_server_release_after(srv.handle, rid, handle) == 1  # (released: unknown)
+    torch.cuda.synchronize()
+    assert srv.stats()["arena_used"] == 0
+    srv.close()
